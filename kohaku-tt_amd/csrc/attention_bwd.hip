@@ -8,41 +8,43 @@
 // mask (the forward's modes), GQA, any head dim that is a multiple of 8 up to 256 (padded
 // to DP with zeros in registers), bf16 / fp16:
 //
-//   attn_bwd_rowdot  the row dots Dr = sum_d dO O (fp32) of every query row and head
-//   attn_bwd_grads   one launch of both gradient passes, their workgroups interleaved:
-//     dQ             per (sequence, query head, 64-row block, key split): over the key
-//                    tiles it sees P = exp2(c S + mask - lse2), dP = dO V^T,
-//                    dS = P (dP - Dr), dQ += dS K
-//     dK / dV        per (sequence, K/V head, 64-key tile, split): over the (query head
-//                    of the group, 32-row query block) items that see the tile -- split
-//                    s takes items s, s + splits, ... -- the same P / dS; dV += P^T dO,
-//                    dK += dS^T Q in fp32 registers.  One split: it writes dK / dV;
-//                    several: fp32 partials per split that
+//   attn_bwd_rowdot  row statistics of every query row and head: the base-2 lse and the
+//                    negated row dots -D, D = sum_d dO O (fp32)
+//   gradients        one launch of both passes, their workgroups interleaved:
+//     dQ             per (sequence, row block, key split): over the key tiles it sees
+//                    P = exp2(c S + mask - lse2), dP = dO V^T, dS = P (dP - D),
+//                    dQ += dS K
+//     dK / dV        per (sequence, K/V head, key tile, split): over the (query head of the
+//                    group, query block) items that see the tile -- split s takes items s,
+//                    s + splits, ... -- the same P / dS; dV += P^T dO, dK += dS^T Q in fp32
+//                    registers.  One split: it writes dK / dV; several: fp32 partials per
+//                    split that
 //   attn_bwd_sums    adds in split order (no atomics: repeat calls are bit-identical),
 //                    together with the key-split dQ partials
+//
+// Head dims padded to 128 or less run the gradients on attn_bwd_tile_kernel
+// (attention_bwd_tile.hpp, 32x32x16 MFMAs); wider ones on attn_bwd_grads here (16x16x32
+// MFMAs: 32 keys' dK and dV at 256 do not fit the tile kernel's registers).
 //
 // Probabilities follow the forward exactly: keys past the causal limit or masked
 // (logit <= -5e5) get P = 0; a row whose lse carries the -5e5 offset of a fully-masked
 // row (the forward ran it over its raw scores) takes every visible key's raw score.
-// S = Q K^T, dP = dO V^T and the three gradient products run on
-// v_mfma_f32_16x16x32_{bf16,f16}; tiles are staged row-major once, and an operand needed
-// along the other index comes out of the same tile through gfx950's transposed LDS reads
-// (tr_frag).  lse is the forward's natural-log row LSE.
+// Tiles are staged row-major once, and an operand needed along the other index comes out of
+// the same tile through gfx950's transposed LDS reads.  lse is the forward's natural-log row
+// LSE.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
-#include "common.hpp"
+#include "attention_bwd_params.hpp"
 
 namespace kmi {
+namespace bwd {
 namespace {
 
 constexpr int BT = 32;          // keys per K/V tile and rows per query block
 constexpr int PP = 20;          // pitch of a wavefront's [32][16] P / dS tiles (elements; 16, 24, 28, 40, 48 measured slower)
-constexpr int BWD_THREADS = 256;
-constexpr float kLog2e = 1.4426950408889634f;
-// A forward lse below this carries the -5e5 offset of a row with no kept key.
-constexpr float kRawLse = 0.5f * kMaskedLogit;
 
 template <typename T>
 struct BwdMfma;
@@ -88,122 +90,6 @@ __device__ __forceinline__ typename BwdMfma<T>::v8 tr_frag(const T* tile, int pi
     return __builtin_bit_cast(typename BwdMfma<T>::v8, u32x4{lo[0], lo[1], hi[0], hi[1]});
 }
 
-
-struct BwdParams {
-    const void *q, *k, *v, *o, *dout;
-    const float* lse;
-    void *dq, *dk, *dv;
-    float* dr;  // [hq][rows_total] fp32 row dots
-    // dK / dV partials [hkv][splits][keys_total][DP] fp32 (splits > 1), else null.
-    float *pdk, *pdv;
-    // dQ partials [hq][ksplit][rows_total][DP] fp32 (ksplit > 1), else null.
-    float* pdq;
-    int splits, ksplit;
-    int64_t qs[3], ks[3], vs[3], os[3], dos[3], dqs[3], dks[3], dvs[3], ls[3];
-    const void* mask;
-    int64_t ms[4];
-    int64_t mask_numel;
-    int mask_mode;
-    const int64_t* mask_off;
-    const int32_t *cu_q, *cu_k;
-    const int32_t* klen;  // dense key lengths [batch] (or null)
-    int total_q, total_k;
-    int batch, hq, hkv, group, seq_q, seq_k, causal;
-    int d, dval;  // q / k and v / out head dims (DP: the larger, padded)
-    int64_t rows_total, keys_total;
-    float scale, c2;  // c2 = scale * log2(e)
-};
-
-// One sequence's geometry: query rows [q0, q0 + lq) and keys [k0, k0 + lk) of the packed
-// (varlen) tensors, or the whole batch entry (dense); causal: row i sees keys
-// j <= i + coff (top-left dense: coff = 0; bottom-right varlen: coff = lk - lq).
-struct Geo {
-    int q0, lq, k0, lk, coff;
-    int64_t row_base, key_base;       // row / key index in [rows_total] / [keys_total]
-    int64_t qb, kb, vb, ob, dob, dqb, dkb, dvb, lb;  // batch-entry element offsets (dense)
-    int64_t mbase;                    // the mask element of (head 0, row 0, key 0)
-    int64_t mrow;                     // mask elements per query row
-    int64_t mkey;                     // mask elements per key
-    int64_t mend;                     // mask elements (reads at or past it count as masked)
-};
-
-__device__ __forceinline__ Geo geo_of(const BwdParams& p, int seq) {
-    Geo g;
-    if (p.cu_q) {
-        g.q0 = min(max(p.cu_q[seq], 0), p.total_q);
-        g.lq = min(min(max(p.cu_q[seq + 1], g.q0), p.total_q) - g.q0, p.seq_q);
-        g.k0 = min(max(p.cu_k[seq], 0), p.total_k);
-        g.lk = min(min(max(p.cu_k[seq + 1], g.k0), p.total_k) - g.k0, p.seq_k);
-        g.coff = g.lk - g.lq;
-        g.row_base = g.q0;
-        g.key_base = g.k0;
-        g.qb = g.kb = g.vb = g.ob = g.dob = g.dqb = g.dkb = g.dvb = g.lb = 0;
-    } else {
-        g.q0 = 0;
-        g.lq = p.seq_q;
-        g.k0 = 0;
-        g.lk = p.klen ? min(max(p.klen[seq], 1), p.seq_k) : p.seq_k;
-        g.coff = 0;
-        g.row_base = static_cast<int64_t>(seq) * p.seq_q;
-        g.key_base = static_cast<int64_t>(seq) * p.seq_k;
-        g.qb = seq * p.qs[0];
-        g.kb = seq * p.ks[0];
-        g.vb = seq * p.vs[0];
-        g.ob = seq * p.os[0];
-        g.dob = seq * p.dos[0];
-        g.dqb = seq * p.dqs[0];
-        g.dkb = seq * p.dks[0];
-        g.dvb = seq * p.dvs[0];
-        g.lb = seq * p.ls[0];
-    }
-    g.mbase = 0;
-    g.mrow = 0;
-    g.mkey = 0;
-    g.mend = INT64_MAX;
-    if (p.mask_mode == KMI_MASK_PACKED) {
-        int64_t off = 0;
-        if (p.mask_off) {
-            off = p.mask_off[seq];
-        } else {
-            for (int s = 0; s < seq; ++s) {
-                const int a0 = min(max(p.cu_q[s], 0), p.total_q), a1 = min(max(p.cu_q[s + 1], a0), p.total_q);
-                const int b0 = min(max(p.cu_k[s], 0), p.total_k), b1 = min(max(p.cu_k[s + 1], b0), p.total_k);
-                off += static_cast<int64_t>(a1 - a0) * (b1 - b0);
-            }
-        }
-        g.mbase = off;
-        g.mrow = g.lk;
-        g.mkey = 1;
-        g.mend = p.mask_numel;
-    } else if (p.mask_mode == KMI_MASK_STRIDED) {
-        g.mbase = p.cu_q ? static_cast<int64_t>(g.q0) * p.ms[2] + static_cast<int64_t>(g.k0) * p.ms[3] : seq * p.ms[0];
-        g.mrow = p.ms[2];
-        g.mkey = p.ms[3];
-    }
-    return g;
-}
-
-// The mask logit of (head h, row i, key j) of a sequence (0 without a mask).
-template <int MK>
-__device__ __forceinline__ float mask_at(const BwdParams& p, const Geo& g, int h, int i, int j) {
-    if constexpr (MK == MK_NONE) {
-        return 0.f;
-    } else {
-        typedef typename MaskRaw<MK>::type R;
-        const int64_t idx = g.mbase + h * p.ms[1] + i * g.mrow + j * g.mkey;
-        if (idx >= g.mend) return kMaskedLogit;
-        return mask_logit_of<MK>(static_cast<const R*>(p.mask)[idx]);
-    }
-}
-
-// Row statistics of row i (i < lq): base-2 lse of the row's softmax and whether the row
-// ran over its raw scores (no kept key in the forward).  Rows past the end or without
-// keys get +inf (P = 0).
-__device__ __forceinline__ void row_stats(float lse_nat, bool valid, float& lse2, bool& raw) {
-    raw = valid && lse_nat < kRawLse;
-    const float l = raw ? lse_nat - kMaskedLogit : lse_nat;
-    lse2 = (valid && l != -INFINITY) ? l * kLog2e : INFINITY;
-}
 
 // Staging of rows [r0, r0 + 32) of a [S, D] operand (row stride rs elements) in two steps:
 // loads into registers (16-byte chunks), issued a tile ahead, and their LDS stores,
@@ -364,7 +250,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdParams& p, const int bid)
         if (wave == 0) {
             const int ic = min(r0 + srow, g.lq - 1);
             lv_n = p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + ic) * p.ls[2]];
-            dr_n = p.dr[h * p.rows_total + g.row_base + ic];
+            dr_n = p.nd[h * p.rows_total + g.row_base + ic];
         }
     };
     int gi = nblk > 0 ? split / nblk : 0, bi = split - gi * nblk;
@@ -389,7 +275,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdParams& p, const int bid)
             row_stats(lv_n, ok, l2, raw);
             lse2[srow] = l2;
             raws[srow] = raw ? 1 : 0;
-            drs[srow] = ok ? dr_n : 0.f;
+            drs[srow] = ok ? -dr_n : 0.f;
         }
         __syncthreads();
         if (it + p.splits < items) {  // the next item's loads overlap this item's products
@@ -553,7 +439,15 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_rowdot(const BwdParams p
 #pragma unroll
         for (int o = CP / 2; o > 0; o >>= 1) dot += __shfl_xor(dot, o, kWave);
         const int row = row0 + RPI * i;
-        if (c == 0 && row < g.lq) p.dr[h * p.rows_total + g.row_base + row] = dot;
+        if (c == 0 && row < g.lq) {
+            const int64_t at = h * p.rows_total + g.row_base + row, plane = p.hq * p.rows_total;
+            float l2;
+            bool raw;
+            row_stats(p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + row) * p.ls[2]], true, l2, raw);
+            p.stats[at] = l2;
+            p.stats[plane + at] = -dot;
+            if (p.mask_mode != KMI_MASK_NONE) p.stats[2 * plane + at] = raw ? 1.f : 0.f;
+        }
     }
 }
 
@@ -659,9 +553,9 @@ __device__ __forceinline__ void attn_bwd_dq(const BwdParams& p, const int bid) {
         const int row = rw0 + 4 * g4 + j;
         const int rc = min(row, g.lq - 1);
         const float lv = p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + rc) * p.ls[2]];
-        const float dv = p.dr[h * p.rows_total + g.row_base + rc];
+        const float dv = p.nd[h * p.rows_total + g.row_base + rc];
         row_stats(lv, row < g.lq, l2[j], raw[j]);
-        drv[j] = row < g.lq ? dv : 0.f;
+        drv[j] = row < g.lq ? -dv : 0.f;
     }
     f32x4 dq[DB];
 #pragma unroll
@@ -886,18 +780,7 @@ const char* check_bwd(const kmi_attn_bwd_args* a) {
 int64_t rows_total_of(const kmi_attn_bwd_args* a) { return a->cu_seqlens_q ? a->total_q : a->batch * a->seq_q; }
 int64_t keys_total_of(const kmi_attn_bwd_args* a) { return a->cu_seqlens_q ? a->total_k : a->batch * a->seq_k; }
 
-// Split rules.  dK / dV and dQ workgroups run interleaved in one launch, so each kind
-// needs enough work per workgroup to amortise its set-up and few enough splits to keep
-// the fp32 partials small, rather than a grid that fills the chip alone.  A dK / dV
-// workgroup takes at most kBwdItemsPerWg64 (query head, 32-row block) items up to head
-// dim 64 and kBwdItemsPerWg128 at 128 (in proportion fewer past it) when splitting allows
-// it, a dQ workgroup at most kBwdTilesPerWg 32-key tiles; below kBwdMinWgs workgroups of a
-// kind, splits go down to kBwdMinItems items (or tiles) each.  Measured on C1 / C4 varlen
-// (us): items per workgroup 20 / 24 / 32 / 40 / 48 at every head dim gave 101 / 96 / 92 /
-// 88 / 95 on C1 (19 / 19 / 14 / 12 / 10 splits) and 225 / 180 / 205 / 204 / 204 on C4 (4 /
-// 3 / 2 / 2 / 2 splits); 43 scaled by 64 / head dim gave 90.3 (11 splits) / 179.0 (3).
-// dQ tiles per workgroup 16 / 24 / 32 / 48: C1 94 / 93 / 91 / 92, C4 249 / 248 / 205 / 205.
-constexpr int64_t kBwdItemsPerWg64 = 40;
+// Split rules of the head dims padded past 128 (attn_bwd_grads).
 constexpr int64_t kBwdItemsPerWg128 = 22;
 constexpr int64_t kBwdTilesPerWg = 32;
 constexpr int64_t kBwdMinWgs = 512;
@@ -913,15 +796,6 @@ int64_t bwd_split_count(int64_t units, int64_t work, int64_t per_wg, int64_t cap
     return std::max<int64_t>(1, std::min<int64_t>({cap, std::max(by_work, by_fill), std::max<int64_t>(1, work)}));
 }
 
-// dK / dV splits over the (query head of the group, 32-row block) items of a key tile.
-int bwd_splits(const kmi_attn_bwd_args* a) {
-    const int64_t wgs = a->batch * a->heads_kv * ceil_div(a->seq_k, KW);
-    const int64_t items = (a->heads_q / a->heads_kv) * ceil_div(a->seq_q, BT);
-    const int64_t dp = padded_head_dim(std::max(a->head_dim, bwd_value_dim(a)));
-    const int64_t per_wg = dp <= 64 ? kBwdItemsPerWg64 : ceil_div(kBwdItemsPerWg128 * 128, dp);
-    return static_cast<int>(bwd_split_count(wgs, items, per_wg, kBwdMaxSplits));
-}
-
 // KMI_BWD_KSPLIT=n (read once; tuning): pins the dQ key splits.
 int bwd_ksplit_override() {
     static const int v = [] {
@@ -931,55 +805,130 @@ int bwd_ksplit_override() {
     return v;
 }
 
-// dQ key splits over the 32-key tiles of a (query head, 64-row block).
-int bwd_ksplit(const kmi_attn_bwd_args* a) {
-    const int64_t tiles = ceil_div(a->seq_k, BT);
-    if (bwd_ksplit_override() > 0)
-        return static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
-    const int64_t wgs = a->batch * a->heads_q * ceil_div(a->seq_q, QW);
-    return static_cast<int>(bwd_split_count(wgs, tiles, kBwdTilesPerWg, kBwdMaxKsplit));
-}
-
-// Workspace floats: row dot products (padded to 16 bytes); with GQA or splits the dK / dV
-// partials; with key splits the dQ partials.
-struct BwdLayout {
-    size_t dr, part, pdq;
+struct BwdPlan {
+    bool tile;  // attn_bwd_tile_kernel (padded head dims up to 128), else attn_bwd_grads
+    int splits, ksplit;
+    BwdGrid grid;
 };
 
-BwdLayout bwd_layout(const kmi_attn_bwd_args* a) {
+// Split rules of attn_bwd_tile_kernel.  The fp32 partials of a split cost about what
+// several items do, so a dK / dV workgroup is split by its work (at most kTileItems 32-row
+// items each while that leaves at most kTileMaxWgs workgroups) and, below kTileFewWgs
+// workgroups, to fill the chip with at least kTileMinItems each.  Measured (us of the whole
+// backward, by splits; * what the rule takes):
+//   2x8/2x3062x128 causal (96 workgroups, 384 items): 2 317, 3 228, 4 188, 6* 177, 8 198
+//   1x24x4396x128 (840, 138): 1 984, 2* 922-944, 3 1050-1190
+//   3x32/8x1718x40 (648, 216): 1 344, 2 338, 3* 295, 4 295
+//   8x16/8x655/204x128 (128, 42): 1 109, 2 94, 3 87, 4* 88, 6 102
+//   32x14/2x80x128 causal (64, 21): 1 50, 2 39, 3* 35, 4 39
+//   1x14/2x2048x64 causal (64, 448): 8* 54, 10 52, 12 55
+//   4x12x512x64 causal (384, 16): 1* 22, 2 33
+// 64-key dK / dV workgroups (two wavefronts per 32 keys) at padded head dims up to 64:
+// 4x16x1024x64 83 against 93 with 128 keys, 3x32/8x1718x40 295 against 309.  64-row dQ
+// workgroups only where 128 rows leave CUs idle (4x16x1024x64, 512 workgroups: 95 against
+// 83; 1x14/2x2048x64, 224 workgroups: 54 against 57).
+constexpr int64_t kTileItems = 72;
+constexpr int64_t kTileMaxWgs = 2048;
+constexpr int64_t kTileFewWgs = 256;
+constexpr int64_t kTileMinItems = 7;
+
+BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
+    BwdPlan pl{};
+    const int64_t dp = padded_head_dim(std::max(a->head_dim, bwd_value_dim(a)));
+    const int64_t units = a->batch * a->heads_kv, G = a->heads_q / a->heads_kv;
+    pl.tile = dp <= 128;
+    if (!pl.tile) {
+        const int64_t per_wg = ceil_div(kBwdItemsPerWg128 * 128, dp), tiles = ceil_div(a->seq_k, BT);
+        pl.splits = static_cast<int>(
+            bwd_split_count(units * ceil_div(a->seq_k, KW), G * ceil_div(a->seq_q, BT), per_wg, kBwdMaxSplits));
+        pl.ksplit = static_cast<int>(bwd_split_count(a->batch * a->heads_q * ceil_div(a->seq_q, QW), tiles,
+                                                     kBwdTilesPerWg, kBwdMaxKsplit));
+        if (bwd_ksplit_override() > 0)
+            pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
+        return pl;
+    }
+    pl.grid.half_k = dp <= 64;
+    const int64_t nk = units * ceil_div(a->seq_k, pl.grid.half_k ? 64 : 128);
+    const int64_t work = G * ceil_div(a->seq_q, 32);
+    const int64_t by_work = std::min(ceil_div(work, kTileItems), ceil_div(kTileMaxWgs, nk));
+    const int64_t by_fill = nk < kTileFewWgs ? std::min(ceil_div(2 * kTileFewWgs, nk), work / kTileMinItems) : 1;
+    pl.splits = static_cast<int>(std::max<int64_t>(1, std::min(std::max(by_work, by_fill), kBwdMaxSplits)));
+    // dQ: by the query heads (a call with K / V repeated per query head splits alike, so its
+    // dQ is the same bit for bit).
+    const int64_t nq = a->batch * a->heads_q * ceil_div(a->seq_q, 128), tiles = ceil_div(a->seq_k, 64);
+    pl.grid.half_q = nq < kTileFewWgs;
+    const int64_t nqw = pl.grid.half_q ? a->batch * a->heads_q * ceil_div(a->seq_q, 64) : nq;
+    pl.ksplit = static_cast<int>(std::max<int64_t>(
+        1, std::min<int64_t>({ceil_div(kTileFewWgs, 2 * nqw), tiles / 8, kBwdMaxKsplit})));
+    if (bwd_ksplit_override() > 0)
+        pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
+    pl.grid.tiles_q = static_cast<int>(ceil_div(a->seq_q * G, pl.grid.half_q ? 64 : 128));
+    pl.grid.nk = static_cast<int>(nk * pl.splits);
+    pl.grid.nq = static_cast<int>(units * pl.grid.tiles_q * pl.ksplit);
+    return pl;
+}
+
+// Workspace floats: the row statistics (padded to 16 bytes); with splits the dK / dV
+// partials; with key splits the dQ partials.
+struct BwdLayout {
+    size_t stats, part, pdq;
+};
+
+BwdLayout bwd_layout(const kmi_attn_bwd_args* a, const BwdPlan& pl) {
     BwdLayout l{};
     const int64_t dp = padded_head_dim(std::max(a->head_dim, bwd_value_dim(a)));
-    l.dr = static_cast<size_t>(ceil_div(a->heads_q * rows_total_of(a), 4) * 4);
+    const int64_t planes = a->mask_mode == KMI_MASK_NONE ? 2 : 3;
+    l.stats = static_cast<size_t>(ceil_div(planes * a->heads_q * rows_total_of(a), 4) * 4);
     // One split sums the query heads of a K/V head in its registers and writes dK / dV.
-    const int s = bwd_splits(a);
-    if (s > 1) l.part = static_cast<size_t>(a->heads_kv * s * keys_total_of(a) * dp);
-    const int ks = bwd_ksplit(a);
-    if (ks > 1) l.pdq = static_cast<size_t>(a->heads_q * ks * rows_total_of(a) * dp);
+    if (pl.splits > 1) l.part = static_cast<size_t>(a->heads_kv * pl.splits * keys_total_of(a) * dp);
+    if (pl.ksplit > 1) l.pdq = static_cast<size_t>(a->heads_q * pl.ksplit * rows_total_of(a) * dp);
     return l;
 }
 
-size_t bwd_ws_bytes(const kmi_attn_bwd_args* a) {
-    const BwdLayout l = bwd_layout(a);
-    return (l.dr + 2 * l.part + l.pdq) * sizeof(float);
-}
+size_t bwd_ws_bytes(const BwdLayout& l) { return (l.stats + 2 * l.part + l.pdq) * sizeof(float); }
 
+// The gradient kernel of head dims padded past 128.
 template <typename T, int DP, int MK>
-hipError_t launch_bwd(const BwdParams& p, hipStream_t s) {
+hipError_t launch_grads(const BwdParams& p, hipStream_t s) {
     const int64_t ntk = ceil_div(p.seq_k, KW), nqb = ceil_div(p.seq_q, QW);
-    // The row dots first (both gradient passes read them), then dK / dV and dQ in one grid.
-    const dim3 grd(static_cast<unsigned>(static_cast<int64_t>(p.batch) * p.hq * nqb));
     const int64_t ndq = static_cast<int64_t>(p.batch) * p.hq * nqb * p.ksplit;
     const int64_t nkv = static_cast<int64_t>(p.batch) * p.hkv * ntk * p.splits;
     const dim3 grid(static_cast<unsigned>(nkv + ndq));
-    if (p.dval != p.d) {
-        hipLaunchKernelGGL((attn_bwd_rowdot<T, DP, true>), grd, dim3(BWD_THREADS), 0, s, p);
+    if (p.dval != p.d)
         hipLaunchKernelGGL((attn_bwd_grads<T, DP, MK, true>), grid, dim3(BWD_THREADS), 0, s, p, static_cast<int>(nkv),
                            static_cast<int>(ndq));
-    } else {
-        hipLaunchKernelGGL((attn_bwd_rowdot<T, DP, false>), grd, dim3(BWD_THREADS), 0, s, p);
+    else
         hipLaunchKernelGGL((attn_bwd_grads<T, DP, MK, false>), grid, dim3(BWD_THREADS), 0, s, p, static_cast<int>(nkv),
                            static_cast<int>(ndq));
+    return hipGetLastError();
+}
+
+template <typename T, int DP>
+hipError_t launch_grads_mask(const BwdParams& p, int mk, hipStream_t s) {
+    switch (mk) {
+        case MK_NONE: return launch_grads<T, DP, MK_NONE>(p, s);
+        case MK_BOOL: return launch_grads<T, DP, MK_BOOL>(p, s);
+        case MK_BF16: return launch_grads<T, DP, MK_BF16>(p, s);
+        case MK_F16: return launch_grads<T, DP, MK_F16>(p, s);
+        default: return launch_grads<T, DP, MK_F32>(p, s);
     }
+}
+
+// The call's launches: row statistics, gradients, split sums.
+template <typename T, int DP>
+hipError_t launch_bwd(const BwdParams& p, const BwdPlan& pl, int mk, hipStream_t s) {
+    const int64_t nqb = ceil_div(p.seq_q, QW);
+    const dim3 grd(static_cast<unsigned>(static_cast<int64_t>(p.batch) * p.hq * nqb));
+    if (p.dval != p.d)
+        hipLaunchKernelGGL((attn_bwd_rowdot<T, DP, true>), grd, dim3(BWD_THREADS), 0, s, p);
+    else
+        hipLaunchKernelGGL((attn_bwd_rowdot<T, DP, false>), grd, dim3(BWD_THREADS), 0, s, p);
+    hipError_t err;
+    if constexpr (DP <= 128)
+        err = launch_tile<T, DP>(p, pl.grid, mk, s);
+    else
+        err = launch_grads_mask<T, DP>(p, mk, s);
+    if (err != hipSuccess) return err;
     const int64_t dq_blocks = p.pdq ? ceil_div(static_cast<int64_t>(p.hq) * p.rows_total * (p.d / 4), 256) : 0;
     const int64_t kv_blocks =
         p.pdk ? ceil_div(static_cast<int64_t>(p.hkv) * p.keys_total * (std::max(p.d, p.dval) / 4), 256) : 0;
@@ -989,44 +938,38 @@ hipError_t launch_bwd(const BwdParams& p, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <typename T, int DP>
-hipError_t launch_bwd_mask(const BwdParams& p, int mk, hipStream_t s) {
-    switch (mk) {
-        case MK_NONE: return launch_bwd<T, DP, MK_NONE>(p, s);
-        case MK_BOOL: return launch_bwd<T, DP, MK_BOOL>(p, s);
-        case MK_BF16: return launch_bwd<T, DP, MK_BF16>(p, s);
-        case MK_F16: return launch_bwd<T, DP, MK_F16>(p, s);
-        default: return launch_bwd<T, DP, MK_F32>(p, s);
-    }
-}
-
 template <typename T>
-hipError_t launch_bwd_dim(const BwdParams& p, int mk, hipStream_t s) {
+hipError_t launch_bwd_dim(const BwdParams& p, const BwdPlan& pl, int mk, hipStream_t s) {
     switch (padded_head_dim(std::max(p.d, p.dval))) {
-        case 32: return launch_bwd_mask<T, 32>(p, mk, s);
-        case 64: return launch_bwd_mask<T, 64>(p, mk, s);
-        case 96: return launch_bwd_mask<T, 96>(p, mk, s);
-        case 128: return launch_bwd_mask<T, 128>(p, mk, s);
-        case 192: return launch_bwd_mask<T, 192>(p, mk, s);
-        default: return launch_bwd_mask<T, 256>(p, mk, s);
+        case 32: return launch_bwd<T, 32>(p, pl, mk, s);
+        case 64: return launch_bwd<T, 64>(p, pl, mk, s);
+        case 96: return launch_bwd<T, 96>(p, pl, mk, s);
+        case 128: return launch_bwd<T, 128>(p, pl, mk, s);
+        case 192: return launch_bwd<T, 192>(p, pl, mk, s);
+        default: return launch_bwd<T, 256>(p, pl, mk, s);
     }
 }
 
 }  // namespace
+}  // namespace bwd
 }  // namespace kmi
 
 extern "C" int kmi_attn_bwd_workspace_bytes(const kmi_attn_bwd_args* a, size_t* bytes) {
     using namespace kmi;
+    using namespace kmi::bwd;
     if (!bytes) return fail(KMI_EINVAL, "kmi_attn_bwd_workspace_bytes: null bytes");
     if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd_workspace_bytes: ") + why);
-    *bytes = bwd_ws_bytes(a);
+    *bytes = bwd_ws_bytes(bwd_layout(a, bwd_plan(a)));
     return KMI_OK;
 }
 
 extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace kmi;
+    using namespace kmi::bwd;
     if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd: ") + why);
-    const size_t need = bwd_ws_bytes(a);
+    const BwdPlan pl = bwd_plan(a);
+    const BwdLayout l = bwd_layout(a, pl);
+    const size_t need = bwd_ws_bytes(l);
     if (!workspace || workspace_bytes < need || reinterpret_cast<uintptr_t>(workspace) % 16)
         return fail(KMI_EWORKSPACE, "kmi_attn_bwd: workspace missing or smaller than kmi_attn_bwd_workspace_bytes");
     BwdParams p{};
@@ -1039,18 +982,16 @@ extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t 
     p.dq = a->grad_q;
     p.dk = a->grad_k;
     p.dv = a->grad_v;
-    p.dr = static_cast<float*>(workspace);
-    p.splits = bwd_splits(a);
-    p.ksplit = bwd_ksplit(a);
-    {
-        // Partials start 16-byte aligned after the row dot products (DP is a multiple of 4).
-        const BwdLayout l = bwd_layout(a);
-        if (l.part) {
-            p.pdk = p.dr + l.dr;
-            p.pdv = p.pdk + l.part;
-        }
-        if (l.pdq) p.pdq = p.dr + l.dr + 2 * l.part;
+    p.splits = pl.splits;
+    p.ksplit = pl.ksplit;
+    // Partials start 16-byte aligned after the row statistics (DP is a multiple of 4).
+    p.stats = static_cast<float*>(workspace);
+    p.nd = p.stats + a->heads_q * rows_total_of(a);
+    if (l.part) {
+        p.pdk = p.stats + l.stats;
+        p.pdv = p.pdk + l.part;
     }
+    if (l.pdq) p.pdq = p.stats + l.stats + 2 * l.part;
     for (int i = 0; i < 3; ++i) {
         p.qs[i] = a->q_stride[i];
         p.ks[i] = a->k_stride[i];
@@ -1086,7 +1027,11 @@ extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t 
     p.keys_total = keys_total_of(a);
     p.scale = static_cast<float>(a->scale);
     p.c2 = static_cast<float>(a->scale * 1.4426950408889634);
+    // A zero scale becomes one that finite scores vanish under (minus infinity does not).
+    if (pl.tile && std::fabs(p.c2) < 1e-30f) p.c2 = p.c2 < 0.f ? -1e-30f : 1e-30f;
+    p.mask_c = static_cast<float>(1.4426950408889634 / static_cast<double>(p.c2));
+    p.hidden = p.c2 > 0.f ? -INFINITY : INFINITY;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const hipError_t err = a->dtype == KMI_BF16 ? launch_bwd_dim<bf16>(p, mk, s) : launch_bwd_dim<f16>(p, mk, s);
+    const hipError_t err = a->dtype == KMI_BF16 ? launch_bwd_dim<bf16>(p, pl, mk, s) : launch_bwd_dim<f16>(p, pl, mk, s);
     return hip_status(err, "kmi_attn_bwd");
 }

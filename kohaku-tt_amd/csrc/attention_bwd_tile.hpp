@@ -1,0 +1,792 @@
+// Attention backward, the gradient kernels for head dims padded to 128 or less (gfx950).
+// What they compute and the launches around them are described in attention_bwd.hip.
+//
+// Both passes run on v_mfma_f32_32x32x16: 256-thread workgroups stage 64-row tiles of the
+// two operands the pass walks over (Q and dO for dK / dV, K and V for dQ) in LDS, double
+// buffered, by buffer loads that write LDS directly, and every wavefront keeps 32 rows of
+// the other side (keys or query rows) in registers as B operands:
+//
+//   dK / dV  S = Q K^T and dP = dO V^T of a 32-row block come out with one key per lane
+//            and 16 query rows in registers, which is the B operand of dV^T += dO^T P and
+//            dK^T += Q^T dS as it stands: P and dS never leave the registers.
+//   dQ       S^T = K Q^T and dP^T = V dO^T: one query row per lane, 16 keys in registers,
+//            the B operand of dQ^T += K^T dS^T.
+//
+// The A operands of the second products (dO^T, Q^T, K^T) are gfx950 transposed LDS reads
+// of the same tiles.  dP accumulates from -D (the row dot), so dS = P dP has no subtraction.
+//
+// What bounds it: a 32x32 block of dK / dV is 2 D / 8 MFMAs (1024 cycles of the matrix unit
+// at D = 128) over about 64 VALU instructions a lane and 48 LDS reads, so with everything
+// in registers the matrix unit should lead; measured it is busy half the time, the rest
+// being waits at the tile barriers and the chain S -> P -> dV / dK within a wavefront (two
+// wavefronts a SIMD at D = 128, three at 64).  Whole backward, before (16x16x32 MFMAs, P
+// and dS through LDS, staging through registers) -> with this kernel, us:
+//   1x24x4396x128        1388 -> 922  (428 -> 644 TFLOP/s)
+//   2x10x4096x64          542 -> 387  (396 -> 556)
+//   2x8/2x3062x128 causal 320 -> 169  (300 -> 570)
+//   1x14/2x2048x64 causal  72 -> 53   (263 -> 353)
+//   8 packed x 16/8 x 128 causal, 64 to 1024 tokens 153 -> 117 (211 -> 277)
+//   2x12x2433x128, additive mask 1426 -> 598 (128 -> 304)
+// What mattered on the way (1x24x4396x128): tiles by registers' leave, without a spill in
+// the loop (1351 with fragments spilled -> 984 with V in LDS and one code path per block);
+// swizzles for 64 banks (LDS busy 39% -> 19% of the time).
+#pragma once
+
+#include <cstddef>
+#include <type_traits>
+
+#include "attention_bwd_params.hpp"
+
+namespace kmi {
+namespace bwd {
+
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <typename T>
+struct Mfma32;
+template <>
+struct Mfma32<bf16> {
+    typedef bf16x8 v8;
+    static __device__ __forceinline__ f32x16 run(v8 a, v8 b, f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    }
+};
+template <>
+struct Mfma32<f16> {
+    typedef f16x8 v8;
+    static __device__ __forceinline__ f32x16 run(v8 a, v8 b, f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+    }
+};
+
+// gfx950's transposed LDS read: within each 16-lane group, output lane j, slot s receives
+// element j % 4 of the 4-element chunk that source lane 4 s + j / 4 addressed.
+template <typename T>
+__device__ __forceinline__ u32x2 lds_tr(uint32_t at) {
+    if constexpr (std::is_same<T, bf16>::value) {
+        typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 x4;
+        return __builtin_bit_cast(u32x2,
+                                  __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) x4*)(at)));
+    } else {
+        typedef __attribute__((__vector_size__(4 * sizeof(__fp16)))) __fp16 x4;
+        return __builtin_bit_cast(u32x2,
+                                  __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) x4*)(at)));
+    }
+}
+
+// LDS DMA: every lane's 16 (or 4) bytes at byte offset `off` of the resource (zeros past
+// its range) go to LDS at dst + 16 (4) lane.  Written as asm because the compiler takes
+// every transposed LDS read for a use of every load of this kind in flight and waits for
+// all of them first, which would end each prefetch at the next read (C1 backward's dK / dV
+// loop had one such wait per 32 rows).  The loops below wait for a tile themselves (all of
+// vmcnt) before the barrier that publishes it.  The nop is the wait state between a write
+// of m0 and its use.
+__device__ __forceinline__ u32x4 dma_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)(static_cast<const char*>(p))));
+}
+__device__ __forceinline__ void dma16(u32x4 rs, uint32_t off, uint32_t dst) {
+    __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                     :
+                     : "v"(off), "s"(rs), "s"(dst)
+                     : "memory");
+}
+__device__ __forceinline__ void dma4(u32x4 rs, uint32_t off, uint32_t dst) {
+    __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds"
+                     :
+                     : "v"(off), "s"(rs), "s"(dst)
+                     : "memory");
+}
+
+// A [TR][DP] tile in LDS: rows of NCH 16-byte chunks (a power of two; at DP = 96 the last
+// four stay zero), chunk c of row r at c ^ swz(r).  LDS reads take 256 bytes a cycle from
+// 64 banks: 16 lanes of a b128 row read (16 rows, one column) and 32 lanes of a transposed
+// read (4 rows of 4 chunks, or 8 rows of 2).  With r0 .. r3 the low bits of the row, the
+// swizzles below put each of those sets on distinct banks (a row of 128 or 64 bytes already
+// takes its half or quarter of the banks from r0, or r0 and r1).
+template <typename T, int DP, int TR>
+struct Tile {
+    typedef typename Mfma32<T>::v8 v8;
+    static constexpr int NCH = DP <= 32 ? 4 : (DP <= 64 ? 8 : 16);
+    static constexpr int PITCH = 8 * NCH;
+    static constexpr int ELEMS = TR * PITCH;
+    // DMA: one instruction fills 1 KiB (RPI rows); wavefront w fills rows RW w .. + RW - 1.
+    static constexpr int RPI = kWave / NCH;
+    static constexpr int RW = TR / 4 < RPI ? RPI : TR / 4;
+    static constexpr int IPW = RW / RPI;
+    static constexpr int NRA = NCH / 2, NTA = NCH / 4;
+    static constexpr uint32_t kNoChunk = 0x80000000u;  // past every range (below 2^31 bytes)
+
+    static __device__ __forceinline__ int swz(int r) {
+        const int r1 = (r >> 1) & 1, r2 = (r >> 2) & 1, r3 = (r >> 3) & 1;
+        return NCH == 4 ? 2 * r2 + r3 : (NCH == 8 ? 4 * r1 + 2 * r2 + r3 : 4 * (r & 3) + 2 * r2 + r3);
+    }
+
+    // A lane's place in a DMA instruction's RPI rows: its row's byte offset, and the chunk it
+    // reads in instruction 0 (instruction i, rows RPI i .., reads chunk ^ swz(RPI i)).
+    struct Offs {
+        uint32_t row, chunk;
+    };
+    static __device__ __forceinline__ Offs offs(int lane, uint32_t stride) {
+        const int r = lane / NCH;
+        return Offs{static_cast<uint32_t>(r) * stride, static_cast<uint32_t>((lane % NCH) ^ swz(r))};
+    }
+    // Requests rows [row0 + RW wave, + RW) of an [nrows, row_bytes] operand (row stride
+    // `stride` bytes, below 2^26) into the tile at LDS address dst; rows at or past nrows
+    // read zeros.
+    static __device__ __forceinline__ void request(const char* base, uint32_t stride, int row0, int nrows, int row_bytes,
+                                                   const Offs& off, int wave, uint32_t dst) {
+        if (RW * wave >= TR) return;
+        const int first = row0 + RW * wave;
+        const u32x4 rs = dma_rsrc(base + static_cast<int64_t>(first) * stride,
+                                  rows_extent(min(RW, nrows - first), stride, static_cast<uint32_t>(row_bytes)));
+        const uint32_t at = dst + RW * wave * PITCH * static_cast<uint32_t>(sizeof(T));
+        // (The offsets are formed per tile: held across the loop they would cost registers.)
+        uint32_t x0 = swz(RW * wave);
+        __asm__ volatile("" : "+s"(x0));
+#pragma unroll
+        for (int i = 0; i < IPW; ++i) {
+            const uint32_t c = 16u * (off.chunk ^ x0 ^ swz(RPI * i));  // chunks past the row read zeros
+            dma16(rs, c < static_cast<uint32_t>(row_bytes) ? off.row + static_cast<uint32_t>(i * RPI) * stride + c : kNoChunk,
+                  at + i * RPI * PITCH * static_cast<uint32_t>(sizeof(T)));
+        }
+    }
+
+    // Lane byte addresses of the operand reads, relative to a tile's first row; tiles start at
+    // multiples of a row's bytes, so that a chunk's swizzled place is an XOR of low bits.
+    struct Addr {
+        uint32_t row;      // A operand: row l32, dims 8 h ..
+        uint32_t tr0, tr1; // A operand transposed: dims lane % 32, rows 4 h + s and 8 + 4 h + s
+    };
+    static __device__ __forceinline__ Addr addr(int lane) {
+        const int l32 = lane & 31, h = lane >> 5, k = lane & 15, dh = (lane >> 4) & 1;
+        auto tr = [&](int r) {
+            return static_cast<uint32_t>(2 * (r * PITCH + 8 * ((2 * dh + ((k & 3) >> 1)) ^ swz(r)) + 4 * (k & 1)));
+        };
+        return Addr{static_cast<uint32_t>(2 * (l32 * PITCH + 8 * (h ^ swz(l32)))), tr(4 * h + (k >> 2)),
+                    tr(8 + 4 * h + (k >> 2))};
+    }
+    // Rows l32, dims 16 c + 8 h .. + 7 at LDS address ra (+ imm, a constant).
+    static __device__ __forceinline__ v8 rows(uint32_t ra, int c, uint32_t imm) {
+        return *(const __attribute__((address_space(3))) v8*)((ra ^ (32u * c)) + imm);
+    }
+    // Dims 32 b + lane % 32, rows 16 kc + {4 h + s, 8 + 4 h + s}: the k order of an
+    // accumulator's registers 8 kc .. + 7 as a B operand.
+    static __device__ __forceinline__ v8 cols(uint32_t t0, uint32_t t1, int kc, int b, uint32_t imm) {
+        const uint32_t at = imm + 2u * 16 * kc * PITCH;
+        const u32x2 lo = lds_tr<T>((t0 ^ (64u * b)) + at), hi = lds_tr<T>((t1 ^ (64u * b)) + at);
+        return __builtin_bit_cast(v8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+    }
+};
+
+// A 16-byte fragment of row `row` at column `col` of an [nrows, d] operand, zeros past
+// the last row or the head dim.
+template <typename V, typename T>
+__device__ __forceinline__ V frag16(const T* base, int64_t rs, int row, int nrows, int col, int d) {
+    const int rc = min(max(row, 0), nrows - 1);
+    const u32x4 x = *reinterpret_cast<const u32x4*>(base + static_cast<int64_t>(rc) * rs + min(col, d - 8));
+    return __builtin_bit_cast(V, (row >= 0 && row < nrows && col < d) ? x : u32x4{0u, 0u, 0u, 0u});
+}
+
+template <typename T>
+__device__ __forceinline__ f32x16 splat16(T x) {
+    f32x16 v;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = x;
+    return v;
+}
+
+// Four consecutive dims of an output row: fp32 partials or the gradient's own type.
+template <typename T>
+__device__ __forceinline__ void store4(T* dst, const f32x4 v) {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    t4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = from_f32<T>(v[e]);
+    *reinterpret_cast<t4*>(dst) = w;
+}
+
+// Scheduling groups (LLVM's sched_group_barrier masks).
+constexpr int SG_VALU = 0x2, SG_MFMA = 0x8, SG_DSREAD = 0x100;
+// Fragments read ahead of the product that takes them.
+constexpr int QA = 4, VA = 2, NFR = 4;
+
+// dK / dV tiles: 64 rows at padded head dims up to 64.  At 96 and 128 the accumulators and
+// the K fragments leave no registers for V's, so V sits in LDS beside 32-row tiles (two
+// workgroups per CU either way).
+template <typename T, int DP>
+struct DkdvShared {
+    static constexpr int TR = DP <= 64 ? 64 : 32;
+    static constexpr bool VL = DP > 64;
+    typedef Tile<T, DP, TR> TL;
+    T tile[2][2][TL::ELEMS];
+    T v[VL ? 128 * TL::PITCH : 8];
+    // Base-2 lse, -D, raw flag (masked calls) of the tile's rows; a DMA instruction fills 64.
+    float stats[2][3][kWave];
+};
+
+// dK / dV of 32 KG keys of one K/V head (wavefront w: key group w % KG; with KG = 2 the
+// two wavefronts of a key group take one 32-row block of each tile each and add their
+// sums at the end) over the split's (query head, query tile) items.
+template <typename T, int DP, int MK, int KG>
+__device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem, const int tile, const int split,
+                                         const int bkv) {
+    typedef DkdvShared<T, DP> SH;
+    typedef typename SH::TL TL;
+    typedef typename TL::v8 v8;
+    constexpr int TR = SH::TR, DC = DP / 16, DB = DP / 32, RB = TR / 32;
+    constexpr int ES = static_cast<int>(sizeof(T));
+    constexpr int RS = 4 / KG;  // wavefronts that share a key group
+    constexpr bool VL = SH::VL;
+    static_assert(RS <= RB, "a wavefront of a key group takes whole 32-row blocks");
+    SH& sh = *reinterpret_cast<SH*>(smem);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h2 = lane >> 5, l32 = lane & 31;
+    const int kg = wave % KG, rsp = wave / KG;
+    const int seq = bkv / p.hkv, kvh = bkv - seq * p.hkv;
+    const Geo g = geo_of(p, seq);
+    const int kt0 = tile * 32 * KG;
+    // Keys written: the sequence's (varlen) or every key row of the batch entry (dense:
+    // keys past a key length get zero gradients).
+    const int kwrite = p.cu_q ? g.lk : p.seq_k;
+    if (kt0 >= kwrite) return;  // uniform: no barrier has run
+    const int kw0 = kt0 + 32 * kg;
+    const int key = kw0 + l32;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
+    constexpr uint32_t TILE_B = TL::ELEMS * sizeof(T);
+
+    // Items: (query head of the group, query tile), tiles from the first that sees this key
+    // tile (causal: rows i >= kt0 - coff); split s takes items s, s + splits, ....  The walk
+    // steps (gi, bi) by (splits / nblk, splits % nblk) with one carry.
+    const int rfirst = p.causal ? max(0, kt0 - g.coff) / TR : 0;
+    const int nblk = (kt0 < g.lk && g.lq > rfirst * TR) ? (g.lq + TR - 1) / TR - rfirst : 0;
+    const int items = nblk * p.group;
+    const int sp_g = nblk > 0 ? p.splits / nblk : 0, sp_b = p.splits - sp_g * nblk;
+    int gi = nblk > 0 ? split / nblk : 0, bi = split - gi * nblk;
+    const uint32_t qst = static_cast<uint32_t>(p.qs[2] * ES), dst = static_cast<uint32_t>(p.dos[2] * ES);
+    const typename TL::Offs oq = TL::offs(lane, qst), od = TL::offs(lane, dst);
+    // Head 0 of the group; head gi is gi * (head stride) bytes on.
+    const char* const qg = reinterpret_cast<const char*>(static_cast<const T*>(p.q) + g.qb + kvh * p.group * p.qs[1] +
+                                                         static_cast<int64_t>(g.q0) * p.qs[2]);
+    const char* const dg = reinterpret_cast<const char*>(static_cast<const T*>(p.dout) + g.dob +
+                                                         kvh * p.group * p.dos[1] + static_cast<int64_t>(g.q0) * p.dos[2]);
+    const int64_t qh = p.qs[1] * ES, dh = p.dos[1] * ES;
+    const float* const sg =
+        p.stats + (static_cast<int64_t>(wave) * p.hq + kvh * p.group) * p.rows_total + g.row_base;
+    auto request = [&](int gi_, int bi_, int buf) {
+        const int r0 = (rfirst + bi_) * TR;
+        const uint32_t at = lds0 + buf * 2 * TILE_B;
+        TL::request(qg + gi_ * qh, qst, r0, g.lq, p.d * ES, oq, wave, at);
+        TL::request(dg + gi_ * dh, dst, r0, g.lq, p.dval * ES, od, wave, at + TILE_B);
+        if (wave < (MK == MK_NONE ? 2 : 3))
+            dma4(dma_rsrc(sg + gi_ * p.rows_total + r0, 4u * static_cast<uint32_t>(min(TR, g.lq - r0))),
+                 4u * lane,
+                 lds0 + static_cast<uint32_t>(offsetof(SH, stats)) + static_cast<uint32_t>((buf * 3 + wave) * kWave * 4));
+    };
+    const typename TL::Addr ad = TL::addr(lane);
+    v8 kf[DC], vf[VL ? 1 : DC];
+    {
+        const T* kp = static_cast<const T*>(p.k) + g.kb + kvh * p.ks[1] + static_cast<int64_t>(g.k0) * p.ks[2];
+        const T* vp = static_cast<const T*>(p.v) + g.vb + kvh * p.vs[1] + static_cast<int64_t>(g.k0) * p.vs[2];
+#pragma unroll
+        for (int c = 0; c < DC; ++c) kf[c] = frag16<v8>(kp, p.ks[2], key, g.lk, 16 * c + 8 * h2, p.d);
+        if constexpr (VL) {
+            // Each wavefront stages and reads its own 32 keys (in order with its vmcnt wait).
+            typedef Tile<T, DP, 128> TV;
+            const uint32_t vst = static_cast<uint32_t>(p.vs[2] * ES);
+            const typename TV::Offs ov = TV::offs(lane, vst);
+            TV::request(reinterpret_cast<const char*>(vp), vst, kt0, g.lk, p.dval * ES, ov, wave,
+                        lds0 + static_cast<uint32_t>(offsetof(SH, v)));
+        } else {
+#pragma unroll
+            for (int c = 0; c < DC; ++c) vf[c] = frag16<v8>(vp, p.vs[2], key, g.lk, 16 * c + 8 * h2, p.dval);
+        }
+    }
+    f32x16 dk[DB], dv[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b) dk[b] = dv[b] = splat16(0.f);
+    typedef typename MaskRaw<MK>::type MRaw;
+
+    // One 32-row block (rows r0b ..) at LDS address qt (dO's a tile on).
+    auto block = [&](uint32_t qt, const float* st, int h, int r0b) {
+        // S starts from what is added to the scaled scores (over c2): 0, the mask's logit, or
+        // p.hidden where the row does not see the key (its P becomes exactly 0).
+        f32x16 s = splat16(0.f), dp;
+        if constexpr (MK != MK_NONE) {
+            const int64_t msz = static_cast<int64_t>(sizeof(MRaw));
+            const int64_t b0 = g.mbase + h * p.ms[1] + r0b * g.mrow;
+            const bool fast = g.mrow >= 0 && g.mkey >= 0 && kw0 + 31 < g.lk && r0b + 31 < g.lq &&
+                              (32 * g.mrow + g.lk * g.mkey) * msz < (int64_t{1} << 30) &&
+                              b0 + 31 * g.mrow + (kw0 + 31) * g.mkey < g.mend;
+            if (fast) {
+                const auto rs = buffer_rsrc(static_cast<const MRaw*>(p.mask) + b0, 0x7fffffffu);
+                const uint32_t off = static_cast<uint32_t>((4 * h2 * g.mrow + key * g.mkey) * msz);
+                MRaw raw[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int so = static_cast<int>((8 * (i / 4) + i % 4) * g.mrow * msz);
+                    if constexpr (sizeof(MRaw) == 1)
+                        raw[i] = __builtin_amdgcn_raw_buffer_load_b8(rs, off, so, 0);
+                    else if constexpr (sizeof(MRaw) == 2)
+                        raw[i] = __builtin_amdgcn_raw_buffer_load_b16(rs, off, so, 0);
+                    else
+                        raw[i] = __builtin_bit_cast(MRaw, __builtin_amdgcn_raw_buffer_load_b32(rs, off, so, 0));
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] = mask_logit_of<MK>(raw[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    s[i] = mask_at<MK>(p, g, h, min(r0b + 8 * (i / 4) + 4 * h2 + i % 4, g.lq - 1), min(key, g.lk - 1));
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 rw = *reinterpret_cast<const f32x4*>(st + 2 * kWave + 8 * q + 4 * h2);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float m = s[4 * q + e];
+                    s[4 * q + e] = rw[e] != 0.f ? 0.f : (m > kMaskedLogit ? m * p.mask_c : p.hidden);
+                }
+            }
+        }
+        // Blocks whose rows all see all 32 keys (uniform) need no per-element test.
+        if (!(kw0 + 31 < g.lk && (!p.causal || kw0 + 31 <= r0b + g.coff))) {
+            // Rows whose index (from this lane's first) is below `seen` do not see the key.
+            const int seen = key >= g.lk ? 32 : (p.causal ? key - g.coff - r0b - 4 * h2 : -1);
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (8 * (i / 4) + i % 4 < seen) s[i] = p.hidden;
+        }
+        // (Opaque lane addresses: the compiler would otherwise keep every sum it can hoist in
+        // registers across the loop, and V's fragments too.)
+        uint32_t ra = qt + ad.row, t0 = qt + ad.tr0, t1 = qt + ad.tr1;
+        uint32_t va = lds0 + static_cast<uint32_t>(offsetof(SH, v)) + 2u * 32 * kg * TL::PITCH + ad.row;
+        __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1), "+v"(va));
+#pragma unroll
+        for (int c = 0; c < DC; ++c) s = Mfma32<T>::run(TL::rows(ra, c, 0), kf[c], s);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 nd = *reinterpret_cast<const f32x4*>(st + kWave + 8 * q + 4 * h2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dp[4 * q + e] = nd[e];
+        }
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            if constexpr (VL)
+                dp = Mfma32<T>::run(TL::rows(ra, c, TILE_B), TL::rows(va, c, 0), dp);
+            else
+                dp = Mfma32<T>::run(TL::rows(ra, c, TILE_B), vf[c], dp);
+        }
+        v8 pb[2], sb[2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 l2 = *reinterpret_cast<const f32x4*>(st + 8 * q + 4 * h2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = 4 * q + e;
+                s[i] = __builtin_amdgcn_exp2f(s[i] * p.c2 - l2[e]);
+                pb[i / 8][i % 8] = from_f32<T>(s[i]);
+            }
+        }
+        if constexpr (VL) {
+            __builtin_amdgcn_sched_group_barrier(SG_DSREAD, QA, 0);
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+                if (c < DC - QA)
+                    __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 1, 0);
+                else
+                    __builtin_amdgcn_sched_group_barrier(SG_DSREAD, (4 + 2 * VA) / QA, 0);
+            }
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+                if (c < DC - VA) __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(SG_VALU, 40 / DC, 0);
+            }
+        } else {
+            __builtin_amdgcn_sched_group_barrier(SG_DSREAD, DC + 4, 0);
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 1, 0);
+            }
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(SG_VALU, 40 / DC, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // dV^T += dO^T P while dS = P (dP - D) is formed, then dK^T += Q^T dS.
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int kc = 0; kc < 2; ++kc) dv[b] = Mfma32<T>::run(TL::cols(t0, t1, kc, b, TILE_B), pb[kc], dv[b]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sb[i / 8][i % 8] = from_f32<T>(s[i] * dp[i]);
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int kc = 0; kc < 2; ++kc) dk[b] = Mfma32<T>::run(TL::cols(t0, t1, kc, b, 0), sb[kc], dk[b]);
+        // The transposed reads run four fragments ahead of the products.
+        __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2 * NFR, 1);
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 1);
+            if (i < 4 * DB - NFR) __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2, 1);
+            if (i < 2 * DB) __builtin_amdgcn_sched_group_barrier(SG_VALU, 24 / (2 * DB), 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (split < items) request(gi, bi, 0);
+    int buf = 0;
+    for (int it = split; it < items; it += p.splits) {
+        const int h = kvh * p.group + gi, r0 = (rfirst + bi) * TR;
+        gi += sp_g;
+        bi += sp_b;
+        if (bi >= nblk) {
+            bi -= nblk;
+            ++gi;
+        }
+        // This item's tiles were requested an item ago; past the barrier every wavefront's
+        // share has landed and the other buffer's reads are done.
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (it + p.splits < items) request(gi, bi, buf ^ 1);
+        if (kw0 < g.lk) {
+#pragma unroll 1
+            for (int rb = RS == 1 ? 0 : rsp; rb < RB; rb += RS) {
+                const int r0b = r0 + 32 * rb;
+                if (r0b >= g.lq || (p.causal && kw0 > r0b + 31 + g.coff)) continue;
+                const uint32_t qt = lds0 + buf * 2 * TILE_B + 2u * 32 * rb * TL::PITCH;
+                const float* st = sh.stats[buf][0] + 32 * rb;
+                block(qt, st, h, r0b);
+            }
+        }
+        buf ^= 1;
+    }
+    if constexpr (RS == 2) {
+        // The second wavefront of each key group hands its sums over through LDS.
+        static_assert(sizeof(sh.tile) >= KG * 2 * DB * 4 * kWave * sizeof(f32x4), "exchange fits the tiles");
+        __syncthreads();  // the last item's tile reads are done
+        f32x4* ex = reinterpret_cast<f32x4*>(smem) + kg * (2 * DB * 4 * kWave);
+        if (rsp == 1) {
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    ex[((2 * b) * 4 + q) * kWave + lane] =
+                        f32x4{dk[b][4 * q], dk[b][4 * q + 1], dk[b][4 * q + 2], dk[b][4 * q + 3]};
+                    ex[((2 * b + 1) * 4 + q) * kWave + lane] =
+                        f32x4{dv[b][4 * q], dv[b][4 * q + 1], dv[b][4 * q + 2], dv[b][4 * q + 3]};
+                }
+        }
+        __syncthreads();
+        if (rsp == 1) return;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 xk = ex[((2 * b) * 4 + q) * kWave + lane], xv = ex[((2 * b + 1) * 4 + q) * kWave + lane];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    dk[b][4 * q + e] += xk[e];
+                    dv[b][4 * q + e] += xv[e];
+                }
+            }
+    }
+    // Lane (l32, h2) of block b, register 4 q + e: key kw0 + l32, dim 32 b + 8 q + 4 h2 + e.
+    if (key >= kwrite) return;
+    auto quad = [](const f32x16& v, int q, float m) {
+        return f32x4{v[4 * q] * m, v[4 * q + 1] * m, v[4 * q + 2] * m, v[4 * q + 3] * m};
+    };
+    if (p.pdk) {
+        const int64_t at = ((static_cast<int64_t>(kvh) * p.splits + split) * p.keys_total + g.key_base + key) * DP;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int d = 32 * b + 8 * q + 4 * h2;
+                if (d < p.d) *reinterpret_cast<f32x4*>(p.pdk + at + d) = quad(dk[b], q, p.scale);
+                if (d < p.dval) *reinterpret_cast<f32x4*>(p.pdv + at + d) = quad(dv[b], q, 1.f);
+            }
+        return;
+    }
+    T* dkp = static_cast<T*>(p.dk) + g.dkb + kvh * p.dks[1] + static_cast<int64_t>(g.k0 + key) * p.dks[2];
+    T* dvp = static_cast<T*>(p.dv) + g.dvb + kvh * p.dvs[1] + static_cast<int64_t>(g.k0 + key) * p.dvs[2];
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int d = 32 * b + 8 * q + 4 * h2;
+            if (d < p.d) store4(dkp + d, quad(dk[b], q, p.scale));
+            if (d < p.dval) store4(dvp + d, quad(dv[b], q, 1.f));
+        }
+}
+
+// dQ of 32 RG "virtual rows" of one (sequence, K/V head): row r is query position r / G of
+// query head kvh G + r % G, so a GQA group shares every K/V tile.  Wavefront w owns row
+// group w % RG; with RG = 2 the two wavefronts of a row group take one 32-key block of
+// each tile each and add their sums at the end.  Split `ksp` takes the 64-key tiles ksp,
+// ksp + ksplit, ....
+template <typename T, int DP, int MK, int RG>
+__device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, const int tile, const int ksp,
+                                       const int bkv) {
+    constexpr int TR = 64;
+    typedef Tile<T, DP, TR> TL;
+    typedef typename TL::v8 v8;
+    constexpr int DC = DP / 16, DB = DP / 32;
+    constexpr int KS = 4 / RG;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h2 = lane >> 5, l32 = lane & 31;
+    const int rg = wave % RG, kspw = wave / RG;
+    const int seq = bkv / p.hkv, kvh = bkv - seq * p.hkv;
+    const Geo g = geo_of(p, seq);
+    const int G = p.group;
+    const int vrows = g.lq * G;
+    const int r0 = tile * 32 * RG;
+    if (r0 >= vrows || g.lk <= 0) return;  // uniform: no barrier has run
+    const int rw0 = r0 + 32 * rg;
+    const int row = rw0 + l32;
+    const int rr = min(row, vrows - 1);  // rows past the end repeat the last (never written)
+    const int pos = rr / G, h = kvh * G + (rr - pos * G);
+
+    v8 qf[DC], of[DC];
+    {
+        const T* qp = static_cast<const T*>(p.q) + g.qb + h * p.qs[1] + static_cast<int64_t>(g.q0 + pos) * p.qs[2];
+        const T* dp = static_cast<const T*>(p.dout) + g.dob + h * p.dos[1] + static_cast<int64_t>(g.q0 + pos) * p.dos[2];
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            qf[c] = frag16<v8>(qp, 0, 0, 1, 16 * c + 8 * h2, p.d);
+            of[c] = frag16<v8>(dp, 0, 0, 1, 16 * c + 8 * h2, p.dval);
+        }
+    }
+    const int64_t srow = static_cast<int64_t>(h) * p.rows_total + g.row_base + pos;
+    const int64_t splane = static_cast<int64_t>(p.hq) * p.rows_total;
+    const float l2 = p.stats[srow], nd = p.stats[splane + srow];
+    bool raw = false;
+    if constexpr (MK != MK_NONE) raw = p.stats[2 * splane + srow] != 0.f;
+    f32x16 dq[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b) dq[b] = splat16(0.f);
+
+    // Causal: keys below lim are visible to this row; those below lim_w to every row of
+    // the wavefront, none at or past kend_w to any.
+    const int lim = p.causal ? min(g.lk, pos + 1 + g.coff) : g.lk;
+    const int first = min(rw0, vrows - 1) / G, last = min(rw0 + 31, vrows - 1) / G;
+    const int lim_w = p.causal ? min(g.lk, first + 1 + g.coff) : g.lk;
+    const int kend_w = rw0 < vrows ? (p.causal ? min(g.lk, last + 1 + g.coff) : g.lk) : 0;
+    const int kend = p.causal ? min(g.lk, max(0, min(r0 + 32 * RG, vrows) - 1) / G + 1 + g.coff) : g.lk;
+    constexpr int ES = static_cast<int>(sizeof(T));
+    const uint32_t kst = static_cast<uint32_t>(p.ks[2] * ES), vst = static_cast<uint32_t>(p.vs[2] * ES);
+    const typename TL::Offs ok = TL::offs(lane, kst), ov = TL::offs(lane, vst);
+    const char* const kbase = reinterpret_cast<const char*>(static_cast<const T*>(p.k) + g.kb + kvh * p.ks[1] +
+                                                            static_cast<int64_t>(g.k0) * p.ks[2]);
+    const char* const vbase = reinterpret_cast<const char*>(static_cast<const T*>(p.v) + g.vb + kvh * p.vs[1] +
+                                                            static_cast<int64_t>(g.k0) * p.vs[2]);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
+    constexpr uint32_t TILE_B = TL::ELEMS * sizeof(T);
+    auto request = [&](int k0, int buf) {
+        TL::request(kbase, kst, k0, g.lk, p.d * ES, ok, wave, lds0 + buf * 2 * TILE_B);
+        TL::request(vbase, vst, k0, g.lk, p.dval * ES, ov, wave, lds0 + (buf * 2 + 1) * TILE_B);
+    };
+    const typename TL::Addr ad = TL::addr(lane);
+    typedef typename MaskRaw<MK>::type MRaw;
+    const int64_t moff = g.mbase + h * p.ms[1] + pos * g.mrow;  // the row's mask values
+
+    // One 32-key block (keys kb0 ..) at LDS address kt (V's a tile on).
+    auto block = [&](uint32_t kt, int kb0) {
+        f32x16 s = splat16(0.f), dp = splat16(nd);  // (s: as in bwd_dkdv)
+        if constexpr (MK != MK_NONE) {
+            // Unit key stride: four consecutive keys per load.
+            const bool vec = g.mkey == 1 && kb0 + 31 < g.lk && (p.mask_mode != KMI_MASK_PACKED || g.mpacked_ok);
+            if (vec) {
+                const MRaw* src = static_cast<const MRaw*>(p.mask) + moff + kb0 + 4 * h2;
+                struct E {
+                    MRaw e[4];
+                } x[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) __builtin_memcpy(&x[q], src + 8 * q, sizeof(E));
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] = mask_logit_of<MK>(x[i / 4].e[i % 4]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    s[i] = mask_at<MK>(p, g, h, pos, min(kb0 + 8 * (i / 4) + 4 * h2 + i % 4, g.lk - 1));
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = raw ? 0.f : (s[i] > kMaskedLogit ? s[i] * p.mask_c : p.hidden);
+        }
+        if (kb0 + 31 >= lim_w) {
+            const int rel = lim - kb0 - 4 * h2;  // keys whose index is below rel are visible
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (8 * (i / 4) + i % 4 >= rel) s[i] = p.hidden;
+        }
+        uint32_t ra = kt + ad.row, t0 = kt + ad.tr0, t1 = kt + ad.tr1;
+        __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1));  // (as in bwd_dkdv)
+#pragma unroll
+        for (int c = 0; c < DC; ++c) s = Mfma32<T>::run(TL::rows(ra, c, 0), qf[c], s);
+#pragma unroll
+        for (int c = 0; c < DC; ++c) dp = Mfma32<T>::run(TL::rows(ra, c, TILE_B), of[c], dp);
+        v8 sb[2];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(s[i] * p.c2 - l2);
+        __builtin_amdgcn_sched_group_barrier(SG_DSREAD, DC, 0);
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 1, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_VALU, 32 / DC, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sb[i / 8][i % 8] = from_f32<T>(s[i] * dp[i]);
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int kc = 0; kc < 2; ++kc) dq[b] = Mfma32<T>::run(TL::cols(t0, t1, kc, b, 0), sb[kc], dq[b]);
+        __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2 * DB < 4 ? 4 * DB : 8, 1);
+        __builtin_amdgcn_sched_group_barrier(SG_VALU, 24, 1);
+#pragma unroll
+        for (int i = 0; i < 2 * DB; ++i) {
+            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 1);
+            if (i < 2 * DB - 4) __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2, 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int kstep = p.ksplit * TR;
+    int k0 = ksp * TR;
+    if (k0 < kend) request(k0, 0);
+    int buf = 0;
+    for (; k0 < kend; k0 += kstep) {
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (as in bwd_dkdv)
+        __syncthreads();
+        if (k0 + kstep < kend) request(k0 + kstep, buf ^ 1);
+#pragma unroll 1
+        for (int kb = KS == 1 ? 0 : kspw; kb < 2; kb += KS) {
+            const int kb0 = k0 + 32 * kb;
+            if (kb0 >= kend_w) continue;
+            const uint32_t kt = lds0 + buf * 2 * TILE_B + 2u * 32 * kb * TL::PITCH;
+            block(kt, kb0);
+        }
+        buf ^= 1;
+    }
+    if constexpr (KS == 2) {
+        __syncthreads();  // the last tile's reads are done
+        f32x4* ex = reinterpret_cast<f32x4*>(smem) + rg * (DB * 4 * kWave);
+        if (kspw == 1) {
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    ex[(b * 4 + q) * kWave + lane] =
+                        f32x4{dq[b][4 * q], dq[b][4 * q + 1], dq[b][4 * q + 2], dq[b][4 * q + 3]};
+        }
+        __syncthreads();
+        if (kspw == 1) return;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 x = ex[(b * 4 + q) * kWave + lane];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dq[b][4 * q + e] += x[e];
+            }
+    }
+    // Lane (l32, h2) of block b, register 4 q + e: row rw0 + l32, dim 32 b + 8 q + 4 h2 + e.
+    if (row >= vrows) return;
+    T* dst = static_cast<T*>(p.dq) + g.dqb + h * p.dqs[1] + static_cast<int64_t>(g.q0 + pos) * p.dqs[2];
+    float* part = p.pdq ? p.pdq + ((static_cast<int64_t>(h) * p.ksplit + ksp) * p.rows_total + g.row_base + pos) * DP
+                        : nullptr;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int d = 32 * b + 8 * q + 4 * h2;
+            if (d >= p.d) continue;
+            const f32x4 v = f32x4{dq[b][4 * q] * p.scale, dq[b][4 * q + 1] * p.scale, dq[b][4 * q + 2] * p.scale,
+                                  dq[b][4 * q + 3] * p.scale};
+            if (part)
+                *reinterpret_cast<f32x4*>(part + d) = v;
+            else
+                store4(dst + d, v);
+        }
+}
+
+// Wavefronts per SIMD the kernel is held to (165 and 237 registers, no spills, unmasked).
+constexpr int bwd_waves(int dp) { return dp <= 64 ? 3 : 2; }
+
+// Both gradient passes in one launch, their workgroups interleaved in proportion (neither
+// reads the other's output).  Workgroups are dealt to the eight XCDs in turn (block b runs
+// on XCD b % 8), so the interleaving is done within each XCD's blocks and a pass's work
+// item number keeps its residue: items with one (sequence, K/V head) fastest stay on few
+// XCDs, whose L2 then holds what they walk over.  Item order: heaviest tiles first.
+template <typename T, int DP, int MK>
+__global__ __launch_bounds__(BWD_THREADS, bwd_waves(DP)) void attn_bwd_tile_kernel(const BwdParams p, const BwdGrid gr) {
+    __shared__ __align__(1024) unsigned char sh[sizeof(DkdvShared<T, DP>) > 4 * sizeof(T) * Tile<T, DP, 64>::ELEMS
+                                                  ? sizeof(DkdvShared<T, DP>)
+                                                  : 4 * sizeof(T) * Tile<T, DP, 64>::ELEMS];
+    const int x = blockIdx.x & 7, s = blockIdx.x >> 3;
+    const int per_q = (gr.nq + 7) >> 3, per_k = (gr.nk + 7) >> 3, tot = per_q + per_k;
+    const int q0 = static_cast<int>(static_cast<int64_t>(s) * per_q / tot);
+    const int q1 = static_cast<int>(static_cast<int64_t>(s + 1) * per_q / tot);
+    const int units = p.batch * p.hkv;
+    if (q1 > q0) {
+        const int i = 8 * q0 + x;
+        if (i >= gr.nq) return;
+        const int rest = i / units, unit = i - rest * units;
+        const int t = rest / p.ksplit, ks = rest - t * p.ksplit;
+        const int tile = p.causal ? gr.tiles_q - 1 - t : t;
+        if (gr.half_q)
+            bwd_dq<T, DP, MK, 2>(p, sh, tile, ks, unit);
+        else
+            bwd_dq<T, DP, MK, 4>(p, sh, tile, ks, unit);
+    } else {
+        const int i = 8 * (s - q0) + x;
+        if (i >= gr.nk) return;
+        const int rest = i / units, unit = i - rest * units;
+        const int t = rest / p.splits, sp = rest - t * p.splits;
+        if constexpr (DP <= 64) {
+            if (gr.half_k) {
+                bwd_dkdv<T, DP, MK, 2>(p, sh, t, sp, unit);
+                return;
+            }
+        }
+        bwd_dkdv<T, DP, MK, 4>(p, sh, t, sp, unit);
+    }
+}
+
+template <typename T, int DP, int MK>
+hipError_t launch_tile_mk(const BwdParams& p, const BwdGrid& gr, hipStream_t s) {
+    const int per = (gr.nq + 7) / 8 + (gr.nk + 7) / 8;
+    const dim3 grid(static_cast<unsigned>(8 * per)), block(BWD_THREADS);
+    hipLaunchKernelGGL((attn_bwd_tile_kernel<T, DP, MK>), grid, block, 0, s, p, gr);
+    return hipGetLastError();
+}
+
+template <typename T, int DP>
+hipError_t launch_tile(const BwdParams& p, const BwdGrid& gr, int mk, hipStream_t s) {
+    switch (mk) {
+        case MK_NONE: return launch_tile_mk<T, DP, MK_NONE>(p, gr, s);
+        case MK_BOOL: return launch_tile_mk<T, DP, MK_BOOL>(p, gr, s);
+        case MK_BF16: return launch_tile_mk<T, DP, MK_BF16>(p, gr, s);
+        case MK_F16: return launch_tile_mk<T, DP, MK_F16>(p, gr, s);
+        default: return launch_tile_mk<T, DP, MK_F32>(p, gr, s);
+    }
+}
+
+}  // namespace bwd
+}  // namespace kmi

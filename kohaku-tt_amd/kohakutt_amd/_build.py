@@ -38,6 +38,7 @@ HIP_SOURCES = [
     *[f"attention_d{d}.hip" for d in (32, 64, 96, 128, 192, 256)],
     "attention_pipe.hip",
     "attention_bwd.hip",
+    *[f"attention_bwd_d{d}.hip" for d in (32, 64, 96, 128)],
 ]
 HIP_FLAGS = [
     f"--offload-arch={ARCH}",

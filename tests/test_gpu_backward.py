@@ -76,6 +76,54 @@ def test_flash_backward_meets_the_float64_ruler(native, dev, case, dtype):
         assert (gg.double() - rr).abs().max().item() <= 3e-2 * max(scale, 1.0), (name, scale)
 
 
+# The 32x32 tiles' edges: one row / key past or short of a 32-row block, a 64-row tile and a
+# 128-key workgroup; head dims padded within a 16-byte-chunk row (40, 96); splits of dK / dV
+# (few key tiles, many query blocks) and of dQ (one query row, many keys).
+TILE_EDGES = [
+    (1, 2, 1, 33, 31, 40, True),
+    (1, 3, 1, 65, 129, 96, False),
+    (2, 4, 2, 64, 63, 128, True),
+    (1, 1, 1, 127, 127, 64, True),
+    (1, 7, 1, 97, 97, 32, True),
+    (1, 8, 2, 1100, 70, 128, False),
+    (1, 6, 2, 700, 700, 64, True),
+    (1, 1, 1, 3, 2100, 64, False),
+]
+
+
+@pytest.mark.parametrize("case", TILE_EDGES, ids=lambda c: "x".join(map(str, c)))
+def test_tile_edges_meet_the_float64_ruler(native, dev, case):
+    test_flash_backward_meets_the_float64_ruler(native, dev, case, torch.bfloat16)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.2])
+@pytest.mark.parametrize("d", [64, 128])
+def test_backward_scale_of_any_sign(native, dev, scale, d):
+    """Score accumulators start from mask logits over the scale: a zero and a negative scale
+    with an additive mask, and a negative one with a causal call, against float64."""
+    print(f"scale {scale} d {d}", flush=True)
+    g = C.gen(970 + d)
+    q, k, v, go = (C.randn(g, 1, 2, 70, d) for _ in range(4))
+    mask = torch.randn(1, 1, 70, 70, generator=g).masked_fill(torch.rand(1, 1, 70, 70, generator=g) < 0.2, -torch.inf)
+    mask[..., 0] = 0.0
+    for m, causal in ((mask.bfloat16(), False), (None, True))[: 1 if scale == 0.0 else 2]:
+        ts = [t.to(dev).requires_grad_() for t in (q, k, v)]
+        out = F.scaled_dot_product_attention(
+            *ts, attn_mask=None if m is None else m.to(dev), is_causal=causal, scale=scale
+        )
+        out.backward(go.to(dev))
+        got = [t.grad.cpu().double() for t in ts]
+        rs = [t.double().requires_grad_() for t in (q, k, v)]
+        bias = torch.zeros(70, 70, dtype=torch.float64) if m is None else m.double()
+        if causal:
+            bias = bias.masked_fill(~torch.ones(70, 70, dtype=torch.bool).tril(), -torch.inf)
+        (torch.softmax(rs[0] @ rs[1].transpose(-1, -2) * scale + bias, -1) @ rs[2]).backward(go.double())
+        want = [t.grad for t in rs]
+        for name, a, b in zip(("dq", "dk", "dv"), got, want):
+            # P and dS round to bf16 (2^-9 each), then the sums once more: 2^-7 of the largest value.
+            assert (a - b).abs().max().item() <= 2.0**-7 * max(b.abs().max().item(), 1e-6), (name, scale, causal)
+
+
 def test_gqa_key_gradients_sum_their_query_heads(native, dev):
     """dk / dv of a K/V head equal the sum over its query heads of the per-head gradients
     (the same call with K/V repeated per query head, reduced afterwards)."""
