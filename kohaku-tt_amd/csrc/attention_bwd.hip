@@ -8,8 +8,8 @@
 // mask (the forward's modes), GQA, any head dim that is a multiple of 8 up to 256 (padded
 // to DP with zeros in registers), bf16 / fp16:
 //
-//   attn_bwd_rowdot  row statistics of every query row and head: the base-2 lse and the
-//                    negated row dots -D, D = sum_d dO O (fp32)
+//   attn_bwd_rowdot  the negated row dots -D, D = sum_d dO O (fp32), of every query row and
+//                    head
 //   gradients        one launch of both passes, their workgroups interleaved:
 //     dQ             per (sequence, row block, key split): over the key tiles it sees
 //                    P = exp2(c S + mask - lse2), dP = dO V^T, dS = P (dP - D),
@@ -395,7 +395,7 @@ constexpr int kSumBatch = 8;
 // dQ: a workgroup takes QW query rows (16 per wavefront).
 constexpr int QW = 64;
 
-// The row dots D = sum(dO * O) (fp32) of every query row and head, read by both gradient
+// The negated row dots -D, D = sum(dO * O) (fp32), of every query row and head, read by both gradient
 // passes, which run concurrently: one workgroup per (sequence, query head, QW-row block),
 // 16 rows per wavefront.  A row's CH = dval / 8 16-byte chunks go to CP (CH rounded up to
 // a power of two) adjacent lanes, so that each load instruction reads whole rows
@@ -439,15 +439,7 @@ __global__ __launch_bounds__(BWD_THREADS) void attn_bwd_rowdot(const BwdParams p
 #pragma unroll
         for (int o = CP / 2; o > 0; o >>= 1) dot += __shfl_xor(dot, o, kWave);
         const int row = row0 + RPI * i;
-        if (c == 0 && row < g.lq) {
-            const int64_t at = h * p.rows_total + g.row_base + row, plane = p.hq * p.rows_total;
-            float l2;
-            bool raw;
-            row_stats(p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + row) * p.ls[2]], true, l2, raw);
-            p.stats[at] = l2;
-            p.stats[plane + at] = -dot;
-            if (p.mask_mode != KMI_MASK_NONE) p.stats[2 * plane + at] = raw ? 1.f : 0.f;
-        }
+        if (c == 0 && row < g.lq) p.nd[h * p.rows_total + g.row_base + row] = -dot;
     }
 }
 
@@ -780,7 +772,12 @@ const char* check_bwd(const kmi_attn_bwd_args* a) {
 int64_t rows_total_of(const kmi_attn_bwd_args* a) { return a->cu_seqlens_q ? a->total_q : a->batch * a->seq_q; }
 int64_t keys_total_of(const kmi_attn_bwd_args* a) { return a->cu_seqlens_q ? a->total_k : a->batch * a->seq_k; }
 
-// Split rules of the head dims padded past 128 (attn_bwd_grads).
+// Split rules of attn_bwd_grads (head dims padded past 128; the others' workspace figure
+// too, see bwd_ws_bytes): a dK / dV workgroup takes at most kBwdItemsPerWg64 (query head,
+// 32-row block) items up to head dim 64 and kBwdItemsPerWg128 at 128 (in proportion fewer
+// past it), a dQ workgroup at most kBwdTilesPerWg 32-key tiles; below kBwdMinWgs workgroups
+// of a kind, splits go down to kBwdMinItems items (or tiles) each.
+constexpr int64_t kBwdItemsPerWg64 = 40;
 constexpr int64_t kBwdItemsPerWg128 = 22;
 constexpr int64_t kBwdTilesPerWg = 32;
 constexpr int64_t kBwdMinWgs = 512;
@@ -803,6 +800,20 @@ int bwd_ksplit_override() {
         return e ? std::atoi(e) : 0;
     }();
     return v;
+}
+
+// attn_bwd_grads' dK / dV splits over the items of a 64-key tile and dQ splits over the
+// 32-key tiles of a 64-row block.
+void grads_splits(const kmi_attn_bwd_args* a, int& splits, int& ksplit) {
+    const int64_t dp = padded_head_dim(std::max(a->head_dim, bwd_value_dim(a)));
+    const int64_t per_wg = dp <= 64 ? kBwdItemsPerWg64 : ceil_div(kBwdItemsPerWg128 * 128, dp);
+    const int64_t items = (a->heads_q / a->heads_kv) * ceil_div(a->seq_q, BT), tiles = ceil_div(a->seq_k, BT);
+    splits = static_cast<int>(
+        bwd_split_count(a->batch * a->heads_kv * ceil_div(a->seq_k, KW), items, per_wg, kBwdMaxSplits));
+    ksplit = static_cast<int>(
+        bwd_split_count(a->batch * a->heads_q * ceil_div(a->seq_q, QW), tiles, kBwdTilesPerWg, kBwdMaxKsplit));
+    if (bwd_ksplit_override() > 0)
+        ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
 }
 
 struct BwdPlan {
@@ -838,13 +849,7 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     const int64_t units = a->batch * a->heads_kv, G = a->heads_q / a->heads_kv;
     pl.tile = dp <= 128;
     if (!pl.tile) {
-        const int64_t per_wg = ceil_div(kBwdItemsPerWg128 * 128, dp), tiles = ceil_div(a->seq_k, BT);
-        pl.splits = static_cast<int>(
-            bwd_split_count(units * ceil_div(a->seq_k, KW), G * ceil_div(a->seq_q, BT), per_wg, kBwdMaxSplits));
-        pl.ksplit = static_cast<int>(bwd_split_count(a->batch * a->heads_q * ceil_div(a->seq_q, QW), tiles,
-                                                     kBwdTilesPerWg, kBwdMaxKsplit));
-        if (bwd_ksplit_override() > 0)
-            pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
+        grads_splits(a, pl.splits, pl.ksplit);
         return pl;
     }
     pl.grid.half_k = dp <= 64;
@@ -868,24 +873,32 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     return pl;
 }
 
-// Workspace floats: the row statistics (padded to 16 bytes); with splits the dK / dV
+// Workspace floats: the row dots (padded to 16 bytes); with splits the dK / dV
 // partials; with key splits the dQ partials.
 struct BwdLayout {
-    size_t stats, part, pdq;
+    size_t nd, part, pdq;
 };
 
-BwdLayout bwd_layout(const kmi_attn_bwd_args* a, const BwdPlan& pl) {
+BwdLayout bwd_layout(const kmi_attn_bwd_args* a, int splits, int ksplit) {
     BwdLayout l{};
     const int64_t dp = padded_head_dim(std::max(a->head_dim, bwd_value_dim(a)));
-    const int64_t planes = a->mask_mode == KMI_MASK_NONE ? 2 : 3;
-    l.stats = static_cast<size_t>(ceil_div(planes * a->heads_q * rows_total_of(a), 4) * 4);
+    l.nd = static_cast<size_t>(ceil_div(a->heads_q * rows_total_of(a), 4) * 4);
     // One split sums the query heads of a K/V head in its registers and writes dK / dV.
-    if (pl.splits > 1) l.part = static_cast<size_t>(a->heads_kv * pl.splits * keys_total_of(a) * dp);
-    if (pl.ksplit > 1) l.pdq = static_cast<size_t>(a->heads_q * pl.ksplit * rows_total_of(a) * dp);
+    if (splits > 1) l.part = static_cast<size_t>(a->heads_kv * splits * keys_total_of(a) * dp);
+    if (ksplit > 1) l.pdq = static_cast<size_t>(a->heads_q * ksplit * rows_total_of(a) * dp);
     return l;
 }
 
-size_t bwd_ws_bytes(const BwdLayout& l) { return (l.stats + 2 * l.part + l.pdq) * sizeof(float); }
+size_t layout_bytes(const BwdLayout& l) { return (l.nd + 2 * l.part + l.pdq) * sizeof(float); }
+
+// The workspace figure: what the plan needs, and never less than attn_bwd_grads' rules give
+// (callers keep buffers sized by it, so a plan with fewer splits does not shrink it).
+size_t bwd_ws_bytes(const kmi_attn_bwd_args* a) {
+    const BwdPlan pl = bwd_plan(a);
+    int splits, ksplit;
+    grads_splits(a, splits, ksplit);
+    return std::max(layout_bytes(bwd_layout(a, pl.splits, pl.ksplit)), layout_bytes(bwd_layout(a, splits, ksplit)));
+}
 
 // The gradient kernel of head dims padded past 128.
 template <typename T, int DP, int MK>
@@ -914,7 +927,7 @@ hipError_t launch_grads_mask(const BwdParams& p, int mk, hipStream_t s) {
     }
 }
 
-// The call's launches: row statistics, gradients, split sums.
+// The call's launches: row dots, gradients, split sums.
 template <typename T, int DP>
 hipError_t launch_bwd(const BwdParams& p, const BwdPlan& pl, int mk, hipStream_t s) {
     const int64_t nqb = ceil_div(p.seq_q, QW);
@@ -959,7 +972,7 @@ extern "C" int kmi_attn_bwd_workspace_bytes(const kmi_attn_bwd_args* a, size_t* 
     using namespace kmi::bwd;
     if (!bytes) return fail(KMI_EINVAL, "kmi_attn_bwd_workspace_bytes: null bytes");
     if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd_workspace_bytes: ") + why);
-    *bytes = bwd_ws_bytes(bwd_layout(a, bwd_plan(a)));
+    *bytes = bwd_ws_bytes(a);
     return KMI_OK;
 }
 
@@ -968,8 +981,8 @@ extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t 
     using namespace kmi::bwd;
     if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd: ") + why);
     const BwdPlan pl = bwd_plan(a);
-    const BwdLayout l = bwd_layout(a, pl);
-    const size_t need = bwd_ws_bytes(l);
+    const BwdLayout l = bwd_layout(a, pl.splits, pl.ksplit);
+    const size_t need = bwd_ws_bytes(a);
     if (!workspace || workspace_bytes < need || reinterpret_cast<uintptr_t>(workspace) % 16)
         return fail(KMI_EWORKSPACE, "kmi_attn_bwd: workspace missing or smaller than kmi_attn_bwd_workspace_bytes");
     BwdParams p{};
@@ -984,14 +997,13 @@ extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t 
     p.dv = a->grad_v;
     p.splits = pl.splits;
     p.ksplit = pl.ksplit;
-    // Partials start 16-byte aligned after the row statistics (DP is a multiple of 4).
-    p.stats = static_cast<float*>(workspace);
-    p.nd = p.stats + a->heads_q * rows_total_of(a);
+    // Partials start 16-byte aligned after the row dots (DP is a multiple of 4).
+    p.nd = static_cast<float*>(workspace);
     if (l.part) {
-        p.pdk = p.stats + l.stats;
+        p.pdk = p.nd + l.nd;
         p.pdv = p.pdk + l.part;
     }
-    if (l.pdq) p.pdq = p.stats + l.stats + 2 * l.part;
+    if (l.pdq) p.pdq = p.nd + l.nd + 2 * l.part;
     for (int i = 0; i < 3; ++i) {
         p.qs[i] = a->q_stride[i];
         p.ks[i] = a->k_stride[i];

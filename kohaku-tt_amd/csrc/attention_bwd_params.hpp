@@ -18,10 +18,7 @@ struct BwdParams {
     const void *q, *k, *v, *o, *dout;
     const float* lse;
     void *dq, *dk, *dv;
-    // Row statistics [3][hq][rows_total] fp32: base-2 lse, the negated row dots -D, and
-    // (masked calls) whether the row ran over its raw scores.
-    float* stats;
-    const float* nd;  // the -D plane of stats
+    float* nd;  // [hq][rows_total] fp32 negated row dots -D
     // dK / dV partials [hkv][splits][keys_total][DP] fp32 (splits > 1), else null.
     float *pdk, *pdv;
     // dQ partials [hq][ksplit][rows_total][DP] fp32 (ksplit > 1), else null.

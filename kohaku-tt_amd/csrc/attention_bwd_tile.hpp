@@ -277,17 +277,19 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
     const char* const dg = reinterpret_cast<const char*>(static_cast<const T*>(p.dout) + g.dob +
                                                          kvh * p.group * p.dos[1] + static_cast<int64_t>(g.q0) * p.dos[2]);
     const int64_t qh = p.qs[1] * ES, dh = p.dos[1] * ES;
-    const float* const sg =
-        p.stats + (static_cast<int64_t>(wave) * p.hq + kvh * p.group) * p.rows_total + g.row_base;
+    const float* const sg = p.nd + static_cast<int64_t>(kvh) * p.group * p.rows_total + g.row_base;
+    const float* const lg = p.lse + g.lb + kvh * p.group * p.ls[1] + static_cast<int64_t>(g.q0) * p.ls[2];
+    float lse_n = 0.f;  // wavefront 0: the requested item's lse, row `lane`
     auto request = [&](int gi_, int bi_, int buf) {
         const int r0 = (rfirst + bi_) * TR;
         const uint32_t at = lds0 + buf * 2 * TILE_B;
         TL::request(qg + gi_ * qh, qst, r0, g.lq, p.d * ES, oq, wave, at);
         TL::request(dg + gi_ * dh, dst, r0, g.lq, p.dval * ES, od, wave, at + TILE_B);
-        if (wave < (MK == MK_NONE ? 2 : 3))
-            dma4(dma_rsrc(sg + gi_ * p.rows_total + r0, 4u * static_cast<uint32_t>(min(TR, g.lq - r0))),
-                 4u * lane,
-                 lds0 + static_cast<uint32_t>(offsetof(SH, stats)) + static_cast<uint32_t>((buf * 3 + wave) * kWave * 4));
+        if (wave == 0) {
+            dma4(dma_rsrc(sg + gi_ * p.rows_total + r0, 4u * static_cast<uint32_t>(min(TR, g.lq - r0))), 4u * lane,
+                 lds0 + static_cast<uint32_t>(offsetof(SH, stats)) + static_cast<uint32_t>((buf * 3 + 1) * kWave * 4));
+            lse_n = lg[gi_ * p.ls[1] + min(r0 + lane, g.lq - 1) * p.ls[2]];
+        }
     };
     const typename TL::Addr ad = TL::addr(lane);
     v8 kf[DC], vf[VL ? 1 : DC];
@@ -458,6 +460,13 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
         // This item's tiles were requested an item ago; past the barrier every wavefront's
         // share has landed and the other buffer's reads are done.
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (wave == 0) {
+            float l2;
+            bool raw;
+            row_stats(lse_n, r0 + lane < g.lq, l2, raw);
+            sh.stats[buf][0][lane] = l2;
+            if constexpr (MK != MK_NONE) sh.stats[buf][2][lane] = raw ? 1.f : 0.f;
+        }
         __syncthreads();
         if (it + p.splits < items) request(gi, bi, buf ^ 1);
         if (kw0 < g.lk) {
@@ -569,11 +578,10 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
             of[c] = frag16<v8>(dp, 0, 0, 1, 16 * c + 8 * h2, p.dval);
         }
     }
-    const int64_t srow = static_cast<int64_t>(h) * p.rows_total + g.row_base + pos;
-    const int64_t splane = static_cast<int64_t>(p.hq) * p.rows_total;
-    const float l2 = p.stats[srow], nd = p.stats[splane + srow];
-    bool raw = false;
-    if constexpr (MK != MK_NONE) raw = p.stats[2 * splane + srow] != 0.f;
+    const float nd = p.nd[static_cast<int64_t>(h) * p.rows_total + g.row_base + pos];
+    float l2;
+    bool raw;
+    row_stats(p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + pos) * p.ls[2]], true, l2, raw);
     f32x16 dq[DB];
 #pragma unroll
     for (int b = 0; b < DB; ++b) dq[b] = splat16(0.f);
