@@ -77,6 +77,15 @@ bool pipe_enabled() {
     return v;
 }
 
+// KMI_ATTN_TILE=0 (read once) keeps prefill calls off attn_tile_kernel.
+bool tile_enabled() {
+    static const bool v = [] {
+        const char* e = std::getenv("KMI_ATTN_TILE");
+        return !(e && std::atoi(e) == 0);
+    }();
+    return v;
+}
+
 // KMI_ATTN_DECODE_FUSED=0 (read once) merges decode splits in a separate launch.
 bool decode_fused_enabled() {
     static const bool v = [] {
@@ -100,6 +109,51 @@ int splits_override() {
 bool nqb_allowed(int dp, int nqb, bool masked) {
     if (masked) return nqb == 1 || (nqb == 2 && dp == 64);
     return nqb == 1 || (nqb == 2 && dp <= 128) || (nqb == 4 && dp == 64);
+}
+
+// Whether attn_tile_kernel takes a planned call: 4 (128 rows a workgroup), 2 (64 rows) or 0
+// (the plan's other kernel).  The line lies where the workgroups fill the chip, two per CU:
+// below it the other kernels' 16- to 64-row workgroups win by their number.  w4 and w2 are
+// the workgroups of 128 and 64 rows.  Measured (us, other kernel / 128 rows / 64 rows):
+//   head dims 96 and 128, causal: 2x16x1000 (w4 256) 29 / 25 / 21, 4x16x1000 (512) 50 / 30 /
+//     35, 2x32/8x3000 (1504) 262 / 158 / 187; 1x16x1000 (w2 256) 17 / 24 / 18
+//   not causal: 4x16x512 (w4 256) 26 / 17 / 18, 24x4396 (840) 361 / 266 / 291, 2x16x512 (w2
+//     256) 15 / 15 / 12; up to 128 keys the row split stays ahead (2x10x4096/77 15 / 20 / 23)
+//   additive mask: 4x16x1000 169 / 77 / 68, 1x16x1000 (w2 256) 46 / 61 / 28
+//   padding mask: 2x16x2000 282 / 79 / 119, 4x16x512 (w4 256) 55 / 25 / 20
+//   head dims up to 64, not causal: 4x16x512 (w4 256) 15 / 11 / 11, 4x16x1000 (512) 36 / 26 /
+//     29, 2x10x4096 (640: a second round a quarter full) 114 / 123 / 115; up to 256 keys the
+//     row split stays ahead (32x12x197 15 / 17 / 21)
+//   causal (attn_pipe_kernel at 64): 8x16x700 (w4 768) 22 / 22 / 24, 4x32/8x3576 (3584) 300 /
+//     257 / 296
+//   additive mask: 16x2048 (w4 256) 80 / 71 / 45, 4x16x1000 (512) 89 / 50 / 57
+//   head dims past 128 (64 rows): 16x1600 170 / 77, 2x8x500 (w2 128) 24 / 19, causal 18 / 19
+int tile_row_groups(const kmi_attn_args* a, const Plan& pl, int dp) {
+    if (pl.decode || pl.splits > 1 || nqb_override() != 0 || !tile_enabled()) return 0;
+    const int64_t G = a->heads_q / a->heads_kv;
+    auto wgs = [&](int64_t rows) {
+        return a->cu_seqlens_q ? ceil_div(a->total_q * G, rows) * a->heads_kv
+                               : ceil_div(a->seq_q * G, rows) * a->batch * a->heads_kv;
+    };
+    const int64_t w4 = wgs(128), w2 = wgs(64);
+    const bool masked = a->mask_mode != KMI_MASK_NONE;
+    // A mask that depends on the key alone skips whole tiles in every row.
+    const bool by_key = a->mask_mode == KMI_MASK_STRIDED && a->mask_stride[1] == 0 && a->mask_stride[2] == 0;
+    if (dp > 128) return w2 >= (a->causal ? 192 : 128) ? 2 : 0;
+    if (masked) {
+        if (w4 >= (by_key ? 320 : 448) && (by_key || dp <= 64)) return 4;
+        return w2 >= (by_key ? 128 : 192) ? 2 : 0;
+    }
+    if (dp > 64) {
+        if (!a->causal && a->seq_k <= kRsTiles * WN) return 0;
+        if (w4 >= (a->causal ? 448 : 256)) return 4;
+        return w2 >= (a->causal ? 384 : 256) ? 2 : 0;
+    }
+    if (pl.rs) return 0;
+    if (pl.pipe) return w4 >= 1024 && a->seq_k >= 512 ? 4 : 0;
+    // (Two workgroups per CU: 512 a round; a last round that is mostly empty loses the gain.)
+    if (w4 >= 1024 || (w4 >= 448 && (w4 <= 512 || w4 >= 716))) return 4;
+    return w4 < 448 && w2 >= 400 ? 2 : 0;
 }
 
 Plan make_plan(const kmi_attn_args* a) {
@@ -191,6 +245,12 @@ Plan make_plan(const kmi_attn_args* a) {
     const bool span32 = a->seq_k * std::max<int64_t>({a->k_stride[2], a->v_stride[2], 64}) * 2 < (int64_t{1} << 31);
     pl.pipe = a->causal && !pl.decode && !pl.rs && pl.splits == 1 && a->mask_mode == KMI_MASK_NONE && !a->cu_seqlens_q &&
               !a->key_lengths && a->head_dim == 64 && value_dim(a) == 64 && out16 && span32 && pipe_enabled();
+    pl.row_groups = tile_row_groups(a, pl, dp);
+    if (pl.row_groups > 0) {
+        pl.tile = true;
+        pl.pipe = pl.rs = false;
+        pl.nx = static_cast<int>(ceil_div(vrows, 32 * pl.row_groups));
+    }
     pl.rows_total = a->cu_seqlens_q ? a->total_q : a->batch * a->seq_q;
     pl.ws_bytes = 0;
     return pl;
@@ -200,6 +260,16 @@ Plan make_plan(const kmi_attn_args* a) {
 template <typename T>
 hipError_t launch_dim(const AttnParams& p, const Plan& pl, hipStream_t s) {
     if (pl.pipe) return launch_pipe<T>(p, s);
+    if (pl.tile) {
+        switch (padded_head_dim(std::max(p.d, p.dv))) {
+            case 32: return launch_tile<T, 32>(p, pl.row_groups, s);
+            case 64: return launch_tile<T, 64>(p, pl.row_groups, s);
+            case 96: return launch_tile<T, 96>(p, pl.row_groups, s);
+            case 128: return launch_tile<T, 128>(p, pl.row_groups, s);
+            case 192: return launch_tile<T, 192>(p, pl.row_groups, s);
+            default: return launch_tile<T, 256>(p, pl.row_groups, s);
+        }
+    }
     switch (padded_head_dim(std::max(p.d, p.dv))) {
         case 32: return launch_all<T, 32>(p, pl, s);
         case 64: return launch_all<T, 64>(p, pl, s);

@@ -100,22 +100,6 @@ __device__ __forceinline__ V head_frag(const T* row, int col, int d) {
     return __builtin_bit_cast(V, col < d ? x : u32x4{0u, 0u, 0u, 0u});
 }
 
-// Where sequence `seq`'s block of a block-packed mask starts (host-computed offsets when
-// given, else the block sizes of the sequences before it added up).
-__device__ __forceinline__ int64_t packed_block_offset(const AttnParams& p, int seq) {
-    if (p.mask_off) return p.mask_off[seq];
-    int64_t off = 0;
-    for (int s = 0; s < seq; ++s) {
-        const int a0 = min(max(p.cu_q[s], 0), p.total_q);
-        const int a1 = min(max(p.cu_q[s + 1], a0), p.total_q);
-        const int b0 = min(max(p.cu_k[s], 0), p.total_k);
-        const int b1 = min(max(p.cu_k[s + 1], b0), p.total_k);
-        off += static_cast<int64_t>(a1 - a0) * (b1 - b0);
-    }
-    return off;
-}
-
-
 // D: the padded head dim (a multiple of 32; the call's own head dim, a multiple of 8, is
 // AttnParams::d and the columns past it are zeros in registers and LDS).
 // Unmasked, head-dim-64 tiles of 32 keys and 32 or 64 rows take K and V from global memory

@@ -95,10 +95,27 @@ struct AttnParams {
     unsigned long long* ctr;
 };
 
+// Where sequence `seq`'s block of a block-packed mask starts (host-computed offsets when
+// given, else the block sizes of the sequences before it added up).
+__device__ __forceinline__ int64_t packed_block_offset(const AttnParams& p, int seq) {
+    if (p.mask_off) return p.mask_off[seq];
+    int64_t off = 0;
+    for (int s = 0; s < seq; ++s) {
+        const int a0 = min(max(p.cu_q[s], 0), p.total_q);
+        const int a1 = min(max(p.cu_q[s + 1], a0), p.total_q);
+        const int b0 = min(max(p.cu_k[s], 0), p.total_k);
+        const int b1 = min(max(p.cu_k[s + 1], b0), p.total_k);
+        off += static_cast<int64_t>(a1 - a0) * (b1 - b0);
+    }
+    return off;
+}
+
 struct Plan {
     bool decode;  // attn_decode_kernel: per-wavefront key ranges, fp32 partials + merge
     bool rs;      // row split: short key ranges, one row block per wavefront
     bool rs_shared;  // row split with the unit's key tiles (at most four) staged in LDS once
+    bool tile;       // attn_tile_kernel: 32x32x16 MFMAs (attention_tile.hpp)
+    int row_groups;  // of attn_tile_kernel: 4 (128 rows a workgroup) or 2 (64); 0 otherwise
     bool pipe;       // attn_pipe_kernel: head dim 64, unmasked, dense, one split (attention_pipe.hip)
     int nqb, nx, splits, tiles_per_split;
     int64_t rows_total;
@@ -118,6 +135,11 @@ hipError_t launch_all(const AttnParams& p, const Plan& pl, hipStream_t stream);
 // different streams never share a word), or null when a call over `units` units must
 // merge in a separate launch.
 unsigned long long* decode_counters(hipStream_t stream, int64_t units);
+
+// Enqueues attn_tile_kernel for a call the plan gave it (instantiated per padded head dim
+// in attention_tile_d<D>.hip).
+template <typename T, int DP>
+hipError_t launch_tile(const AttnParams& p, int row_groups, hipStream_t stream);
 
 // Enqueues attn_pipe_kernel for a call the plan gave it (instantiated in attention_pipe.hip).
 template <typename T>

@@ -1,0 +1,149 @@
+"""The 32x32x16 tile forward (attn_tile_kernel) against float64, at sizes its plan takes:
+row and key counts one off its 32-row groups, 64- and 128-row workgroups and 32- to 128-key
+tiles, GQA, causal, masks (rows that keep no key among them), key lengths, packed ragged
+batches, every padded head dim, a value head dim of its own, and scales of any sign."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def _attend(q, k, v, bias, scale):
+    """float64 attention and its lse; a row whose every key is masked is over its raw scores
+    and its lse carries the -5e5 offset (bias: -inf where masked)."""
+    s = q.double() @ k.double().transpose(-1, -2).contiguous() * scale
+    if bias is not None:
+        b = bias.double()
+        dead = (b == -math.inf).all(-1, keepdim=True)
+        s = s + torch.where(dead, torch.zeros_like(b), b)
+    p = torch.softmax(s, -1)
+    lse = torch.logsumexp(s, -1)
+    if bias is not None:
+        lse = lse - 5e5 * dead.squeeze(-1)
+    return p @ v.double(), p @ v.double().abs(), lse
+
+
+HALF_ULP = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}
+
+
+def _close(got, want, weight, dtype):
+    # P rounds to the operand type (half an ulp of each weight), its row sum is of the rounded
+    # weights (the same again at most), and the result rounds once: three half ulps of sum(P |v|).
+    err = (got.double() - want).abs()
+    bound = 3 * HALF_ULP[dtype] * weight + 1e-6
+    assert torch.isfinite(got).all() and (err <= bound).all(), (err / bound).max().item()
+
+
+CASES = [
+    # b, hq, hk, sq, sk, d, causal, mask, dtype
+    (16, 16, 16, 129, 131, 128, False, None, torch.bfloat16),
+    (16, 28, 4, 65, 65, 128, True, None, torch.bfloat16),
+    (4, 24, 24, 127, 257, 96, False, None, torch.float16),
+    (2, 12, 2, 700, 700, 128, True, None, torch.float16),
+    (8, 16, 16, 513, 300, 64, False, None, torch.bfloat16),
+    (8, 12, 12, 300, 297, 40, False, None, torch.float16),
+    (8, 16, 16, 1030, 1030, 64, True, None, torch.bfloat16),
+    (4, 12, 12, 330, 330, 32, True, None, torch.bfloat16),
+    (3, 8, 8, 350, 333, 256, False, None, torch.bfloat16),
+    (2, 12, 6, 600, 600, 160, True, None, torch.bfloat16),
+    (4, 16, 16, 255, 259, 64, False, "add", torch.bfloat16),
+    (8, 16, 16, 300, 300, 64, False, "add", torch.float16),
+    (6, 8, 8, 400, 401, 128, False, "add", torch.bfloat16),
+    (6, 8, 4, 300, 129, 128, False, "f32", torch.bfloat16),
+    (3, 8, 8, 450, 449, 128, False, "bool", torch.bfloat16),
+    (6, 12, 12, 256, 256, 64, False, "pad", torch.bfloat16),
+    (12, 12, 12, 385, 384, 80, False, "pad", torch.float16),
+    (4, 8, 2, 200, 320, 256, False, "pad", torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_dense_calls_meet_float64(native, dev, case):
+    b, hq, hk, sq, sk, d, causal, mask, dtype = case
+    print(f"tile {case}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(sum(case[:6]))
+    randn = lambda *s: torch.randn(*s, generator=g, device=dev).to(dtype)  # noqa: E731
+    q, k, v = randn(b, hq, sq, d), randn(b, hk, sk, d), randn(b, hk, sk, d)
+    m = bias = None
+    if mask in ("add", "f32"):
+        m = randn(1, 1, sq, sk) if mask == "add" else randn(b, 1, sq, sk).float()
+        m = m.masked_fill(torch.rand(m.shape, generator=g, device=dev) < 0.3, -math.inf)
+        m[:, :, sq // 3] = -math.inf  # a row that keeps no key
+        m[:, :, : sq // 2, sk // 2 :] = -math.inf  # whole tiles masked for some rows
+        bias = m
+    elif mask == "bool":
+        m = torch.rand(b, hq, sq, sk, generator=g, device=dev) < 0.5
+        m[:, 1, 7] = False
+    elif mask == "pad":
+        lens = torch.randint(1, sk + 1, (b,), generator=g, device=dev)
+        lens[0] = sk
+        m = (torch.arange(sk, device=dev)[None] < lens[:, None]).view(b, 1, 1, sk)
+        m[1] = False  # no key at all: raw scores
+    if m is not None and m.dtype == torch.bool:
+        bias = torch.zeros(m.shape, device=dev).masked_fill(~m, -math.inf)
+    if causal:
+        bias = torch.zeros(sq, sk, device=dev).masked_fill(~torch.ones(sq, sk, dtype=torch.bool, device=dev).tril(), -math.inf)
+    native.reset_counters()
+    out, lse = torch.ops.aten._scaled_dot_product_fused_attention_overrideable(q, k, v, m, 0.0, causal)[:2]
+    torch.cuda.synchronize()
+    assert native.counters()["attention"] == 1
+    kr, vr = k.repeat_interleave(hq // hk, 1), v.repeat_interleave(hq // hk, 1)
+    for i in range(b):
+        bi = None if bias is None else (bias if bias.dim() == 2 else bias[min(i, bias.size(0) - 1)])
+        want, weight, want_lse = _attend(q[i], kr[i], vr[i], bi, 1 / math.sqrt(d))
+        _close(out[i], want, weight, dtype)
+        # The row sum is of the rounded weights: half an ulp; fp32 for the rest.
+        off = ((lse[i].double() - want_lse).abs() - 2e-6 * want_lse.abs()).max().item()
+        assert off <= HALF_ULP[dtype] + 1e-4, off
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0])
+@pytest.mark.parametrize("mask", [False, True])
+def test_scale_of_any_sign(native, dev, scale, mask):
+    print(f"scale {scale} mask {mask}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(11)
+    q, k, v = (torch.randn(8, 16, 260, 128, generator=g, device=dev).bfloat16() for _ in range(3))
+    m = torch.randn(1, 1, 260, 260, generator=g, device=dev).bfloat16() if mask else None
+    out = F.scaled_dot_product_attention(q, k, v, attn_mask=m, scale=scale)
+    for i in (0, 7):
+        want, weight, _ = _attend(q[i], k[i], v[i], None if m is None else m[0], scale)
+        _close(out[i], want, weight, torch.bfloat16)
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (128, 64), (96, 256)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_packed_ragged_batches_meet_float64(native, dev, d, dv, causal):
+    print(f"packed {d} {dv} {causal}", flush=True)
+    lens = [700, 1, 129, 64, 333, 520, 65, 31, 250, 400, 128, 610]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    g = torch.Generator(device=dev).manual_seed(d + dv)
+    randn = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()  # noqa: E731
+    q, k, v = randn(cu[-1], 24, d), randn(cu[-1], 12, d), randn(cu[-1], 12, dv)
+    out = native.sdpa_varlen(q, k, v, torch.tensor(cu, dtype=torch.int32, device=dev), max_q=max(lens), max_k=max(lens),
+                             is_causal=causal)
+    for a, b in zip(cu[:-1], cu[1:]):
+        qs, ks, vs = (t[a:b].transpose(0, 1) for t in (q, k.repeat_interleave(2, 1), v.repeat_interleave(2, 1)))
+        bias = None
+        if causal:
+            bias = torch.zeros(b - a, b - a, device=dev)
+            bias = bias.masked_fill(~torch.ones(b - a, b - a, dtype=torch.bool, device=dev).tril(), -math.inf)
+        want, weight, _ = _attend(qs, ks, vs, bias, 1 / math.sqrt(d))
+        _close(out[a:b].transpose(0, 1), want, weight, torch.bfloat16)
+
+
+def test_key_lengths_meet_float64(native, dev):
+    g = torch.Generator(device=dev).manual_seed(5)
+    q, k, v = (torch.randn(8, 16, 300, 128, generator=g, device=dev).bfloat16() for _ in range(3))
+    lens = torch.tensor([1, 31, 32, 64, 65, 200, 299, 300], dtype=torch.int32, device=dev)
+    out = native.sdpa(q, k, v, key_lengths=lens)
+    for i, n in enumerate(lens.tolist()):
+        want, weight, _ = _attend(q[i], k[i, :, :n], v[i, :, :n], None, 1 / math.sqrt(128))
+        _close(out[i], want, weight, torch.bfloat16)
