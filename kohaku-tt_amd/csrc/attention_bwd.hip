@@ -835,7 +835,9 @@ struct BwdPlan {
 //   1x14/2x2048x64 causal (64, 448): 8* 54, 10 52, 12 55
 //   4x12x512x64 causal (384, 16): 1* 22, 2 33
 // 64-key dK / dV workgroups (two wavefronts per 32 keys) at padded head dims up to 64:
-// 4x16x1024x64 83 against 93 with 128 keys, 3x32/8x1718x40 295 against 309.  64-row dQ
+// 4x16x1024x64 83 against 93 with 128 keys, 3x32/8x1718x40 295 against 309.  Past 64, where
+// they leave one workgroup per CU, only for calls that give no CU two: 2x12x251x128 causal
+// 19 against 26, 1x8x100x128 15 against 18; but 32x14/2x80x128 46 against 34.  64-row dQ
 // workgroups only where 128 rows leave CUs idle (4x16x1024x64, 512 workgroups: 95 against
 // 83; 1x14/2x2048x64, 224 workgroups: 54 against 57).
 constexpr int64_t kTileItems = 72;
@@ -852,12 +854,6 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
         grads_splits(a, pl.splits, pl.ksplit);
         return pl;
     }
-    pl.grid.half_k = dp <= 64;
-    const int64_t nk = units * ceil_div(a->seq_k, pl.grid.half_k ? 64 : 128);
-    const int64_t work = G * ceil_div(a->seq_q, 32);
-    const int64_t by_work = std::min(ceil_div(work, kTileItems), ceil_div(kTileMaxWgs, nk));
-    const int64_t by_fill = nk < kTileFewWgs ? std::min(ceil_div(2 * kTileFewWgs, nk), work / kTileMinItems) : 1;
-    pl.splits = static_cast<int>(std::max<int64_t>(1, std::min(std::max(by_work, by_fill), kBwdMaxSplits)));
     // dQ: by the query heads (a call with K / V repeated per query head splits alike, so its
     // dQ is the same bit for bit).
     const int64_t nq = a->batch * a->heads_q * ceil_div(a->seq_q, 128), tiles = ceil_div(a->seq_k, 64);
@@ -865,6 +861,13 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     const int64_t nqw = pl.grid.half_q ? a->batch * a->heads_q * ceil_div(a->seq_q, 64) : nq;
     pl.ksplit = static_cast<int>(std::max<int64_t>(
         1, std::min<int64_t>({ceil_div(kTileFewWgs, 2 * nqw), tiles / 8, kBwdMaxKsplit})));
+    const int64_t nk64 = units * ceil_div(a->seq_k, 64);
+    pl.grid.half_k = dp <= 64 || nk64 + nqw <= kTileFewWgs;
+    const int64_t nk = pl.grid.half_k ? nk64 : units * ceil_div(a->seq_k, 128);
+    const int64_t work = G * ceil_div(a->seq_q, 32);
+    const int64_t by_work = std::min(ceil_div(work, kTileItems), ceil_div(kTileMaxWgs, nk));
+    const int64_t by_fill = nk < kTileFewWgs ? std::min(ceil_div(2 * kTileFewWgs, nk), work / kTileMinItems) : 1;
+    pl.splits = static_cast<int>(std::max<int64_t>(1, std::min(std::max(by_work, by_fill), kBwdMaxSplits)));
     if (bwd_ksplit_override() > 0)
         pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
     pl.grid.tiles_q = static_cast<int>(ceil_div(a->seq_q * G, pl.grid.half_q ? 64 : 128));

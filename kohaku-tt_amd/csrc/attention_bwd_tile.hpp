@@ -64,16 +64,19 @@ __device__ __forceinline__ void store4(T* dst, const f32x4 v) {
 // Fragments read ahead of the product that takes them.
 constexpr int QA = 4, VA = 2, NFR = 4;
 
-// dK / dV tiles: 64 rows at padded head dims up to 64.  At 96 and 128 the accumulators and
-// the K fragments leave no registers for V's, so V sits in LDS beside 32-row tiles (two
-// workgroups per CU either way).
-template <typename T, int DP>
+// dK / dV workgroups take 32 KG keys: 64 (two wavefronts per 32 keys) at padded head dims
+// up to 64 and, at 96 and 128, where 128 keys (one wavefront per 32) would leave most of the
+// chip idle (HALF).  Past head dim 64 the accumulators and the K fragments leave no registers
+// for V's, so V sits in LDS beside the tiles: 32-row tiles with 128 keys (two workgroups per
+// CU), 64-row ones with 64 (one).
+template <typename T, int DP, bool HALF>
 struct DkdvShared {
-    static constexpr int TR = DP <= 64 ? 64 : 32;
+    static constexpr int KG = DP <= 64 || HALF ? 2 : 4;
+    static constexpr int TR = KG == 2 ? 64 : 32;
     static constexpr bool VL = DP > 64;
     typedef Tile<T, DP, TR> TL;
     T tile[2][2][TL::ELEMS];
-    T v[VL ? 128 * TL::PITCH : 8];
+    T v[VL ? 32 * KG * TL::PITCH : 8];
     // Base-2 lse, -D, raw flag (masked calls) of the tile's rows; a DMA instruction fills 64.
     float stats[2][3][kWave];
 };
@@ -81,13 +84,13 @@ struct DkdvShared {
 // dK / dV of 32 KG keys of one K/V head (wavefront w: key group w % KG; with KG = 2 the
 // two wavefronts of a key group take one 32-row block of each tile each and add their
 // sums at the end) over the split's (query head, query tile) items.
-template <typename T, int DP, int MK, int KG>
+template <typename T, int DP, int MK, bool HALF>
 __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem, const int tile, const int split,
                                          const int bkv) {
-    typedef DkdvShared<T, DP> SH;
+    typedef DkdvShared<T, DP, HALF> SH;
     typedef typename SH::TL TL;
     typedef typename TL::v8 v8;
-    constexpr int TR = SH::TR, DC = DP / 16, DB = DP / 32, RB = TR / 32;
+    constexpr int KG = SH::KG, TR = SH::TR, DC = DP / 16, DB = DP / 32, RB = TR / 32;
     constexpr int ES = static_cast<int>(sizeof(T));
     constexpr int RS = 4 / KG;  // wavefronts that share a key group
     constexpr bool VL = SH::VL;
@@ -147,8 +150,8 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
 #pragma unroll
         for (int c = 0; c < DC; ++c) kf[c] = frag16<v8>(kp, p.ks[2], key, g.lk, 16 * c + 8 * h2, p.d);
         if constexpr (VL) {
-            // Each wavefront stages and reads its own 32 keys (in order with its vmcnt wait).
-            typedef Tile<T, DP, 128> TV;
+            // (Published with the first item's tiles.)
+            typedef Tile<T, DP, 32 * KG> TV;
             const uint32_t vst = static_cast<uint32_t>(p.vs[2] * ES);
             const typename TV::Offs ov = TV::offs(lane, vst);
             TV::request(reinterpret_cast<const char*>(vp), vst, kt0, g.lk, p.dval * ES, ov, wave,
@@ -590,11 +593,11 @@ constexpr int bwd_waves(int dp) { return dp <= 64 ? 3 : 2; }
 // on XCD b % 8), so the interleaving is done within each XCD's blocks and a pass's work
 // item number keeps its residue: items with one (sequence, K/V head) fastest stay on few
 // XCDs, whose L2 then holds what they walk over.  Item order: heaviest tiles first.
-template <typename T, int DP, int MK>
+template <typename T, int DP, int MK, bool HALF>
 __global__ __launch_bounds__(BWD_THREADS, bwd_waves(DP)) void attn_bwd_tile_kernel(const BwdParams p, const BwdGrid gr) {
-    __shared__ __align__(1024) unsigned char sh[sizeof(DkdvShared<T, DP>) > 4 * sizeof(T) * Tile<T, DP, 64>::ELEMS
-                                                  ? sizeof(DkdvShared<T, DP>)
-                                                  : 4 * sizeof(T) * Tile<T, DP, 64>::ELEMS];
+    constexpr size_t DQ_BYTES = 4 * sizeof(T) * Tile<T, DP, 64>::ELEMS;
+    constexpr size_t KV_BYTES = sizeof(DkdvShared<T, DP, HALF>);
+    __shared__ __align__(1024) unsigned char sh[KV_BYTES > DQ_BYTES ? KV_BYTES : DQ_BYTES];
     const int x = blockIdx.x & 7, s = blockIdx.x >> 3;
     const int per_q = (gr.nq + 7) >> 3, per_k = (gr.nk + 7) >> 3, tot = per_q + per_k;
     const int q0 = static_cast<int>(static_cast<int64_t>(s) * per_q / tot);
@@ -615,13 +618,7 @@ __global__ __launch_bounds__(BWD_THREADS, bwd_waves(DP)) void attn_bwd_tile_kern
         if (i >= gr.nk) return;
         const int rest = i / units, unit = i - rest * units;
         const int t = rest / p.splits, sp = rest - t * p.splits;
-        if constexpr (DP <= 64) {
-            if (gr.half_k) {
-                bwd_dkdv<T, DP, MK, 2>(p, sh, t, sp, unit);
-                return;
-            }
-        }
-        bwd_dkdv<T, DP, MK, 4>(p, sh, t, sp, unit);
+        bwd_dkdv<T, DP, MK, HALF>(p, sh, t, sp, unit);
     }
 }
 
@@ -629,7 +626,13 @@ template <typename T, int DP, int MK>
 hipError_t launch_tile_mk(const BwdParams& p, const BwdGrid& gr, hipStream_t s) {
     const int per = (gr.nq + 7) / 8 + (gr.nk + 7) / 8;
     const dim3 grid(static_cast<unsigned>(8 * per)), block(BWD_THREADS);
-    hipLaunchKernelGGL((attn_bwd_tile_kernel<T, DP, MK>), grid, block, 0, s, p, gr);
+    if constexpr (DP > 64) {
+        if (!gr.half_k) {
+            hipLaunchKernelGGL((attn_bwd_tile_kernel<T, DP, MK, false>), grid, block, 0, s, p, gr);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((attn_bwd_tile_kernel<T, DP, MK, true>), grid, block, 0, s, p, gr);
     return hipGetLastError();
 }
 
