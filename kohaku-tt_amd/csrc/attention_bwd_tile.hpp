@@ -15,21 +15,21 @@
 // The A operands of the second products (dO^T, Q^T, K^T) are gfx950 transposed LDS reads
 // of the same tiles.  dP accumulates from -D (the row dot), so dS = P dP has no subtraction.
 //
-// What bounds it: a 32x32 block of dK / dV is 2 D / 8 MFMAs (1024 cycles of the matrix unit
+// What bounds it: a 32x32 block of dK / dV is D / 4 MFMAs (1024 cycles of the matrix unit
 // at D = 128) over about 64 VALU instructions a lane and 48 LDS reads, so with everything
-// in registers the matrix unit should lead; measured it is busy half the time, the rest
-// being waits at the tile barriers and the chain S -> P -> dV / dK within a wavefront (two
-// wavefronts a SIMD at D = 128, three at 64).  Whole backward, before (16x16x32 MFMAs, P
-// and dS through LDS, staging through registers) -> with this kernel, us:
-//   1x24x4396x128        1388 -> 922  (428 -> 644 TFLOP/s)
-//   2x10x4096x64          542 -> 387  (396 -> 556)
-//   2x8/2x3062x128 causal 320 -> 169  (300 -> 570)
-//   1x14/2x2048x64 causal  72 -> 53   (263 -> 353)
-//   8 packed x 16/8 x 128 causal, 64 to 1024 tokens 153 -> 117 (211 -> 277)
-//   2x12x2433x128, additive mask 1426 -> 598 (128 -> 304)
-// What mattered on the way (1x24x4396x128): tiles by registers' leave, without a spill in
-// the loop (1351 with fragments spilled -> 984 with V in LDS and one code path per block);
-// swizzles for 64 banks (LDS busy 39% -> 19% of the time).
+// in registers the matrix unit should lead; what is left are waits at the tile barriers and
+// the chain S -> P -> dV / dK within a wavefront (two wavefronts a SIMD at D = 128, three at
+// 64).  Whole backward, before (16x16x32 MFMAs, P and dS through LDS, staging through
+// registers) -> with this kernel, us:
+//   1x24x4396x128        1388 -> 861  (428 -> 689 TFLOP/s)
+//   2x10x4096x64          542 -> 371  (396 -> 579)
+//   2x8/2x3062x128 causal 320 -> 161  (300 -> 597)
+//   1x14/2x2048x64 causal  72 -> 51   (263 -> 373)
+//   8 packed x 16/8 x 128 causal, 64 to 1024 tokens 153 -> 92 (211 -> 354)
+//   2x12x2433x128, additive mask 1426 -> 567 (128 -> 321)
+// What mattered on the way (1x24x4396x128): no spill in the loop (1351 with fragments
+// spilled -> 984 with V in LDS and one code path per block); swizzles for 64 banks (LDS busy
+// 39% -> 19% of the time); the order of the products (925 -> 861).
 #pragma once
 
 #include <cstddef>
@@ -60,9 +60,6 @@ __device__ __forceinline__ void store4(T* dst, const f32x4 v) {
     for (int e = 0; e < 4; ++e) w[e] = from_f32<T>(v[e]);
     *reinterpret_cast<t4*>(dst) = w;
 }
-
-// Fragments read ahead of the product that takes them.
-constexpr int QA = 4, VA = 2, NFR = 4;
 
 // dK / dV workgroups take 32 KG keys: 64 (two wavefronts per 32 keys) at padded head dims
 // up to 64 and, at 96 and 128, where 128 keys (one wavefront per 32) would leave most of the
@@ -170,6 +167,7 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
     auto block = [&](uint32_t qt, const float* st, int h, int r0b) {
         // S starts from what is added to the scaled scores (over c2): 0, the mask's logit, or
         // p.hidden where the row does not see the key (its P becomes exactly 0).
+        constexpr int LA = DP <= 64 ? 1 : 3;
         f32x16 s = splat16(0.f), dp;
         if constexpr (MK != MK_NONE) {
             const int64_t msz = static_cast<int64_t>(sizeof(MRaw));
@@ -208,6 +206,41 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
                 }
             }
         }
+        // (Opaque lane addresses: the compiler would otherwise keep every sum it can hoist in
+        // registers across the loop, and V's fragments too.)
+        uint32_t ra = qt + ad.row, t0 = qt + ad.tr0, t1 = qt + ad.tr1;
+        uint32_t va = lds0 + static_cast<uint32_t>(offsetof(SH, v)) + 2u * 32 * kg * TL::PITCH + ad.row;
+        __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1), "+v"(va));
+        // The order below is kept by the fences: one MFMA, the LDS read of the operand LA
+        // products on, and a share of the VALU work per group.  (Left alone, the compiler reads
+        // each operand where it is used and bunches the exponentials: 8 packed x 16/8 x 128 121
+        // us against 92, 1x24x4396x128 925 against 861.  LA as far as the registers go: 2 at
+        // head dim 64 spills, 89 us against 78 on 4x16x1024x64.)
+        v8 fa[LA], fb[VL ? LA : 1];
+        auto col = [&](int j, uint32_t imm) { return TL::cols(t0, t1, j / DB, j % DB, imm); };
+#pragma unroll
+        for (int c = 0; c < LA; ++c) fa[c] = TL::rows(ra, c, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            s = Mfma32<T>::run(fa[c % LA], kf[c], s);
+            if (c + LA < DC) {
+                fa[c % LA] = TL::rows(ra, c + LA, 0);
+            } else {
+                fa[c % LA] = TL::rows(ra, (c + LA) - DC, TILE_B);
+                if constexpr (VL) fb[(c + LA) - DC] = TL::rows(va, (c + LA) - DC, 0);
+            }
+            if (c >= DC - 4 || DC < 4) {
+                const int q = DC < 4 ? c : c - (DC - 4);
+#pragma unroll
+                for (int qq = q * (DC < 4 ? 4 / DC : 1); qq < (q + 1) * (DC < 4 ? 4 / DC : 1); ++qq) {
+                    const f32x4 nd = *reinterpret_cast<const f32x4*>(st + kWave + 8 * qq + 4 * h2);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dp[4 * qq + e] = nd[e];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // Blocks whose rows all see all 32 keys (uniform) need no per-element test.
         if (!(kw0 + 31 < g.lk && (!p.causal || kw0 + 31 <= r0b + g.coff))) {
             // Rows whose index (from this lane's first) is below `seen` do not see the key.
@@ -216,87 +249,60 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
             for (int i = 0; i < 16; ++i)
                 if (8 * (i / 4) + i % 4 < seen) s[i] = p.hidden;
         }
-        // (Opaque lane addresses: the compiler would otherwise keep every sum it can hoist in
-        // registers across the loop, and V's fragments too.)
-        uint32_t ra = qt + ad.row, t0 = qt + ad.tr0, t1 = qt + ad.tr1;
-        uint32_t va = lds0 + static_cast<uint32_t>(offsetof(SH, v)) + 2u * 32 * kg * TL::PITCH + ad.row;
-        __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1), "+v"(va));
-#pragma unroll
-        for (int c = 0; c < DC; ++c) s = Mfma32<T>::run(TL::rows(ra, c, 0), kf[c], s);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 nd = *reinterpret_cast<const f32x4*>(st + kWave + 8 * q + 4 * h2);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) dp[4 * q + e] = nd[e];
-        }
+        __builtin_amdgcn_sched_barrier(0);
+        // dP, with P formed from S meanwhile.
+        v8 pb[2], sb[2];
+        f32x4 l2[2];
+        auto lse4 = [&](int q) { return *reinterpret_cast<const f32x4*>(st + 8 * q + 4 * h2); };
+        l2[0] = lse4(0);
+        l2[1] = lse4(1);
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
+            // (Ring slots: dO's fragment c was read into slot (DC - LA + c) % LA.)
+            const int slot = (DC - LA + c) % LA;
             if constexpr (VL)
-                dp = Mfma32<T>::run(TL::rows(ra, c, TILE_B), TL::rows(va, c, 0), dp);
+                dp = Mfma32<T>::run(fa[slot], fb[c % LA], dp);
             else
-                dp = Mfma32<T>::run(TL::rows(ra, c, TILE_B), vf[c], dp);
+                dp = Mfma32<T>::run(fa[slot], vf[c], dp);
+            if (c + LA < DC) {
+                fa[slot] = TL::rows(ra, c + LA, TILE_B);
+                if constexpr (VL) fb[c % LA] = TL::rows(va, c + LA, 0);
+            } else {
+                fa[slot] = col((c + LA) - DC, TILE_B);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k * DC / 8 == c) {
+#pragma unroll
+                    for (int i = 2 * k; i < 2 * k + 2; ++i) {
+                        s[i] = __builtin_amdgcn_exp2f(s[i] * p.c2 - l2[(k / 2) % 2][i % 4]);
+                        pb[i / 8][i % 8] = from_f32<T>(s[i]);
+                    }
+                    if (k % 2 == 1 && k / 2 + 2 < 4) l2[(k / 2) % 2] = lse4(k / 2 + 2);
+                }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        v8 pb[2], sb[2];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 l2 = *reinterpret_cast<const f32x4*>(st + 8 * q + 4 * h2);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = 4 * q + e;
-                s[i] = __builtin_amdgcn_exp2f(s[i] * p.c2 - l2[e]);
-                pb[i / 8][i % 8] = from_f32<T>(s[i]);
-            }
-        }
-        if constexpr (VL) {
-            __builtin_amdgcn_sched_group_barrier(SG_DSREAD, QA, 0);
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-                if (c < DC - QA)
-                    __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 1, 0);
-                else
-                    __builtin_amdgcn_sched_group_barrier(SG_DSREAD, (4 + 2 * VA) / QA, 0);
-            }
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-                if (c < DC - VA) __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(SG_VALU, 40 / DC, 0);
-            }
-        } else {
-            __builtin_amdgcn_sched_group_barrier(SG_DSREAD, DC + 4, 0);
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 1, 0);
-            }
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(SG_VALU, 40 / DC, 0);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
         // dV^T += dO^T P while dS = P (dP - D) is formed, then dK^T += Q^T dS.
+        constexpr int NP = 2 * DB;
 #pragma unroll
-        for (int b = 0; b < DB; ++b)
+        for (int j = 0; j < 2 * NP; ++j) {
+            const int slot = (2 * DC - LA + j) % LA;
+            if (j < NP)
+                dv[j % DB] = Mfma32<T>::run(fa[slot], pb[j / DB], dv[j % DB]);
+            else
+                dk[j % DB] = Mfma32<T>::run(fa[slot], sb[(j - NP) / DB], dk[j % DB]);
+            if (j + LA < NP)
+                fa[slot] = col(j + LA, TILE_B);
+            else if (j + LA < 2 * NP)
+                fa[slot] = col(j + LA - NP, 0);
 #pragma unroll
-            for (int kc = 0; kc < 2; ++kc) dv[b] = Mfma32<T>::run(TL::cols(t0, t1, kc, b, TILE_B), pb[kc], dv[b]);
+            for (int k = 0; k < 8; ++k)
+                if (j < NP && k * NP / 8 == j) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sb[i / 8][i % 8] = from_f32<T>(s[i] * dp[i]);
-#pragma unroll
-        for (int b = 0; b < DB; ++b)
-#pragma unroll
-            for (int kc = 0; kc < 2; ++kc) dk[b] = Mfma32<T>::run(TL::cols(t0, t1, kc, b, 0), sb[kc], dk[b]);
-        // The transposed reads run four fragments ahead of the products.
-        __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2 * NFR, 1);
-#pragma unroll
-        for (int i = 0; i < 4 * DB; ++i) {
-            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 1);
-            if (i < 4 * DB - NFR) __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2, 1);
-            if (i < 2 * DB) __builtin_amdgcn_sched_group_barrier(SG_VALU, 24 / (2 * DB), 1);
+                    for (int i = 2 * k; i < 2 * k + 2; ++i) sb[i / 8][i % 8] = from_f32<T>(s[i] * dp[i]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
     };
     if (split < items) request(gi, bi, 0);
     int buf = 0;
@@ -484,47 +490,53 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[i] = raw ? 0.f : (s[i] > kMaskedLogit ? s[i] * p.mask_c : p.hidden);
         }
+        uint32_t ra = kt + ad.row, t0 = kt + ad.tr0, t1 = kt + ad.tr1;
+        __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1));  // (as in bwd_dkdv)
+        // S, dP with the exponentials, dQ: the operands in one stream, LA ahead.
+        constexpr int LA = DP <= 64 ? 2 : 3, NP = 2 * DB, TOT = 2 * DC + NP;
+        v8 fa[LA], sb[2];
+        auto operand = [&](int i) {
+            if (i < 2 * DC) return TL::rows(ra, i % DC, i < DC ? 0u : TILE_B);
+            return TL::cols(t0, t1, (i - 2 * DC) / DB, (i - 2 * DC) % DB, 0);
+        };
+#pragma unroll
+        for (int i = 0; i < LA; ++i) fa[i] = operand(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < DC; ++i) {
+            s = Mfma32<T>::run(fa[i % LA], qf[i], s);
+            fa[i % LA] = operand(i + LA);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (kb0 + 31 >= lim_w) {
             const int rel = lim - kb0 - 4 * h2;  // keys whose index is below rel are visible
 #pragma unroll
             for (int i = 0; i < 16; ++i)
                 if (8 * (i / 4) + i % 4 >= rel) s[i] = p.hidden;
         }
-        uint32_t ra = kt + ad.row, t0 = kt + ad.tr0, t1 = kt + ad.tr1;
-        __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1));  // (as in bwd_dkdv)
-#pragma unroll
-        for (int c = 0; c < DC; ++c) s = Mfma32<T>::run(TL::rows(ra, c, 0), qf[c], s);
-#pragma unroll
-        for (int c = 0; c < DC; ++c) dp = Mfma32<T>::run(TL::rows(ra, c, TILE_B), of[c], dp);
-        v8 sb[2];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(s[i] * p.c2 - l2);
-        __builtin_amdgcn_sched_group_barrier(SG_DSREAD, DC, 0);
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 1, 0);
-        }
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(SG_VALU, 32 / DC, 0);
-        }
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < DC; ++i) {
+            dp = Mfma32<T>::run(fa[(DC + i) % LA], of[i], dp);
+            fa[(DC + i) % LA] = operand(DC + i + LA);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k * DC / 8 == i) {
+                    s[2 * k] = __builtin_amdgcn_exp2f(s[2 * k] * p.c2 - l2);
+                    s[2 * k + 1] = __builtin_amdgcn_exp2f(s[2 * k + 1] * p.c2 - l2);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int i = 0; i < 16; ++i) sb[i / 8][i % 8] = from_f32<T>(s[i] * dp[i]);
-#pragma unroll
-        for (int b = 0; b < DB; ++b)
-#pragma unroll
-            for (int kc = 0; kc < 2; ++kc) dq[b] = Mfma32<T>::run(TL::cols(t0, t1, kc, b, 0), sb[kc], dq[b]);
-        __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2 * DB < 4 ? 4 * DB : 8, 1);
-        __builtin_amdgcn_sched_group_barrier(SG_VALU, 24, 1);
-#pragma unroll
-        for (int i = 0; i < 2 * DB; ++i) {
-            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 1);
-            if (i < 2 * DB - 4) __builtin_amdgcn_sched_group_barrier(SG_DSREAD, 2, 1);
-        }
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const int i = 2 * DC + j;
+            dq[j % DB] = Mfma32<T>::run(fa[i % LA], sb[j / DB], dq[j % DB]);
+            if (i + LA < TOT) fa[i % LA] = operand(i + LA);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     const int kstep = p.ksplit * TR;
     int k0 = ksp * TR;
@@ -535,12 +547,8 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
         __syncthreads();
         if (k0 + kstep < kend) request(k0 + kstep, buf ^ 1);
 #pragma unroll 1
-        for (int kb = KS == 1 ? 0 : kspw; kb < 2; kb += KS) {
-            const int kb0 = k0 + 32 * kb;
-            if (kb0 >= kend_w) continue;
-            const uint32_t kt = lds0 + buf * 2 * TILE_B + 2u * 32 * kb * TL::PITCH;
-            block(kt, kb0);
-        }
+        for (int kb = KS == 1 ? 0 : kspw; kb < 2; kb += KS)
+            if (k0 + 32 * kb < kend_w) block(lds0 + buf * 2 * TILE_B + 2u * 32 * kb * TL::PITCH, k0 + 32 * kb);
         buf ^= 1;
     }
     if constexpr (KS == 2) {

@@ -162,7 +162,4 @@ __device__ __forceinline__ f32x16 splat16(T x) {
     return v;
 }
 
-// Scheduling groups (LLVM's sched_group_barrier masks).
-constexpr int SG_VALU = 0x2, SG_MFMA = 0x8, SG_DSREAD = 0x100;
-
 }  // namespace kmi
