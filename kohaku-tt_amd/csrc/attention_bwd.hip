@@ -658,15 +658,10 @@ __device__ __forceinline__ void attn_bwd_dq(const BwdParams& p, const int bid) {
 // neither reads the other's output), their workgroups interleaved in proportion (block b
 // is dQ workgroup floor(b n_dq / n) when that count steps at b, else a dK / dV workgroup),
 // so that the two kinds share every CU from the start.
-// Workgroups per CU the fused kernel keeps resident (the register budget it compiles to,
-// without spills): those of the dK / dV kernel alone at head dims 64 and 128 for the
-// unmasked equal-dim variants, one fewer for masked or value-dim ones.
-constexpr int bwd_min_blocks(int dp, bool plain) {
-    return dp <= 64 ? (plain ? 4 : 3) : (dp <= 128 ? (plain ? 3 : 2) : 1);
-}
-
+// At these head dims the accumulators alone take a wavefront per SIMD's registers: one
+// workgroup per CU.
 template <typename T, int DP, int MK, bool DV>
-__global__ __launch_bounds__(BWD_THREADS, bwd_min_blocks(DP, MK == MK_NONE && !DV)) void attn_bwd_grads(
+__global__ __launch_bounds__(BWD_THREADS, 1) void attn_bwd_grads(
     const BwdParams p, const int kv_blocks, const int dq_blocks) {
     const int64_t b = blockIdx.x, n = static_cast<int64_t>(kv_blocks) + dq_blocks;
     const int q0 = static_cast<int>(b * dq_blocks / n), q1 = static_cast<int>((b + 1) * dq_blocks / n);
