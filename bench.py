@@ -165,7 +165,7 @@ def build_rows():
     # Backward FLOPs: S, dP, dV, dK, dQ = 2.5x the forward's two products.
     rows["c1_attn_bwd"] = Row(
         "c1_attn_bwd", "extra: C1 attention backward (flash dQ/dK/dV from the forward's lse)", "mfma",
-        2.5 * C.attn_flops(64, 14, C.causal_pairs(1, 2048)), None, (bwd_make, bwd_cpu), "attn_bwd_dkdv",
+        2.5 * C.attn_flops(64, 14, C.causal_pairs(1, 2048)), None, (bwd_make, bwd_cpu), "attn_bwd_tile_kernel",
         "attention_backward")
     norm_row("c1_rms", "C1 rms_norm [1,2048,896]", c1["x"], c1["w"], None, 1e-6, "rms")
 
@@ -267,7 +267,7 @@ def build_rows():
 
         extra = 4 * sum(n * n for n in L) if masked else 0
         rows[name] = Row(name, label, "mfma", C.attn_flops(128, 16, pairs), v4_bytes + extra, (make, cpu),
-                         "attn_fwd_kernel", "attention")
+                         "attn_tile_kernel", "attention")
 
     varlen_row("c4_varlen", f"C4 varlen causal GQA 8 seqs T={t} 16/8x128", False)
     varlen_row("c4_varlen_masked", "C4 varlen causal + packed additive mask", True)
@@ -297,7 +297,7 @@ def build_rows():
 
     rows["c4_varlen_bwd"] = Row(
         "c4_varlen_bwd", "extra: C4 varlen causal backward (one launch set over the packed batch)", "mfma",
-        2.5 * C.attn_flops(128, 16, pairs), None, (varlen_bwd_make, varlen_bwd_cpu), "attn_bwd_dkdv",
+        2.5 * C.attn_flops(128, 16, pairs), None, (varlen_bwd_make, varlen_bwd_cpu), "attn_bwd_tile_kernel",
         "attention_backward")
 
     c5 = C.config5()
