@@ -1,7 +1,8 @@
 // Attention forward, host side: argument checks, the launch plan and the C ABI entry
 // points (kmi_attn_workspace_bytes, kmi_attn_fwd).  The kernels are in
-// attention_kernels.hpp, instantiated per padded head dim in attention_d<D>.hip; what they
-// compute and how is described there.
+// attention_kernels.hpp (decode, short and small calls), attention_tile.hpp (prefill that
+// fills the chip) and attention_pipe.hip (the other causal head-dim-64 prefill), the first
+// two instantiated per padded head dim; what they compute and how is described there.
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>

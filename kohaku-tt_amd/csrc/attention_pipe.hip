@@ -1,5 +1,5 @@
-// Attention forward for head dim 64, unmasked dense causal calls (top-left): the prefill
-// shape of BASELINE config 1 (causal GQA 1x14/2x2048x64), the headline row.
+// Attention forward for head dim 64, unmasked dense causal calls (top-left), as in a
+// 1x14/2x2048x64 GQA prefill, up to the size where attn_tile_kernel takes them.
 //
 // What it computes is what attn_fwd_kernel computes for these calls (attention_kernels.hpp:
 // logits scale * q.k in base 2, online softmax with a lazy rescale, P rounded to the
