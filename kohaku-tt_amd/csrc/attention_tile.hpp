@@ -361,7 +361,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
         auto next = [&](int t, bool all) {
             if (skip && !all)
                 while (t < nt && __builtin_amdgcn_readfirstlane(flag[t]) == 0) ++t;
-            return t;
+            return __builtin_amdgcn_readfirstlane(t);  // (scalar, as the staging's addresses are)
         };
         // Two passes at most: over the kept keys, and (when a row of the workgroup kept none)
         // over the raw scores of the rows that kept none.

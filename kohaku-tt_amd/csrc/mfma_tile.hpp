@@ -47,8 +47,13 @@ __device__ __forceinline__ u32x2 lds_tr(uint32_t at) {
 // every transposed LDS read for a use of every load of this kind in flight and waits for
 // all of them first, which would end each prefetch at the next read (C1 backward's dK / dV
 // loop had one such wait per 32 rows).  The loops below wait for a tile themselves (all of
-// vmcnt) before the barrier that publishes it.  The nop is the wait state between a write
-// of m0 and its use.
+// vmcnt) before the barrier that publishes it.
+//
+// The compiler does not see the load inside the asm, so the asm holds the wait states itself:
+// one between a write of m0 and its use, and five between a VALU write of the resource's
+// registers (readfirstlane, or a reload of spilled ones, which the compiler may put right
+// before the asm) and the load that reads them: the move and a nop of four.  Every load holds
+// them, since nothing ties the resource to its registers from one load to the next.
 __device__ __forceinline__ u32x4 dma_rsrc(const void* base, uint32_t bytes) {
     // (Uniform; readfirstlane keeps it in scalar registers where the compiler cannot tell.)
     const uint64_t a = reinterpret_cast<uint64_t>(base);
@@ -61,16 +66,16 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
         reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)(static_cast<const char*>(p))));
 }
 __device__ __forceinline__ void dma16(u32x4 rs, uint32_t off, uint32_t dst) {
-    __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+    __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                      :
                      : "v"(off), "s"(rs), "s"(dst)
-                     : "memory");
+                     : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(u32x4 rs, uint32_t off, uint32_t dst) {
-    __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds"
+    __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dword %0, %1, 0 offen lds"
                      :
                      : "v"(off), "s"(rs), "s"(dst)
-                     : "memory");
+                     : "memory", "m0");
 }
 
 // A [TR][DP] tile in LDS: rows of NCH 16-byte chunks (a power of two; at DP = 96 and 192 the
