@@ -11,9 +11,10 @@
 //
 // Unmasked calls are software-pipelined: while tile t's exponentials and PV products run,
 // tile t + 1's S products run with them (its K is staged a tile earlier than its V).
-// Masked calls start the score accumulators from the mask's logits (over the scale, which
-// the exponent multiplies back) or minus infinity, skip tiles in which a wavefront keeps no
-// key, and run a second pass over the raw scores only for rows that kept none.
+// Masked calls hold a tile's mask logits beside its products, add them in one FMA once the
+// products are whole and select minus infinity for masked keys (whatever their K row holds),
+// skip tiles in which a wavefront keeps no key, and run a second pass over the raw scores only
+// for rows that kept none.
 #pragma once
 
 #include "attention_params.hpp"
@@ -23,7 +24,7 @@ namespace kmi {
 namespace fwd {
 
 constexpr float kTileLazy = 8.f;  // log2 units a row max may grow before O is rescaled
-constexpr float kTileLog2e = 1.4426950408889634f, kTileLn2 = 0.6931471805599453f;
+constexpr float kTileLn2 = 0.6931471805599453f;
 
 // Row groups of a workgroup: 4 (128 rows, one wavefront per 32), or 2 (64 rows, two
 // wavefronts per 32 that take one half of each key tile and merge their states at the end).
@@ -144,6 +145,8 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
     float m = -INFINITY, thr = -INFINITY, neg_m = 0.f, lsum = 0.f;
 
     const int kw = 32 * NB * kp;  // the wavefront's first key within a tile
+    // Scores in units of 1 / xs (base 2): the products, or (masked calls) scaled already.
+    const float xs = MASKED ? 1.f : c2;
     // Minus infinity where the row does not see the key.
     auto edge = [&](f32x16 (&s)[NB], int t) {
         if (t * KT + kw + 32 * NB <= lim_w) return;
@@ -165,8 +168,8 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
     // Moves the reference points that the tile's scores exceed by more than 2^kTileLazy.
     auto rescale = [&](const f32x16 (&s)[NB]) {
         const float lmax = block_max(s);
-        if (__builtin_amdgcn_ballot_w64(lmax * c2 > thr)) {
-            const float mt = fmaxf(lmax, other_half(lmax)) * c2;
+        if (__builtin_amdgcn_ballot_w64(lmax * xs > thr)) {
+            const float mt = fmaxf(lmax, other_half(lmax)) * xs;
             const bool move = mt > thr;
             const float alpha = move ? __builtin_amdgcn_exp2f(m - mt) : 1.f;  // 0 while m was -inf
             if (move) {
@@ -194,8 +197,8 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
     };
     auto pair = [&](const f32x16 (&s)[NB], v8 (&pb)[NB][2], int k) {
         const int n = k / 8, i = 2 * (k % 8);
-        pb[n][i / 8][i % 8] = from_f32<T>(__builtin_amdgcn_exp2f(s[n][i] * c2 + neg_m));
-        pb[n][i / 8][i % 8 + 1] = from_f32<T>(__builtin_amdgcn_exp2f(s[n][i + 1] * c2 + neg_m));
+        pb[n][i / 8][i % 8] = from_f32<T>(__builtin_amdgcn_exp2f(s[n][i] * xs + neg_m));
+        pb[n][i / 8][i % 8 + 1] = from_f32<T>(__builtin_amdgcn_exp2f(s[n][i + 1] * xs + neg_m));
         lsum = dot_ones<T>(__builtin_bit_cast(u32x4, pb[n][i / 8])[(i % 8) / 2], lsum);
     };
     // PV of a tile from its probabilities (the pairs past `done` groups are formed here).
@@ -316,7 +319,6 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
                    head * p.ms[1] + static_cast<int64_t>(pos) * p.ms[2];
         }
         const MRaw* const mp = static_cast<const MRaw*>(p.mask);
-        const float mask_c = kTileLog2e / c2;
         // A padding mask (the keys alone decide): tiles that keep no key are not staged, once
         // some key is kept.  The flags are one byte per tile.
         constexpr int FLAGS = 2048, EPV = 16 / static_cast<int>(sizeof(MRaw));
@@ -376,30 +378,33 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             while (t < nt) {
                 const int tn = next(t + 1, pass == 1);
                 landed();
-                f32x16 s[NB];
+                f32x16 s[NB], ml[NB];  // ml: the logits, kMaskedLogit or less where masked or not seen
                 if (pass == 0) {
 #pragma unroll
                     for (int n = 0; n < NB; ++n)
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            const float ml = mask_logit_of<MK>(raw[n][i]);
-                            s[n][i] = ml > kMaskedLogit ? ml * mask_c : -INFINITY;
-                        }
+                        for (int i = 0; i < 16; ++i) ml[n][i] = mask_value_of<MK>(raw[n][i]);
                 } else {
 #pragma unroll
-                    for (int n = 0; n < NB; ++n) s[n] = splat16(dead ? 0.f : -INFINITY);
+                    for (int n = 0; n < NB; ++n) ml[n] = splat16(dead ? 0.f : kMaskedLogit);
                 }
                 if (tn < nt) {
                     request_k(tn, buf ^ 1);
                     request_v(tn, buf ^ 1);
                     if (pass == 0) load_mask(raw, tn);
                 }
-                edge(s, t);
+                edge(ml, t);
                 // (Uniform.)  A tile in which no row of the wavefront keeps a key adds nothing.
-                if (__builtin_amdgcn_ballot_w64(block_max(s) > -INFINITY)) {
+                if (__builtin_amdgcn_ballot_w64(block_max(ml) > kMaskedLogit)) {
                     uint32_t ra = k_addr(buf) + ad.row, t0 = v_addr(buf) + ad.tr0, t1 = v_addr(buf) + ad.tr1;
                     __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1));
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) s[n] = splat16(0.f);
                     scores(s, ra);
+#pragma unroll
+                    for (int n = 0; n < NB; ++n)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) s[n][i] = masked_score(s[n][i], c2, ml[n][i]);
                     finish(s, t0, t1);
                 }
                 t = tn;

@@ -159,6 +159,32 @@ struct Tile {
     }
 };
 
+// A loaded mask element as a logit: a kept key's value, anything at or below kMaskedLogit for a
+// masked key (mask_logit_of without its clamp, which only the raw-score rows of the 16x16
+// kernels need).
+template <int MK, typename R>
+__device__ __forceinline__ float mask_value_of(R raw) {
+    if constexpr (MK == MK_BF16) {
+        const uint32_t mag = __builtin_bit_cast(uint16_t, raw) & 0x7fffu;
+        return mag > 0x7f80u ? kMaskedLogit : static_cast<float>(__builtin_bit_cast(bf16, raw));
+    } else if constexpr (MK == MK_F16) {
+        const uint32_t mag = __builtin_bit_cast(uint16_t, raw) & 0x7fffu;
+        return mag > 0x7c00u ? kMaskedLogit : static_cast<float>(__builtin_bit_cast(f16, raw));
+    } else if constexpr (MK == MK_F32) {
+        const uint32_t mag = __builtin_bit_cast(uint32_t, raw) & 0x7fffffffu;
+        return mag > 0x7f800000u ? kMaskedLogit : raw;
+    } else {
+        return mask_logit_of<MK>(raw);
+    }
+}
+
+// A masked call's scaled score (base 2) from the whole product s: a kept key's logit joins in
+// one rounding; a masked key's is minus infinity whatever its product holds (a select, since
+// the product may be NaN or infinite).
+__device__ __forceinline__ float masked_score(float s, float c2, float logit) {
+    return logit > kMaskedLogit ? logit * 1.4426950408889634f + s * c2 : -INFINITY;
+}
+
 template <typename T>
 __device__ __forceinline__ f32x16 splat16(T x) {
     f32x16 v;

@@ -147,3 +147,64 @@ def test_key_lengths_meet_float64(native, dev):
     for i, n in enumerate(lens.tolist()):
         want, weight, _ = _attend(q[i], k[i, :, :n], v[i, :, :n], None, 1 / math.sqrt(128))
         _close(out[i], want, weight, torch.bfloat16)
+
+
+@pytest.mark.parametrize("case", [
+    # b, h, s, d, kind, dtype: the tile kernel (64 and 128 rows) and the smaller calls' kernel
+    (2, 16, 400, 64, "add", torch.bfloat16),
+    (8, 16, 400, 64, "add", torch.float16),
+    (6, 8, 401, 128, "bool", torch.bfloat16),
+    (8, 16, 300, 128, "pad", torch.bfloat16),
+    (4, 8, 200, 256, "pad", torch.bfloat16),
+    (1, 2, 100, 64, "add", torch.bfloat16),
+    (1, 2, 100, 128, "pad", torch.bfloat16),
+], ids=lambda c: "x".join(map(str, c)))  # fmt: skip
+def test_masked_keys_may_hold_anything(native, dev, case):
+    """A masked key has weight 0 whatever its K row holds: NaN, infinities, or values whose
+    product overflows.  The result is that of the same call with zeros there, bit for bit."""
+    b, h, s, d, kind, dtype = case
+    print(f"masked rows {case}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(s + d)
+    q, k, v = (torch.randn(b, h, s, d, generator=g, device=dev).to(dtype) for _ in range(3))
+    hidden = torch.rand(s, generator=g, device=dev) < 0.4
+    hidden[::32] = False  # each tile keeps a key
+    if kind == "pad":
+        m = (~hidden).view(1, 1, 1, s).expand(b, 1, 1, s)
+    else:
+        m = (torch.rand(1, 1, s, s, generator=g, device=dev) >= 0.2) & ~hidden
+        m[..., 0] = True
+        m[..., ::32] = True
+        if kind == "add":
+            m = torch.randn(1, 1, s, s, generator=g, device=dev).to(dtype).masked_fill(~m, -math.inf)
+    clean = k.masked_fill(hidden[None, None, :, None], 0.0)
+    spoilt = clean.clone()
+    at = torch.nonzero(hidden).flatten()
+    for i, value in enumerate((math.nan, math.inf, -math.inf, torch.finfo(dtype).max)):
+        spoilt[:, :, at[i::4]] = value
+    attend = torch.ops.aten._scaled_dot_product_fused_attention_overrideable
+    out, lse = attend(q, spoilt, v, m, 0.0, False)[:2]
+    want, want_lse = attend(q, clean, v, m, 0.0, False)[:2]
+    assert torch.isfinite(want).all()
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_additive_mask_rounds_once(native, dev, d):
+    """A logit of -1e5 over whole rows (kept: above -5e5) leaves the weights as they are but
+    for the rounding of score + logit.  In base 2 that sum lies within 2^17 .. 2^18, so one
+    rounding is off by 2^-6 / sqrt(12) in the mean, and a weight by ln 2 of it; f16 rounds the
+    weights and the result by 2^-11 / sqrt(3) each."""
+    b, h, s = 4, 8, 384
+    g = torch.Generator(device=dev).manual_seed(d)
+    q, k, v = (torch.randn(b, h, s, d, generator=g, device=dev).half() for _ in range(3))
+    m = torch.full((1, 1, s, s), -1e5, device=dev)
+    out = F.scaled_dot_product_attention(q, k, v, attn_mask=m)
+    want = off = 0.0
+    for i in range(b):
+        ref, _, _ = _attend(q[i], k[i], v[i], None, 1 / math.sqrt(d))
+        off += (out[i].double() - ref).square().sum().item()
+        want += ref.square().sum().item()
+    got = math.sqrt(off / want)
+    once = math.hypot(2.0**-6 / math.sqrt(12) * math.log(2), 2.0**-11 / math.sqrt(3) * math.sqrt(2))
+    print(f"d {d}: {got:.2e}, one rounding {once:.2e}", flush=True)
+    assert got <= 1.15 * once  # (one rounding: 15% for what is left of a small sample)
