@@ -1039,7 +1039,6 @@ extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t 
     p.c2 = static_cast<float>(a->scale * 1.4426950408889634);
     // A zero scale becomes one that finite scores vanish under (minus infinity does not).
     if (pl.tile && std::fabs(p.c2) < 1e-30f) p.c2 = p.c2 < 0.f ? -1e-30f : 1e-30f;
-    p.mask_c = static_cast<float>(1.4426950408889634 / static_cast<double>(p.c2));
     p.hidden = p.c2 > 0.f ? -INFINITY : INFINITY;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const hipError_t err = a->dtype == KMI_BF16 ? launch_bwd_dim<bf16>(p, pl, mk, s) : launch_bwd_dim<f16>(p, pl, mk, s);

@@ -37,10 +37,9 @@ struct BwdParams {
     int d, dval;  // q / k and v / out head dims (DP: the larger, padded)
     int64_t rows_total, keys_total;
     float scale, c2;  // c2 = scale * log2(e) (attn_bwd_tile_kernel: never 0)
-    // attn_bwd_tile_kernel: what a score accumulator starts from, in units of 1 / c2: a mask
-    // logit times mask_c = log2(e) / c2, or hidden (minus infinity with c2's sign) for a key
-    // the row does not see.
-    float mask_c, hidden;
+    // attn_bwd_tile_kernel, unmasked: the score of a key the row does not see (minus infinity
+    // with c2's sign).
+    float hidden;
 };
 
 // One sequence's geometry: query rows [q0, q0 + lq) and keys [k0, k0 + lk) of the packed

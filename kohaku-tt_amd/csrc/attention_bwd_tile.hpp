@@ -162,14 +162,17 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
 #pragma unroll
     for (int b = 0; b < DB; ++b) dk[b] = dv[b] = splat16(0.f);
     typedef typename MaskRaw<MK>::type MRaw;
+    // S in units of 1 / xs (base 2): the products, or (masked calls) scaled already; `hidden`
+    // makes P exactly 0 where the row does not see the key.
+    constexpr bool MASKED = MK != MK_NONE;
+    const float xs = MASKED ? 1.f : p.c2, hidden = MASKED ? -INFINITY : p.hidden;
 
     // One 32-row block (rows r0b ..) at LDS address qt (dO's a tile on).
     auto block = [&](uint32_t qt, const float* st, int h, int r0b) {
-        // S starts from what is added to the scaled scores (over c2): 0, the mask's logit, or
-        // p.hidden where the row does not see the key (its P becomes exactly 0).
+        // ml: the mask's logits, added once S is whole (masked_score).
         constexpr int LA = DP <= 64 ? 1 : 3;
-        f32x16 s = splat16(0.f), dp;
-        if constexpr (MK != MK_NONE) {
+        f32x16 s = splat16(0.f), ml, dp;
+        if constexpr (MASKED) {
             const int64_t msz = static_cast<int64_t>(sizeof(MRaw));
             const int64_t b0 = g.mbase + h * p.ms[1] + r0b * g.mrow;
             const bool fast = g.mrow >= 0 && g.mkey >= 0 && kw0 + 31 < g.lk && r0b + 31 < g.lq &&
@@ -190,19 +193,20 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
                         raw[i] = __builtin_bit_cast(MRaw, __builtin_amdgcn_raw_buffer_load_b32(rs, off, so, 0));
                 }
 #pragma unroll
-                for (int i = 0; i < 16; ++i) s[i] = mask_logit_of<MK>(raw[i]);
+                for (int i = 0; i < 16; ++i) ml[i] = mask_value_of<MK>(raw[i]);
             } else {
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
-                    s[i] = mask_at<MK>(p, g, h, min(r0b + 8 * (i / 4) + 4 * h2 + i % 4, g.lq - 1), min(key, g.lk - 1));
+                    ml[i] = mask_at<MK>(p, g, h, min(r0b + 8 * (i / 4) + 4 * h2 + i % 4, g.lq - 1), min(key, g.lk - 1));
             }
+            // (Uniform; rows that kept no key are rare.)
+            if (__builtin_amdgcn_ballot_w64(st[2 * kWave + l32] != 0.f)) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const f32x4 rw = *reinterpret_cast<const f32x4*>(st + 2 * kWave + 8 * q + 4 * h2);
+                for (int q = 0; q < 4; ++q) {
+                    const f32x4 rw = *reinterpret_cast<const f32x4*>(st + 2 * kWave + 8 * q + 4 * h2);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float m = s[4 * q + e];
-                    s[4 * q + e] = rw[e] != 0.f ? 0.f : (m > kMaskedLogit ? m * p.mask_c : p.hidden);
+                    for (int e = 0; e < 4; ++e)
+                        if (rw[e] != 0.f) ml[4 * q + e] = 0.f;
                 }
             }
         }
@@ -217,6 +221,11 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
         // us against 92, 1x24x4396x128 925 against 861.  LA as far as the registers go: 2 at
         // head dim 64 spills, 89 us against 78 on 4x16x1024x64.)
         v8 fa[LA], fb[VL ? LA : 1];
+        auto neg_dots = [&](int q) {
+            const f32x4 nd = *reinterpret_cast<const f32x4*>(st + kWave + 8 * q + 4 * h2);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dp[4 * q + e] = nd[e];
+        };
         auto col = [&](int j, uint32_t imm) { return TL::cols(t0, t1, j / DB, j % DB, imm); };
 #pragma unroll
         for (int c = 0; c < LA; ++c) fa[c] = TL::rows(ra, c, 0);
@@ -230,16 +239,19 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
                 fa[c % LA] = TL::rows(ra, (c + LA) - DC, TILE_B);
                 if constexpr (VL) fb[(c + LA) - DC] = TL::rows(va, (c + LA) - DC, 0);
             }
-            if (c >= DC - 4 || DC < 4) {
+            // (Masked: dP's start follows below, in the registers that ml leaves.)
+            if (!MASKED && (c >= DC - 4 || DC < 4)) {
                 const int q = DC < 4 ? c : c - (DC - 4);
 #pragma unroll
-                for (int qq = q * (DC < 4 ? 4 / DC : 1); qq < (q + 1) * (DC < 4 ? 4 / DC : 1); ++qq) {
-                    const f32x4 nd = *reinterpret_cast<const f32x4*>(st + kWave + 8 * qq + 4 * h2);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) dp[4 * qq + e] = nd[e];
-                }
+                for (int qq = q * (DC < 4 ? 4 / DC : 1); qq < (q + 1) * (DC < 4 ? 4 / DC : 1); ++qq) neg_dots(qq);
             }
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = masked_score(s[i], p.c2, ml[i]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) neg_dots(q);
         }
         // Blocks whose rows all see all 32 keys (uniform) need no per-element test.
         if (!(kw0 + 31 < g.lk && (!p.causal || kw0 + 31 <= r0b + g.coff))) {
@@ -247,7 +259,7 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
             const int seen = key >= g.lk ? 32 : (p.causal ? key - g.coff - r0b - 4 * h2 : -1);
 #pragma unroll
             for (int i = 0; i < 16; ++i)
-                if (8 * (i / 4) + i % 4 < seen) s[i] = p.hidden;
+                if (8 * (i / 4) + i % 4 < seen) s[i] = hidden;
         }
         __builtin_amdgcn_sched_barrier(0);
         // dP, with P formed from S meanwhile.
@@ -275,7 +287,7 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
                 if (k * DC / 8 == c) {
 #pragma unroll
                     for (int i = 2 * k; i < 2 * k + 2; ++i) {
-                        s[i] = __builtin_amdgcn_exp2f(s[i] * p.c2 - l2[(k / 2) % 2][i % 4]);
+                        s[i] = __builtin_amdgcn_exp2f(s[i] * xs - l2[(k / 2) % 2][i % 4]);
                         pb[i / 8][i % 8] = from_f32<T>(s[i]);
                     }
                     if (k % 2 == 1 && k / 2 + 2 < 4) l2[(k / 2) % 2] = lse4(k / 2 + 2);
@@ -322,7 +334,7 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
             bool raw;
             row_stats(lse_n, r0 + lane < g.lq, l2, raw);
             sh.stats[buf][0][lane] = l2;
-            if constexpr (MK != MK_NONE) sh.stats[buf][2][lane] = raw ? 1.f : 0.f;
+            if constexpr (MASKED) sh.stats[buf][2][lane] = raw ? 1.f : 0.f;
         }
         __syncthreads();
         if (it + p.splits < items) request(gi, bi, buf ^ 1);
@@ -465,12 +477,14 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
     };
     const typename TL::Addr ad = TL::addr(lane);
     typedef typename MaskRaw<MK>::type MRaw;
+    constexpr bool MASKED = MK != MK_NONE;
+    const float xs = MASKED ? 1.f : p.c2, hidden = MASKED ? -INFINITY : p.hidden;  // (as in bwd_dkdv)
     const int64_t moff = g.mbase + h * p.ms[1] + pos * g.mrow;  // the row's mask values
 
     // One 32-key block (keys kb0 ..) at LDS address kt (V's a tile on).
     auto block = [&](uint32_t kt, int kb0) {
-        f32x16 s = splat16(0.f), dp = splat16(nd);  // (s: as in bwd_dkdv)
-        if constexpr (MK != MK_NONE) {
+        f32x16 s = splat16(0.f), ml, dp = splat16(nd);  // (ml: as in bwd_dkdv)
+        if constexpr (MASKED) {
             // Unit key stride: four consecutive keys per load.
             const bool vec = g.mkey == 1 && kb0 + 31 < g.lk && (p.mask_mode != KMI_MASK_PACKED || g.mpacked_ok);
             if (vec) {
@@ -481,14 +495,16 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
 #pragma unroll
                 for (int q = 0; q < 4; ++q) __builtin_memcpy(&x[q], src + 8 * q, sizeof(E));
 #pragma unroll
-                for (int i = 0; i < 16; ++i) s[i] = mask_logit_of<MK>(x[i / 4].e[i % 4]);
+                for (int i = 0; i < 16; ++i) ml[i] = mask_value_of<MK>(x[i / 4].e[i % 4]);
             } else {
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
-                    s[i] = mask_at<MK>(p, g, h, pos, min(kb0 + 8 * (i / 4) + 4 * h2 + i % 4, g.lk - 1));
+                    ml[i] = mask_at<MK>(p, g, h, pos, min(kb0 + 8 * (i / 4) + 4 * h2 + i % 4, g.lk - 1));
             }
+            if (__builtin_amdgcn_ballot_w64(raw)) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = raw ? 0.f : (s[i] > kMaskedLogit ? s[i] * p.mask_c : p.hidden);
+                for (int i = 0; i < 16; ++i) ml[i] = raw ? 0.f : ml[i];
+            }
         }
         uint32_t ra = kt + ad.row, t0 = kt + ad.tr0, t1 = kt + ad.tr1;
         __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1));  // (as in bwd_dkdv)
@@ -508,11 +524,15 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
             fa[i % LA] = operand(i + LA);
             __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = masked_score(s[i], p.c2, ml[i]);
+        }
         if (kb0 + 31 >= lim_w) {
             const int rel = lim - kb0 - 4 * h2;  // keys whose index is below rel are visible
 #pragma unroll
             for (int i = 0; i < 16; ++i)
-                if (8 * (i / 4) + i % 4 >= rel) s[i] = p.hidden;
+                if (8 * (i / 4) + i % 4 >= rel) s[i] = hidden;
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -522,8 +542,8 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 if (k * DC / 8 == i) {
-                    s[2 * k] = __builtin_amdgcn_exp2f(s[2 * k] * p.c2 - l2);
-                    s[2 * k + 1] = __builtin_amdgcn_exp2f(s[2 * k + 1] * p.c2 - l2);
+                    s[2 * k] = __builtin_amdgcn_exp2f(s[2 * k] * xs - l2);
+                    s[2 * k + 1] = __builtin_amdgcn_exp2f(s[2 * k + 1] * xs - l2);
                 }
             __builtin_amdgcn_sched_barrier(0);
         }

@@ -407,3 +407,60 @@ def test_torch_varlen_attn_forward_and_backward(native, dev):
     for name, got, want in zip(("dq", "dk", "dv"), (qd.grad, kd.grad, vd.grad), ref):
         err = (got.cpu().double() - want).abs().max().item()
         assert err <= 3e-2 * max(want.abs().max().item(), 1.0), (name, err)
+
+
+def _grads_of(q, k, v, go, mask):
+    ts = [t.detach().requires_grad_() for t in (q, k, v)]
+    F.scaled_dot_product_attention(*ts, attn_mask=mask).backward(go)
+    return [t.grad for t in ts]
+
+
+@pytest.mark.parametrize("kind", ["add", "bool", "pad"])
+@pytest.mark.parametrize("b,h,s,d", [(1, 2, 70, 64), (1, 2, 70, 128), (4, 8, 257, 128), (4, 8, 257, 96)])
+def test_masked_keys_may_hold_anything(native, dev, b, h, s, d, kind):
+    """dK and dV do not depend on the K rows of masked keys (NaN, infinities, values whose
+    product overflows) and are exactly 0 there.  (dQ sums dS K over every key, so a NaN row
+    reaches it.)"""
+    print(f"masked rows {b}x{h}x{s}x{d} {kind}", flush=True)
+    g = C.gen(980 + d)
+    q, k, v, go = (C.randn(g, b, h, s, d).to(dev) for _ in range(4))
+    hidden = torch.rand(s, generator=g) < 0.4
+    hidden[::32] = False  # each tile keeps a key
+    if kind == "pad":
+        m = (~hidden).view(1, 1, 1, s).expand(b, 1, 1, s)
+    else:
+        m = (torch.rand(1, 1, s, s, generator=g) >= 0.2) & ~hidden
+        m[..., ::32] = True
+        if kind == "add":
+            m = torch.randn(1, 1, s, s, generator=g).bfloat16().masked_fill(~m, -torch.inf)
+    hidden, m = hidden.to(dev), m.to(dev)
+    clean = k.masked_fill(hidden[None, None, :, None], 0.0)
+    spoilt = clean.clone()
+    at = torch.nonzero(hidden).flatten()
+    for i, value in enumerate((torch.nan, torch.inf, -torch.inf, torch.finfo(k.dtype).max)):
+        spoilt[:, :, at[i::4]] = value
+    _, dk, dv = _grads_of(q, spoilt, v, go, m)
+    _, want_dk, want_dv = _grads_of(q, clean, v, go, m)
+    assert torch.isfinite(want_dk).all() and torch.isfinite(want_dv).all()
+    assert torch.equal(dk, want_dk) and torch.equal(dv, want_dv)
+    assert not dk[:, :, at].any() and not dv[:, :, at].any()
+
+
+@pytest.mark.parametrize("b,h,s", [(2, 2, 128), (4, 8, 257)])
+def test_additive_mask_rounds_once(native, dev, b, h, s):
+    """A logit of -1e5 over whole rows leaves the probabilities as they are but for roundings
+    at its size.  In base 2 (2^17 .. 2^18, a rounding is off by 2^-6 / sqrt(12) in the mean):
+    one of score + logit, one of the forward's lse before and one after it is scaled back to
+    base 2, and one of its natural value (2^-7 log2(e) / sqrt(12)).  dV is off by ln 2 times
+    their root sum of squares."""
+    print(f"rounds once {b}x{h}x{s}", flush=True)
+    g = C.gen(990 + s)
+    q, k, v, go = (C.randn(g, b, h, s, 128).half() for _ in range(4))
+    mask = torch.full((1, 1, s, s), -1e5)
+    _, _, dv = _grads_of(q.to(dev), k.to(dev), v.to(dev), go.to(dev), mask.to(dev))
+    p = torch.softmax(q.double() @ k.double().transpose(-1, -2) / 128**0.5, -1)
+    want = p.transpose(-1, -2) @ go.double()
+    off = ((dv.cpu().double() - want).norm() / want.norm()).item()
+    once = 2.0**-6 / 12**0.5 * (3 + (np.log2(np.e) / 2) ** 2) ** 0.5 * np.log(2)
+    print(f"  {off:.2e}, derived {once:.2e}", flush=True)
+    assert off <= 1.2 * once
