@@ -326,7 +326,9 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdParams& p, const int bid)
                     bool keep = key < g.lk && (!p.causal || key <= row + g.coff);
                     float add = 0.f;
                     if constexpr (MK != MK_NONE) {
-                        const float ml = (keep && row < g.lq) ? mask_at<MK>(p, g, h, row, key) : 0.f;
+                        // (Rows past the end keep nothing: their lse alone would not hide a
+                        // masked key whose product is NaN.)
+                        const float ml = (keep && row < g.lq) ? mask_at<MK>(p, g, h, row, key) : kMaskedLogit;
                         keep = keep && (raw || ml > kMaskedLogit);
                         add = raw ? 0.f : ml * kLog2e;
                     }

@@ -416,7 +416,7 @@ def _grads_of(q, k, v, go, mask):
 
 
 @pytest.mark.parametrize("kind", ["add", "bool", "pad"])
-@pytest.mark.parametrize("b,h,s,d", [(1, 2, 70, 64), (1, 2, 70, 128), (4, 8, 257, 128), (4, 8, 257, 96)])
+@pytest.mark.parametrize("b,h,s,d", [(1, 2, 70, 64), (1, 2, 70, 128), (4, 8, 257, 128), (4, 8, 257, 96), (2, 2, 66, 256)])
 def test_masked_keys_may_hold_anything(native, dev, b, h, s, d, kind):
     """dK and dV do not depend on the K rows of masked keys (NaN, infinities, values whose
     product overflows) and are exactly 0 there.  (dQ sums dS K over every key, so a NaN row
