@@ -464,3 +464,53 @@ def test_additive_mask_rounds_once(native, dev, b, h, s):
     once = 2.0**-6 / 12**0.5 * (3 + (np.log2(np.e) / 2) ** 2) ** 0.5 * np.log(2)
     print(f"  {off:.2e}, derived {once:.2e}", flush=True)
     assert off <= 1.2 * once
+
+
+@pytest.mark.parametrize("kind", ["bool", "additive", "float32", "pad"])
+@pytest.mark.parametrize("b,hq,hk,sq,sk,d,dtype", [
+    (4, 8, 8, 257, 259, 128, torch.bfloat16),
+    (4, 8, 8, 257, 259, 96, torch.float16),
+    (6, 12, 6, 161, 225, 128, torch.float16),
+])  # fmt: skip
+def test_masked_backward_of_128_key_workgroups(native, dev, b, hq, hk, sq, sk, d, dtype, kind):
+    """Masked calls large enough that a dK / dV workgroup takes 128 keys (32-row tiles, V in
+    LDS), with key and row counts off both, and a row that keeps no key."""
+    # 64-key and 64- or 128-row workgroups in all: more than the 256 that keep 64 keys each.
+    dq_wgs = b * hq * -(-sq // 128)
+    assert b * hk * -(-sk // 64) + (dq_wgs if dq_wgs >= 256 else b * hq * -(-sq // 64)) > 256
+    print(f"128-key workgroups {b}x{hq}/{hk}x{sq}/{sk}x{d} {kind}", flush=True)
+    g = C.gen(d + sq + len(kind))
+    q, go = C.randn(g, b, hq, sq, d).to(dtype), C.randn(g, b, hq, sq, d).to(dtype)
+    k, v = C.randn(g, b, hk, sk, d).to(dtype), C.randn(g, b, hk, sk, d).to(dtype)
+    if kind == "bool":
+        mask = torch.rand(b, hq, sq, sk, generator=g) > 0.3
+        mask[1, 1, 7] = False
+    elif kind == "pad":
+        lens = torch.randint(1, sk + 1, (b,), generator=g)
+        mask = (torch.arange(sk)[None, :] < lens[:, None]).reshape(b, 1, 1, sk)
+    else:
+        mask = torch.randn(b if kind == "float32" else 1, 1, sq, sk, generator=g)
+        mask = mask.masked_fill(torch.rand(mask.shape, generator=g) < 0.2, -torch.inf)
+        mask[0, 0, 3] = -torch.inf
+        if kind == "additive":
+            mask = mask.to(dtype)
+    ts = [t.to(dev).requires_grad_() for t in (q, k, v)]
+    native.reset_counters()
+    out = F.scaled_dot_product_attention(*ts, attn_mask=mask.to(dev), enable_gqa=hq != hk)
+    out.backward(go.to(dev))
+    assert native.counters()["attention_backward"] == 1
+    keep = mask if kind in ("bool", "pad") else mask > -torch.inf
+    dead = ~keep.any(-1, keepdim=True)  # these rows are over their raw scores
+    bias = torch.zeros(mask.shape, dtype=torch.float64) if kind in ("bool", "pad") else mask.double().masked_fill(~keep, 0.0)
+    bias = bias.masked_fill(~keep & ~dead, -torch.inf)
+    rs = [t.double().requires_grad_() for t in (q, k, v)]
+    kr, vr = (t.repeat_interleave(hq // hk, 1) for t in rs[1:])
+    p = torch.softmax(rs[0] @ kr.transpose(-1, -2) / d**0.5 + bias, -1)
+    (p @ vr).backward(go.double())
+    half_ulp = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
+    for name, a, r in zip(("dq", "dk", "dv"), ts, rs):
+        # P, dS, out and the gradient itself round to the type, O in the row dot too: five half
+        # ulps of what the gradient's size is made of, in the mean over a tensor.
+        off = ((a.grad.cpu().double() - r.grad).norm() / r.grad.norm()).item()
+        print(f"  {name} {off:.2e}", flush=True)
+        assert torch.isfinite(a.grad).all() and off <= 5 * half_ulp, (name, off)
