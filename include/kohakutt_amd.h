@@ -135,6 +135,11 @@ typedef struct kmi_attn_args {
 /* Bytes of workspace kmi_attn_fwd needs for `args` (0 when it does not split). */
 int kmi_attn_workspace_bytes(const kmi_attn_args* args, size_t* bytes);
 
+/* The kernel kmi_attn_fwd runs `args` on, a static string: "decode" (at most 16 rows per
+ * K/V head), "tile128" or "tile64" (attn_tile_kernel by rows per workgroup), "pipe"
+ * (attn_pipe_kernel), "row_split" or "general" (attn_fwd_kernel).  For tests and profiles. */
+int kmi_attn_fwd_kernel(const kmi_attn_args* args, const char** name);
+
 /*
  * Enqueues the attention forward of `args` on `stream` (hipStream_t).  Split decode calls
  * merge their splits in the same launch through a library-owned counter array (one slab

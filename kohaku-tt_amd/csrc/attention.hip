@@ -429,6 +429,17 @@ extern "C" int kmi_attn_workspace_bytes(const kmi_attn_args* args, size_t* bytes
     return KMI_OK;
 }
 
+extern "C" int kmi_attn_fwd_kernel(const kmi_attn_args* args, const char** name) {
+    using namespace kmi;
+    using namespace kmi::fwd;
+    if (!name) return fail(KMI_EINVAL, "kmi_attn_fwd_kernel: null name");
+    if (const char* why = check_args(args)) return fail(KMI_EINVAL, std::string("kmi_attn_fwd_kernel: ") + why);
+    const Plan pl = make_plan(args);
+    *name = pl.tile ? (pl.row_groups == 4 ? "tile128" : "tile64")
+                    : (pl.decode ? "decode" : (pl.pipe ? "pipe" : (pl.rs ? "row_split" : "general")));
+    return KMI_OK;
+}
+
 extern "C" int kmi_attn_fwd(const kmi_attn_args* a, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace kmi;
     using namespace kmi::fwd;

@@ -19,6 +19,7 @@ KMI_MASK_NONE, KMI_MASK_STRIDED, KMI_MASK_PACKED = 0, 1, 2
 
 EXPORTS = (
     "kmi_attn_workspace_bytes",
+    "kmi_attn_fwd_kernel",
     "kmi_attn_fwd",
     "kmi_attn_fwd_noalloc",
     "kmi_attn_bwd_workspace_bytes",
@@ -140,6 +141,7 @@ def lib():
         h = ctypes.CDLL(str(LIB_PATH))
         vp, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32
         h.kmi_attn_workspace_bytes.argtypes = [ctypes.POINTER(AttnArgs), ctypes.POINTER(ctypes.c_size_t)]
+        h.kmi_attn_fwd_kernel.argtypes = [ctypes.POINTER(AttnArgs), ctypes.POINTER(ctypes.c_char_p)]
         h.kmi_attn_fwd.argtypes = [ctypes.POINTER(AttnArgs), vp, ctypes.c_size_t, vp]
         h.kmi_attn_fwd_noalloc.argtypes = [ctypes.POINTER(AttnArgs), vp]
         h.kmi_attn_bwd_workspace_bytes.argtypes = [ctypes.POINTER(AttnBwdArgs), ctypes.POINTER(ctypes.c_size_t)]
@@ -170,6 +172,13 @@ def workspace_bytes(args: AttnArgs) -> int:
     n = ctypes.c_size_t(0)
     check(lib().kmi_attn_workspace_bytes(ctypes.byref(args), ctypes.byref(n)))
     return n.value
+
+
+def attn_fwd_kernel(args: AttnArgs) -> str:
+    """The kernel ``kmi_attn_fwd`` runs the call on."""
+    name = ctypes.c_char_p()
+    check(lib().kmi_attn_fwd_kernel(ctypes.byref(args), ctypes.byref(name)))
+    return name.value.decode()
 
 
 def attn_fwd(args: AttnArgs, workspace: int, workspace_bytes_: int, stream: int) -> None:

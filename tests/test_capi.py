@@ -103,6 +103,29 @@ def test_workspace_sizes_follow_the_split_plan():
     assert capi.workspace_bytes(b) == 0
 
 
+@pytest.mark.parametrize(
+    "kw,kernel",
+    [
+        (dict(batch=8, heads_q=16, seq_q=1, seq_k=4096), "decode"),
+        (dict(batch=32, heads_q=12, heads_kv=12, seq_q=197, seq_k=197), "row_split"),
+        (dict(heads_q=14, seq_q=2048, seq_k=2048, causal=1), "pipe"),
+        (dict(batch=2, heads_q=10, heads_kv=10, seq_q=4096, seq_k=4096), "general"),
+        (dict(heads_q=24, heads_kv=24, seq_q=4396, seq_k=4396, head_dim=128), "tile128"),
+        (dict(heads_q=16, heads_kv=16, seq_q=2048, seq_k=2048, mask=0x2000, mask_dtype=capi.KMI_BF16,
+              mask_mode=capi.KMI_MASK_STRIDED, mask_stride=(ctypes.c_int64 * 4)(0, 0, 2048, 1)), "tile64"),
+        (dict(batch=8, heads_q=16, heads_kv=8, seq_q=1024, seq_k=1024, head_dim=128, causal=1, cu_seqlens_q=0x3000,
+              cu_seqlens_k=0x3000, total_q=4349, total_k=4349), "tile128"),
+    ],
+)  # fmt: skip
+def test_the_plan_names_its_kernel(kw, kernel):
+    assert capi.attn_fwd_kernel(_args(**kw)) == kernel
+
+
+def test_the_kernel_of_a_refused_call_is_an_error():
+    with pytest.raises(capi.KmiError, match="heads_kv must divide"):
+        capi.attn_fwd_kernel(_args(heads_kv=3))
+
+
 def test_value_head_dim_sizes_the_split_partials():
     # The split partials are as wide as the larger head dim, padded (to 32, 64, 96, 128,
     # 192 or 256; head_dim_v 0 means head_dim): D 128 with Dv 200 keeps partials of 256

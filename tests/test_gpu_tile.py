@@ -1,7 +1,10 @@
-"""The 32x32x16 tile forward (attn_tile_kernel) against float64, at sizes its plan takes:
-row and key counts one off its 32-row groups, 64- and 128-row workgroups and 32- to 128-key
-tiles, GQA, causal, masks (rows that keep no key among them), key lengths, packed ragged
-batches, every padded head dim, a value head dim of its own, and scales of any sign."""
+"""Prefill forwards against float64 around the plan's line for the 32x32x16 tile kernel
+(attn_tile_kernel): row and key counts one off its 32-row groups, 64- and 128-row workgroups
+and 32- to 128-key tiles, GQA, causal, masks (rows that keep no key among them), key lengths,
+packed ragged batches, a value head dim of its own, and scales of any sign.  CASES and the
+packed batch lie on both sides of the line; ROUTED and the longer packed batch name the form
+that takes them (the plan is asked) and cover each padded head dim, both workgroup sizes, both
+types, each mask type and packed masks."""
 
 from __future__ import annotations
 
@@ -10,6 +13,8 @@ import math
 import pytest
 import torch
 import torch.nn.functional as F
+
+from kohakutt_amd import capi
 
 pytestmark = pytest.mark.gpu
 
@@ -63,9 +68,70 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def _kernel(q, k, v, mask=None, causal=False, cu=None, longest=0):
+    """The kernel the plan gives a call: dense [B, H, S, D], or packed [T, H, D] with host
+    offsets (mask then flat and block-packed)."""
+    a = capi.AttnArgs()
+    a.q, a.k, a.v, a.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), q.data_ptr()
+    a.dtype = {torch.bfloat16: capi.KMI_BF16, torch.float16: capi.KMI_F16}[q.dtype]
+    a.causal = int(causal)
+    a.head_dim, a.head_dim_v, a.scale = q.size(-1), v.size(-1), 1.0
+    axes = (0, 1, 2)
+    if cu is None:
+        a.batch, a.heads_q, a.seq_q = q.shape[:3]
+        a.heads_kv, a.seq_k = k.shape[1:3]
+    else:
+        a.batch, a.heads_q, a.heads_kv, a.seq_q, a.seq_k = len(cu) - 1, q.size(1), k.size(1), longest, longest
+        a.cu_seqlens_q = a.cu_seqlens_k = q.data_ptr()
+        a.total_q = a.total_k = q.size(0)
+        axes = (0, 1, 0)
+    for field, t in (("q_stride", q), ("k_stride", k), ("v_stride", v)):
+        getattr(a, field)[:] = [t.stride(i) for i in axes]
+    a.o_stride[:] = [8 * math.ceil(s / 8) for s in a.q_stride]
+    if mask is not None:
+        a.mask = mask.data_ptr()
+        a.mask_dtype = {torch.bool: capi.KMI_BOOL, torch.bfloat16: capi.KMI_BF16, torch.float16: capi.KMI_F16,
+                        torch.float32: capi.KMI_F32}[mask.dtype]  # fmt: skip
+        if cu is None:
+            a.mask_mode = capi.KMI_MASK_STRIDED
+            m = mask.expand(q.size(0), q.size(1), q.size(2), k.size(2))
+            a.mask_stride[:] = list(m.stride())
+        else:
+            a.mask_mode, a.mask_numel = capi.KMI_MASK_PACKED, mask.numel()
+    return capi.attn_fwd_kernel(a)
+
+
+BF, HF = torch.bfloat16, torch.float16
+ROUTED = [
+    # as CASES, and the kernel
+    (8, 16, 16, 300, 297, 32, False, None, BF, "tile64"),
+    (10, 16, 16, 300, 300, 32, True, None, HF, "tile128"),
+    (8, 16, 16, 300, 290, 64, False, None, HF, "tile64"),
+    (10, 16, 16, 300, 261, 64, False, None, BF, "tile128"),
+    (4, 24, 24, 129, 257, 96, False, None, HF, "tile64"),
+    (4, 24, 24, 300, 257, 96, False, None, BF, "tile128"),
+    (6, 24, 24, 300, 300, 96, True, None, BF, "tile64"),
+    (7, 24, 24, 300, 300, 96, True, None, HF, "tile128"),
+    (4, 24, 12, 300, 200, 128, False, None, HF, "tile64"),
+    (8, 24, 12, 300, 300, 128, True, None, HF, "tile128"),
+    (4, 16, 16, 300, 300, 32, False, "bool", HF, "tile64"),
+    (8, 16, 16, 400, 300, 32, False, "add", BF, "tile128"),
+    (8, 16, 16, 400, 333, 40, False, "f32", HF, "tile128"),
+    (8, 16, 16, 400, 333, 64, False, "add", BF, "tile128"),
+    (8, 16, 16, 400, 333, 64, False, "bool", BF, "tile128"),
+    (8, 12, 12, 400, 384, 64, False, "pad", HF, "tile128"),
+    (6, 8, 8, 400, 401, 96, False, "add", HF, "tile64"),
+    (8, 12, 12, 400, 384, 96, False, "pad", BF, "tile128"),
+    (8, 12, 12, 400, 384, 128, False, "pad", BF, "tile128"),
+    (6, 8, 8, 200, 320, 192, False, "bool", BF, "tile64"),
+    (6, 8, 8, 300, 320, 256, False, "pad", BF, "tile64"),
+    (6, 8, 8, 300, 319, 256, False, "add", HF, "tile64"),
+]  # fmt: skip
+
+
+@pytest.mark.parametrize("case", CASES + ROUTED, ids=lambda c: "x".join(map(str, c)))
 def test_dense_calls_meet_float64(native, dev, case):
-    b, hq, hk, sq, sk, d, causal, mask, dtype = case
+    b, hq, hk, sq, sk, d, causal, mask, dtype = case[:9]
     print(f"tile {case}", flush=True)
     g = torch.Generator(device=dev).manual_seed(sum(case[:6]))
     randn = lambda *s: torch.randn(*s, generator=g, device=dev).to(dtype)  # noqa: E731
@@ -87,6 +153,8 @@ def test_dense_calls_meet_float64(native, dev, case):
         m[1] = False  # no key at all: raw scores
     if m is not None and m.dtype == torch.bool:
         bias = torch.zeros(m.shape, device=dev).masked_fill(~m, -math.inf)
+    if len(case) > 9:
+        assert _kernel(q, k, v, m, causal) == case[9]
     if causal:
         bias = torch.zeros(sq, sk, device=dev).masked_fill(~torch.ones(sq, sk, dtype=torch.bool, device=dev).tril(), -math.inf)
     native.reset_counters()
@@ -135,6 +203,42 @@ def test_packed_ragged_batches_meet_float64(native, dev, d, dv, causal):
         if causal:
             bias = torch.zeros(b - a, b - a, device=dev)
             bias = bias.masked_fill(~torch.ones(b - a, b - a, dtype=torch.bool, device=dev).tril(), -math.inf)
+        want, weight, _ = _attend(qs, ks, vs, bias, 1 / math.sqrt(d))
+        _close(out[a:b].transpose(0, 1), want, weight, torch.bfloat16)
+
+
+@pytest.mark.parametrize("d,masked,kernel", [(64, False, "tile128"), (32, True, "tile128"), (64, True, "tile128"),
+                                             (96, False, "tile128"), (128, True, "tile64")])  # fmt: skip
+@pytest.mark.parametrize("causal", [False, True])
+def test_longer_packed_batches_meet_float64(native, dev, d, masked, kernel, causal):
+    """The batch of the test above and one more sequence, with a block-packed mask too (a row
+    that keeps no key in each sequence of more than one)."""
+    lens = [700, 1, 129, 64, 333, 520, 65, 31, 250, 400, 128, 610, 699]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    g = torch.Generator(device=dev).manual_seed(d + causal)
+    randn = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()  # noqa: E731
+    q, k, v = randn(cu[-1], 24, d), randn(cu[-1], 12, d), randn(cu[-1], 12, d)
+    blocks = []
+    for n in lens:
+        m = torch.randn(n, n, generator=g, device=dev).masked_fill(
+            torch.rand(n, n, generator=g, device=dev) < 0.3, -math.inf)
+        if n > 1:
+            m[n // 2] = -math.inf
+        blocks.append(m)
+    packed = torch.cat([m.flatten() for m in blocks]).bfloat16() if masked else None
+    assert _kernel(q, k, v, packed, causal, cu, max(lens)) == kernel
+    out = native.sdpa_varlen(q, k, v, cu, is_causal=causal, packed_mask=packed)
+    for a, b, m in zip(cu[:-1], cu[1:], blocks):
+        n = b - a
+        qs, ks, vs = (t[a:b].transpose(0, 1) for t in (q, k.repeat_interleave(2, 1), v.repeat_interleave(2, 1)))
+        seen = torch.ones(n, n, dtype=torch.bool, device=dev)
+        seen = seen.tril() if causal else seen
+        bias = m.bfloat16().double() if masked else torch.zeros(n, n, device=dev, dtype=torch.float64)
+        kept = ((bias > -math.inf) & seen).any(-1, keepdim=True)
+        # (A row whose seen keys are all masked is over their raw scores.)
+        bias = torch.where(kept, bias, torch.zeros_like(bias)).masked_fill(~seen, -math.inf)
         want, weight, _ = _attend(qs, ks, vs, bias, 1 / math.sqrt(d))
         _close(out[a:b].transpose(0, 1), want, weight, torch.bfloat16)
 
