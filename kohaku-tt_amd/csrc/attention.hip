@@ -122,13 +122,23 @@ bool nqb_allowed(int dp, int nqb, bool masked) {
 //     256) 15 / 15 / 12; up to 128 keys the row split stays ahead (2x10x4096/77 15 / 20 / 23)
 //   additive mask: 4x16x1000 169 / 77 / 68, 1x16x1000 (w2 256) 46 / 61 / 28
 //   padding mask: 2x16x2000 282 / 79 / 119, 4x16x512 (w4 256) 55 / 25 / 20
-//   head dims up to 64, not causal: 4x16x512 (w4 256) 15 / 11 / 11, 4x16x1000 (512) 36 / 26 /
-//     29, 2x10x4096 (640: a second round a quarter full) 114 / 123 / 115; up to 256 keys the
-//     row split stays ahead (32x12x197 15 / 17 / 21)
+//   head dims up to 64, not causal: 4x16x512 (w4 256) 15 / 11 / 11, 4x16x1000 (512) 34 / 25 /
+//     29, 16x12x700 (1152) 61 / 45 / 52, 4x16x4096 (2048) 331 / 324 / 369; up to 256 keys the
+//     row split stays ahead (32x12x197 15 / 17 / 21).  With 513 to 715 workgroups a second
+//     round is mostly empty, which costs head dim 64 with thousands of keys the gain
+//     (2x10x3300 (520) 98 / 104, 3700 (580) 106 / 113, 4096 (640) 114 / 123; 3x10x3000 (720)
+//     99 / 95); a third round costs it nothing (4x10x3300 (1040) 160 / 160, 3700 (1160) 187 /
+//     179), and at smaller head dims and in packed calls the tile kernel leads on both sides
+//     of that line (4x16x1000x32 (512) 29 / 22, 11x16x700x40 (1056) 54 / 38, 12 packed x 24/12
+//     x 31 to 700 x 64 (828) 55 / 38)
 //   causal (attn_pipe_kernel at 64): 8x16x700 (w4 768) 22 / 22 / 24, 4x32/8x3576 (3584) 300 /
 //     257 / 296
 //   additive mask: 16x2048 (w4 256) 80 / 71 / 45, 4x16x1000 (512) 89 / 50 / 57
 //   head dims past 128 (64 rows): 16x1600 170 / 77, 2x8x500 (w2 128) 24 / 19, causal 18 / 19
+// Calls whose rows fit 64 take 64-row workgroups unless they see one tile of keys (512 units;
+// padding mask, 20 rows x 512 keys x 64 16 / 20 / 16, 49 x 512 x 128 55 / 26 / 22; additive, 49 x
+// 512 x 64 30 / 25 / 21, but 64 x 64 x 64 14 / 8 / 15; no mask, 40 x 300 x 96 38 / 27 / 25, 7 query
+// heads x 4 rows x 512 x 64 15 / 14 / 14).
 int tile_row_groups(const kmi_attn_args* a, const Plan& pl, int dp) {
     if (pl.decode || pl.splits > 1 || nqb_override() != 0 || !tile_enabled()) return 0;
     const int64_t G = a->heads_q / a->heads_kv;
@@ -140,20 +150,22 @@ int tile_row_groups(const kmi_attn_args* a, const Plan& pl, int dp) {
     const bool masked = a->mask_mode != KMI_MASK_NONE;
     // A mask that depends on the key alone skips whole tiles in every row.
     const bool by_key = a->mask_mode == KMI_MASK_STRIDED && a->mask_stride[1] == 0 && a->mask_stride[2] == 0;
+    const int64_t keys = a->causal && !a->cu_seqlens_q ? std::min(a->seq_q, a->seq_k) : a->seq_k;
+    const int most = a->seq_q * G <= 64 && keys > 64 ? 2 : 4;
     if (dp > 128) return w2 >= (a->causal ? 192 : 128) ? 2 : 0;
     if (masked) {
-        if (w4 >= (by_key ? 320 : 448) && (by_key || dp <= 64)) return 4;
+        if (w4 >= (by_key ? 320 : 448) && (by_key || dp <= 64)) return most;
         return w2 >= (by_key ? 128 : 192) ? 2 : 0;
     }
     if (dp > 64) {
         if (!a->causal && a->seq_k <= kRsTiles * WN) return 0;
-        if (w4 >= (a->causal ? 448 : 256)) return 4;
+        if (w4 >= (a->causal ? 448 : 256)) return most;
         return w2 >= (a->causal ? 384 : 256) ? 2 : 0;
     }
     if (pl.rs) return 0;
     if (pl.pipe) return w4 >= 1024 && a->seq_k >= 512 ? 4 : 0;
-    // (Two workgroups per CU: 512 a round; a last round that is mostly empty loses the gain.)
-    if (w4 >= 1024 || (w4 >= 448 && (w4 <= 512 || w4 >= 716))) return 4;
+    // (Two workgroups per CU: 512 a round; a second round that is mostly empty loses the gain.)
+    if (w4 >= 448 && (w4 <= 512 || w4 >= 716)) return most;
     return w4 < 448 && w2 >= 400 ? 2 : 0;
 }
 

@@ -92,6 +92,9 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
     const int rw0 = r0 + 32 * rg;
     const int row = rw0 + l32;
     const int rr = min(row, vrows - 1);  // rows past the end repeat the last (never written)
+    // (Uniform.)  A wavefront whose rows all lie past the end stages its share of the tiles and
+    // keeps the barriers, nothing else.
+    const bool live = rw0 < vrows;
     const int pos = fdiv(rr, p.fd_group), head = kvh * G + (rr - pos * G);
     const int coff = p.cu_q ? lk - lq : 0;
 
@@ -285,6 +288,16 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             request_v(0, 0);
             if (nt > 1) request_k(1, 1);
             landed();
+        }
+        if (!live) {
+            // The requests and barriers of the steps below (a test inside them costs their
+            // registers: 44 spills at head dim 128 against 9).
+            for (int t = 0; t < nt; ++t) {
+                landed();
+                if (t + 2 < nt) request_k(t + 2, t & 1);
+                if (t + 1 < nt) request_v(t + 1, (t + 1) & 1);
+            }
+        } else if (nt > 0) {
             f32x16 sa[NB], sb[NB];
             uint32_t ra = k_addr(0) + ad.row;
             __asm__ volatile("" : "+v"(ra));
@@ -373,7 +386,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             if (t < nt) {
                 request_k(t, 0);
                 request_v(t, 0);
-                if (pass == 0) load_mask(raw, t);
+                if (pass == 0 && live) load_mask(raw, t);
             }
             while (t < nt) {
                 const int tn = next(t + 1, pass == 1);
@@ -391,11 +404,11 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
                 if (tn < nt) {
                     request_k(tn, buf ^ 1);
                     request_v(tn, buf ^ 1);
-                    if (pass == 0) load_mask(raw, tn);
+                    if (pass == 0 && live) load_mask(raw, tn);
                 }
                 edge(ml, t);
                 // (Uniform.)  A tile in which no row of the wavefront keeps a key adds nothing.
-                if (__builtin_amdgcn_ballot_w64(block_max(ml) > kMaskedLogit)) {
+                if (live && __builtin_amdgcn_ballot_w64(block_max(ml) > kMaskedLogit)) {
                     uint32_t ra = k_addr(buf) + ad.row, t0 = v_addr(buf) + ad.tr0, t1 = v_addr(buf) + ad.tr1;
                     __asm__ volatile("" : "+v"(ra), "+v"(t0), "+v"(t1));
 #pragma unroll
@@ -420,7 +433,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
                     __syncthreads();
                     l = ls[32 * rg + l32] + ls[64 + 32 * rg + l32];
                 }
-                dead = lim > 0 && l == 0.f;
+                dead = live && lim > 0 && l == 0.f;
                 if (__builtin_amdgcn_readfirstlane(__syncthreads_or(dead)) == 0) break;
             }
         }

@@ -126,6 +126,15 @@ ROUTED = [
     (6, 8, 8, 200, 320, 192, False, "bool", BF, "tile64"),
     (6, 8, 8, 300, 320, 256, False, "pad", BF, "tile64"),
     (6, 8, 8, 300, 319, 256, False, "add", HF, "tile64"),
+    # wavefronts whose rows all lie past the end, in both forms
+    (64, 12, 12, 65, 300, 64, False, None, BF, "tile128"),
+    (128, 28, 4, 4, 300, 64, False, None, BF, "tile64"),
+    (128, 28, 4, 4, 300, 128, False, None, HF, "tile64"),
+    (128, 28, 4, 4, 300, 128, True, None, BF, "tile128"),
+    (32, 16, 16, 20, 512, 64, False, "pad", BF, "tile64"),
+    (64, 12, 12, 70, 80, 128, False, "pad", BF, "tile128"),
+    (32, 16, 16, 31, 300, 64, False, "add", BF, "tile64"),
+    (32, 16, 16, 31, 300, 256, False, "f32", BF, "tile64"),
 ]  # fmt: skip
 
 
