@@ -130,7 +130,10 @@ bool nqb_allowed(int dp, int nqb, bool masked) {
 //     99 / 95); a third round costs it nothing (4x10x3300 (1040) 160 / 160, 3700 (1160) 187 /
 //     179), and at smaller head dims and in packed calls the tile kernel leads on both sides
 //     of that line (4x16x1000x32 (512) 29 / 22, 11x16x700x40 (1056) 54 / 38, 12 packed x 24/12
-//     x 31 to 700 x 64 (828) 55 / 38)
+//     x 31 to 700 x 64 (828) 55 / 38).  Past 4096 keys attn_fwd_kernel is as fast or faster at
+//     head dims 56 and 64 (2x10x4600x64 140 / 141, 6600 296 / 310, 10200 624 / 661, 1x16x16384
+//     1174 / 1205, 2x10x6600x56 292 / 303, 2 packed x 8000 and 9600 x 64 570 / 586), not below
+//     (6600x40 302 / 299, x32 237 / 202) nor causal (2x10x9600x64 353 / 284)
 //   causal (attn_pipe_kernel at 64): 8x16x700 (w4 768) 22 / 22 / 24, 4x32/8x3576 (3584) 300 /
 //     257 / 296
 //   additive mask: 16x2048 (w4 256) 80 / 71 / 45, 4x16x1000 (512) 89 / 50 / 57
@@ -164,6 +167,7 @@ int tile_row_groups(const kmi_attn_args* a, const Plan& pl, int dp) {
     }
     if (pl.rs) return 0;
     if (pl.pipe) return w4 >= 1024 && a->seq_k >= 512 ? 4 : 0;
+    if (dp == 64 && a->head_dim > 48 && !a->causal && a->seq_k > 4096) return 0;
     // (Two workgroups per CU: 512 a round; a second round that is mostly empty loses the gain.)
     if (w4 >= 448 && (w4 <= 512 || w4 >= 716)) return most;
     return w4 < 448 && w2 >= 400 ? 2 : 0;

@@ -115,6 +115,11 @@ def test_workspace_sizes_follow_the_split_plan():
               mask_mode=capi.KMI_MASK_STRIDED, mask_stride=(ctypes.c_int64 * 4)(0, 0, 2048, 1)), "tile64"),
         (dict(batch=8, heads_q=16, heads_kv=8, seq_q=1024, seq_k=1024, head_dim=128, causal=1, cu_seqlens_q=0x3000,
               cu_seqlens_k=0x3000, total_q=4349, total_k=4349), "tile128"),
+        # head dim 64 without a mask: up to 4096 keys; smaller head dims and causal calls past it
+        (dict(batch=4, heads_q=16, heads_kv=16, seq_q=4096, seq_k=4096), "tile128"),
+        (dict(batch=4, heads_q=16, heads_kv=16, seq_q=4096, seq_k=4097), "general"),
+        (dict(batch=4, heads_q=16, heads_kv=16, seq_q=4096, seq_k=4097, head_dim=48), "tile128"),
+        (dict(batch=4, heads_q=16, heads_kv=16, seq_q=4096, seq_k=4097, causal=1), "tile128"),
         # rows that fit 64, with more than a tile of keys or not, and one row more
         (dict(batch=32, heads_q=16, heads_kv=16, seq_q=64, seq_k=512, mask=0x2000, mask_dtype=capi.KMI_BOOL,
               mask_mode=capi.KMI_MASK_STRIDED, mask_stride=(ctypes.c_int64 * 4)(512, 0, 0, 1)), "tile64"),
