@@ -172,7 +172,7 @@ int kmi_attn_fwd_noalloc(const kmi_attn_args* args, void* stream);
  * q, k, v, out, grad_out 16-byte aligned with strides multiples of 8 (row strides below
  * 2^25 elements).  Masks take the
  * forward's modes and strides and get no gradient.  Workspace:
- * kmi_attn_bwd_workspace_bytes, 16-byte aligned (fp32 row dot products; when the query
+ * kmi_attn_bwd_plan_bytes, 16-byte aligned (fp32 row dot products; when the query
  * rows of a key tile or the key tiles of a query block are split over workgroups, also
  * fp32 dK / dV and dQ partials, added in a fixed order).
  * Does the work of the reference's flash backward behind tt_sdpa_overrideable_backward's stats
@@ -225,6 +225,10 @@ typedef struct kmi_attn_bwd_args {
 } kmi_attn_bwd_args;
 
 /* Bytes of workspace kmi_attn_bwd needs for `args`. */
+int kmi_attn_bwd_plan_bytes(const kmi_attn_bwd_args* args, size_t* bytes);
+
+/* An upper bound of kmi_attn_bwd_plan_bytes that also holds the splits of earlier plans: up
+ * to five times as much (1 x 24 heads x 4396 x 128: 1027 MB against 216 MB). */
 int kmi_attn_bwd_workspace_bytes(const kmi_attn_bwd_args* args, size_t* bytes);
 
 /* Enqueues the attention backward of `args` on `stream` (hipStream_t). */

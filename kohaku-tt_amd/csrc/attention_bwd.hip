@@ -891,13 +891,19 @@ BwdLayout bwd_layout(const kmi_attn_bwd_args* a, int splits, int ksplit) {
 
 size_t layout_bytes(const BwdLayout& l) { return (l.nd + 2 * l.part + l.pdq) * sizeof(float); }
 
-// The workspace figure: what the plan needs, and never less than attn_bwd_grads' rules give
-// (callers keep buffers sized by it, so a plan with fewer splits does not shrink it).
-size_t bwd_ws_bytes(const kmi_attn_bwd_args* a) {
+// What the plan needs.
+size_t bwd_plan_bytes(const kmi_attn_bwd_args* a) {
     const BwdPlan pl = bwd_plan(a);
+    return layout_bytes(bwd_layout(a, pl.splits, pl.ksplit));
+}
+
+// kmi_attn_bwd_workspace_bytes' figure: never less than attn_bwd_grads' rules give, which
+// split every head dim when the figure was set (tests hold it to that).  An upper bound only:
+// nothing here allocates or asks for it.
+size_t bwd_ws_bytes(const kmi_attn_bwd_args* a) {
     int splits, ksplit;
     grads_splits(a, splits, ksplit);
-    return std::max(layout_bytes(bwd_layout(a, pl.splits, pl.ksplit)), layout_bytes(bwd_layout(a, splits, ksplit)));
+    return std::max(bwd_plan_bytes(a), layout_bytes(bwd_layout(a, splits, ksplit)));
 }
 
 // The gradient kernel of head dims padded past 128.
@@ -976,15 +982,23 @@ extern "C" int kmi_attn_bwd_workspace_bytes(const kmi_attn_bwd_args* a, size_t* 
     return KMI_OK;
 }
 
+extern "C" int kmi_attn_bwd_plan_bytes(const kmi_attn_bwd_args* a, size_t* bytes) {
+    using namespace kmi;
+    using namespace kmi::bwd;
+    if (!bytes) return fail(KMI_EINVAL, "kmi_attn_bwd_plan_bytes: null bytes");
+    if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd_plan_bytes: ") + why);
+    *bytes = bwd_plan_bytes(a);
+    return KMI_OK;
+}
+
 extern "C" int kmi_attn_bwd(const kmi_attn_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace kmi;
     using namespace kmi::bwd;
     if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd: ") + why);
     const BwdPlan pl = bwd_plan(a);
     const BwdLayout l = bwd_layout(a, pl.splits, pl.ksplit);
-    const size_t need = bwd_ws_bytes(a);
-    if (!workspace || workspace_bytes < need || reinterpret_cast<uintptr_t>(workspace) % 16)
-        return fail(KMI_EWORKSPACE, "kmi_attn_bwd: workspace missing or smaller than kmi_attn_bwd_workspace_bytes");
+    if (!workspace || workspace_bytes < layout_bytes(l) || reinterpret_cast<uintptr_t>(workspace) % 16)
+        return fail(KMI_EWORKSPACE, "kmi_attn_bwd: workspace missing or smaller than kmi_attn_bwd_plan_bytes");
     BwdParams p{};
     p.q = a->q;
     p.k = a->k;

@@ -411,7 +411,7 @@ std::tuple<Tensor, Tensor, Tensor> run_backward(const BwdCall& c) {
         }
     }
     size_t ws = 0;
-    check(kmi_attn_bwd_workspace_bytes(&a, &ws), "kmi_attn_bwd_workspace_bytes");
+    check(kmi_attn_bwd_plan_bytes(&a, &ws), "kmi_attn_bwd_plan_bytes");
     Tensor work = at::empty({static_cast<int64_t>(ws)}, q.options().dtype(at::kByte));
     check(kmi_attn_bwd(&a, work.data_ptr(), ws, stream_of(q)), "kmi_attn_bwd");
     g_attn_bwd_calls.fetch_add(1);

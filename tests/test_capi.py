@@ -215,6 +215,32 @@ def test_backward_rejects_malformed_calls_before_launch():
     assert capi.lib().kmi_attn_bwd_workspace_bytes(ctypes.byref(a), ctypes.byref(n)) == capi.KMI_OK
 
 
+@pytest.mark.parametrize(
+    "sizes,floats",
+    [
+        # (batch, heads_q, heads_kv, seq_q, seq_k, head_dim), fp32 words
+        # row dots alone: one split
+        ((8, 16, 8, 1024, 1024, 128), 16 * 8 * 1024),
+        # 64 key workgroups of 448 items: eight splits to fill the chip, dK and dV partials each
+        ((1, 14, 2, 2048, 2048, 64), 14 * 2048 + 2 * (2 * 8 * 2048 * 64)),
+        # 840 of 138 items: two splits of at most 72
+        ((1, 24, 24, 4396, 4396, 128), 24 * 4396 + 2 * (24 * 2 * 4396 * 128)),
+        # past head dim 128 the bound and the plan are one: 48 of two items
+        ((1, 12, 12, 256, 256, 256), None),
+    ],
+)  # fmt: skip
+def test_backward_takes_what_its_plan_needs(sizes, floats):
+    lib, a, n, most = capi.lib(), capi.AttnBwdArgs(), ctypes.c_size_t(), ctypes.c_size_t()
+    a.q = a.k = a.v = a.out = a.grad_out = a.lse = a.grad_q = a.grad_k = a.grad_v = 0x1000
+    a.dtype = capi.KMI_BF16
+    a.batch, a.heads_q, a.heads_kv, a.seq_q, a.seq_k, a.head_dim = sizes
+    assert lib.kmi_attn_bwd_plan_bytes(ctypes.byref(a), ctypes.byref(n)) == capi.KMI_OK
+    assert lib.kmi_attn_bwd_workspace_bytes(ctypes.byref(a), ctypes.byref(most)) == capi.KMI_OK
+    assert n.value == (most.value if floats is None else 4 * floats) and n.value <= most.value
+    assert lib.kmi_attn_bwd(ctypes.byref(a), 0x1000, n.value - 4, None) == capi.KMI_EWORKSPACE
+    assert "kmi_attn_bwd_plan_bytes" in lib.kmi_last_error().decode()
+
+
 def test_rms_norm_backward_rejects_malformed_calls_before_launch():
     lib = capi.lib()
     n = ctypes.c_size_t()

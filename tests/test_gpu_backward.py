@@ -7,12 +7,15 @@ torch's CPU autograd at the same dtype."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
 
 import attn_cases as C
 import numpy as np
+from kohakutt_amd import capi
 from oracle import attention as oatt
 
 pytestmark = pytest.mark.gpu
@@ -514,3 +517,32 @@ def test_masked_backward_of_128_key_workgroups(native, dev, b, hq, hk, sq, sk, d
         off = ((a.grad.cpu().double() - r.grad).norm() / r.grad.norm()).item()
         print(f"  {name} {off:.2e}", flush=True)
         assert torch.isfinite(a.grad).all() and off <= 5 * half_ulp, (name, off)
+
+
+@pytest.mark.parametrize("b,hq,hk,s,d", [(1, 14, 2, 2048, 64), (1, 24, 24, 1000, 128), (1, 2, 1, 70, 256)])
+def test_backward_in_a_workspace_of_the_plans_size(native, dev, b, hq, hk, s, d):
+    """kmi_attn_bwd in the least workspace it takes gives autograd's gradients and writes
+    nothing past it."""
+    print(f"workspace {b}x{hq}/{hk}x{s}x{d}", flush=True)
+    g = C.gen(77 + d)
+    q, k, v, go = (C.randn(g, b, h, s, d).to(dev) for h in (hq, hk, hk, hq))
+    ts = [t.detach().requires_grad_() for t in (q, k, v)]
+    F.scaled_dot_product_attention(*ts, is_causal=True, enable_gqa=True).backward(go)
+    out, lse = torch.ops.aten._scaled_dot_product_fused_attention_overrideable(q, k, v, None, 0.0, True)[:2]
+    grads = [torch.full_like(t, torch.nan) for t in (q, k, v)]
+    a = capi.AttnBwdArgs()
+    for field, t in zip(("q", "k", "v", "out", "grad_out", "lse", "grad_q", "grad_k", "grad_v"),
+                        (q, k, v, out, go, lse, *grads)):  # fmt: skip
+        setattr(a, field, t.data_ptr())
+    for field, t in zip(("q", "k", "v", "o", "do", "dq", "dk", "dv", "lse"), (q, k, v, out, go, *grads, lse)):
+        getattr(a, field + "_stride")[:] = t.stride()[:3]
+    a.dtype, a.causal, a.scale = capi.KMI_BF16, 1, d**-0.5
+    a.batch, a.heads_q, a.heads_kv, a.seq_q, a.seq_k, a.head_dim = b, hq, hk, s, s, d
+    n = ctypes.c_size_t()
+    capi.check(capi.lib().kmi_attn_bwd_plan_bytes(ctypes.byref(a), ctypes.byref(n)))
+    work = torch.full((n.value + 4096,), 0xAB, dtype=torch.uint8, device=dev)
+    capi.check(capi.lib().kmi_attn_bwd(ctypes.byref(a), work.data_ptr(), n.value, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert (work[n.value :] == 0xAB).all()
+    for got, t in zip(grads, ts):
+        assert torch.equal(got, t.grad)
