@@ -78,6 +78,14 @@ SOURCE_FLAGS.update({f"attention_tile_d{d}.hip": ["-fno-honor-nans"] for d in (3
 # resource usage, which check_dma_spills reads.
 RESOURCE_REMARKS = "-Rpass-analysis=kernel-resource-usage"
 SOURCE_FLAGS["attention_d64.hip"] = SOURCE_FLAGS["attention_d64.hip"] + [RESOURCE_REMARKS]
+# So do the units of the 32x32x16 tile kernels, for check_tile_spills.
+TILE_SOURCES = [src for src in HIP_SOURCES if re.fullmatch(r"attention_(tile|bwd)_d\d+\.hip", src)]
+for _src in TILE_SOURCES:
+    SOURCE_FLAGS[_src] = SOURCE_FLAGS.get(_src, []) + [RESOURCE_REMARKS]
+# The most vector registers a tile kernel may spill (13 today, masked backward at head dim 64).
+# Their waits count no loads, so a spill is slow, not wrong: 1x24x4396x128 backward with its
+# fragments spilled took 1351 us instead of 984.
+TILE_VGPR_SPILLS = 16
 
 # attn_fwd_kernel<T, D, NQB, MK, RS, TWIDTH, NW> as the Itanium ABI mangles it.
 _FWD_KERNEL = re.compile(
@@ -98,6 +106,28 @@ def is_dma_forward(mangled: str) -> bool:
             and (nqb == 2 or (nqb == 4 and rs == 0)))
 
 
+def _kernel_resources(remarks: str) -> dict:
+    """{kernel: {figure: value}} of the compiler's resource remarks."""
+    kernels, name = {}, None
+    for key, value in _REMARK.findall(remarks):
+        if key == "Function Name":
+            name = value
+            kernels[name] = {}
+        elif name is not None:
+            kernels[name][key] = int(value)
+    return kernels
+
+
+def check_tile_spills(remarks: str) -> int:
+    """Fails when a tile kernel spills more than TILE_VGPR_SPILLS vector registers; returns how
+    many the remarks list."""
+    tiles = {k: v for k, v in _kernel_resources(remarks).items() if "attn_tile_kernel" in k or "attn_bwd_tile_kernel" in k}
+    bad = {k: v["VGPRs Spill"] for k, v in tiles.items() if v.get("VGPRs Spill", 0) > TILE_VGPR_SPILLS}
+    if bad:
+        raise RuntimeError(f"tile kernels spill more than {TILE_VGPR_SPILLS} vector registers: {bad}")
+    return len(tiles)
+
+
 def check_dma_spills(remarks: str) -> int:
     """Fails when a DMA-staged forward kernel spills VGPRs or uses scratch; returns how many
     such kernels the remarks list.
@@ -106,14 +136,7 @@ def check_dma_spills(remarks: str) -> int:
     counts only the loads the loop issues itself.  A scratch access between a tile's DMA
     and that wait (a VGPR spill reload) would make the wait release early, a silent race.
     SGPR spills go to VGPR lanes and issue no memory instruction."""
-    kernels, name = {}, None
-    for key, value in _REMARK.findall(remarks):
-        if key == "Function Name":
-            name = value
-            kernels[name] = {}
-        elif name is not None:
-            kernels[name][key] = int(value)
-    dma = {k: v for k, v in kernels.items() if is_dma_forward(k)}
+    dma = {k: v for k, v in _kernel_resources(remarks).items() if is_dma_forward(k)}
     bad = [k for k, v in dma.items() if v.get("VGPRs Spill", 0) or v.get("ScratchSize [bytes/lane]", 0)]
     if bad:
         raise RuntimeError(
@@ -135,7 +158,10 @@ def build_capi(jobs: int = 8) -> Path:
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         outs = list(pool.map(_run, cmds))
     for src, out in zip(HIP_SOURCES, outs):
-        if RESOURCE_REMARKS in SOURCE_FLAGS.get(src, []) and check_dma_spills(out) == 0:
+        if src in TILE_SOURCES:
+            if check_tile_spills(out) == 0:
+                raise RuntimeError(f"{src}: no tile kernel in the resource remarks")
+        elif RESOURCE_REMARKS in SOURCE_FLAGS.get(src, []) and check_dma_spills(out) == 0:
             raise RuntimeError(f"{src}: no DMA-staged forward kernel in the resource remarks")
     tmp = CAPI_LIB.with_suffix(".so.tmp")
     _run([str(HIPCC), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)])

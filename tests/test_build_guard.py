@@ -56,3 +56,20 @@ def test_planted_spilling_dma_variant_fails_the_build(spill, scratch):
 
 def test_the_guarded_unit_is_compiled_with_resource_remarks():
     assert _build.RESOURCE_REMARKS in _build.SOURCE_FLAGS["attention_d64.hip"]
+
+
+BWD_TILE = "_ZN3kmi3bwd20attn_bwd_tile_kernelIDF16bLi64ELi2ELb1EEEvNS0_9BwdParamsENS0_7BwdGridE"
+FWD_TILE = "_ZN3kmi3fwd16attn_tile_kernelIDF16bLi128ELi0ELi4EEEvNS0_10AttnParamsE"
+
+
+def test_tile_kernels_may_spill_a_little():
+    most = _build.TILE_VGPR_SPILLS
+    assert _build.check_tile_spills(_remarks((BWD_TILE, most, 76), (FWD_TILE, 0, 24), (MASKED_32, 99, 400))) == 2
+    with pytest.raises(RuntimeError, match="attn_tile_kernelIDF16bLi128"):
+        _build.check_tile_spills(_remarks((BWD_TILE, 0, 0), (FWD_TILE, most + 1, 180)))
+
+
+def test_tile_units_are_compiled_with_resource_remarks():
+    assert len(_build.TILE_SOURCES) == 10
+    for src in _build.TILE_SOURCES:
+        assert _build.RESOURCE_REMARKS in _build.SOURCE_FLAGS[src]
