@@ -26,7 +26,7 @@
 //   2x8/2x3062x128 causal 320 -> 161  (300 -> 597)
 //   1x14/2x2048x64 causal  72 -> 51   (263 -> 373)
 //   8 packed x 16/8 x 128 causal, 64 to 1024 tokens 153 -> 92 (211 -> 354)
-//   2x12x2433x128, additive mask 1426 -> 567 (128 -> 321)
+//   2x12x2433x128, additive mask 1425 -> 586 (128 -> 311)
 // What mattered on the way (1x24x4396x128): no spill in the loop (1351 with fragments
 // spilled -> 984 with V in LDS and one code path per block); swizzles for 64 banks (LDS busy
 // 39% -> 19% of the time); the order of the products (925 -> 861).
@@ -613,8 +613,11 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
         }
 }
 
-// Wavefronts per SIMD the kernel is held to (165 and 237 registers, no spills, unmasked).
-constexpr int bwd_waves(int dp) { return dp <= 64 ? 3 : 2; }
+// Wavefronts per SIMD the kernel is held to: what its LDS leaves room for, three up to head dim
+// 64 (168 registers), two past it with 128-key dK / dV workgroups (214 and 254), one with 64-key
+// ones.  Unmasked kernels spill no vector registers; masked ones up to 13 (head dim 64).  The
+// build fails past _build.TILE_VGPR_SPILLS.
+constexpr int bwd_waves(int dp, bool half) { return dp <= 64 ? 3 : (half ? 1 : 2); }
 
 // Both gradient passes in one launch, their workgroups interleaved in proportion (neither
 // reads the other's output).  Workgroups are dealt to the eight XCDs in turn (block b runs
@@ -622,7 +625,7 @@ constexpr int bwd_waves(int dp) { return dp <= 64 ? 3 : 2; }
 // item number keeps its residue: items with one (sequence, K/V head) fastest stay on few
 // XCDs, whose L2 then holds what they walk over.  Item order: heaviest tiles first.
 template <typename T, int DP, int MK, bool HALF>
-__global__ __launch_bounds__(BWD_THREADS, bwd_waves(DP)) void attn_bwd_tile_kernel(const BwdParams p, const BwdGrid gr) {
+__global__ __launch_bounds__(BWD_THREADS, bwd_waves(DP, HALF)) void attn_bwd_tile_kernel(const BwdParams p, const BwdGrid gr) {
     constexpr size_t DQ_BYTES = 4 * sizeof(T) * Tile<T, DP, 64>::ELEMS;
     constexpr size_t KV_BYTES = sizeof(DkdvShared<T, DP, HALF>);
     __shared__ __align__(1024) unsigned char sh[KV_BYTES > DQ_BYTES ? KV_BYTES : DQ_BYTES];

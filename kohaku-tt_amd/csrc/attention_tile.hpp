@@ -28,10 +28,10 @@ constexpr float kTileLn2 = 0.6931471805599453f;
 
 // Row groups of a workgroup: 4 (128 rows, one wavefront per 32), or 2 (64 rows, two
 // wavefronts per 32 that take one half of each key tile and merge their states at the end).
-// Keys of a tile: 64 (128 for two row groups up to head dim 64, so that a wavefront still has
-// 64), and 32 a wavefront past head dim 128 or with two row groups at 128: 64 KiB of tiles
-// at most, two workgroups per CU.
-constexpr int tile_keys(int dp, int rg) { return dp <= 64 ? (rg == 4 ? 64 : 128) : (dp <= 128 || rg == 2 ? 64 : 32); }
+// Keys of a tile: 64, and 128 for two row groups up to head dim 64, so that a wavefront there
+// still has 64 (32 past it).  64 KiB of tiles at most up to head dim 128, two workgroups per CU;
+// 128 KiB past it, one.
+constexpr int tile_keys(int dp, int rg) { return dp <= 64 && rg == 2 ? 128 : 64; }
 
 // Sum of a packed pair of probabilities (as rounded for the PV product) onto acc.
 template <typename T>
@@ -190,7 +190,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
     // The step below is laid out by hand: one MFMA, the LDS read of the operand LA products
     // on, and a share of the exponentials per group, with no instruction moving between
     // groups (left alone, the compiler issues all exponentials first and then waits for each
-    // operand where it is used: 2x10x4096x64 127 us, against the figures at the top).
+    // operand where it is used: 2x10x4096x64 127 us against 123).
     constexpr int NS = NB * DC, NP = NB * 2 * DB, LA = DP <= 64 ? 4 : 3;
     constexpr int PAIRS = 8 * NB;                       // pairs of scores of a lane
     constexpr int SPREAD = NB > 1 ? NS + NP / NB : NS;  // groups that share them
