@@ -24,6 +24,16 @@ namespace kmi {
 namespace fwd {
 
 constexpr float kTileLazy = 8.f;  // log2 units a row max may grow before O is rescaled
+// The first tiles a wavefront works on (five with four row groups, three of each of a row's two
+// wavefronts with two) set the reference point to their own maximum, also where that is lower
+// (by kTileDrop at most): one weight of each is exactly 1 and so carries no rounding.
+// attn_fwd_kernel has such a weight per wavefront, and its results' distance from 64-bit ones is
+// kept so (relative, attn_fwd_kernel / the first tile alone / as here): 8 packed x 16/8 x 64 to
+// 1024 x 128 causal 0.001932 / 0.001981 / 0.001929, 24x4396x128 0.002338 / 0.002343 / 0.002330,
+// 16x2048x64 additive 0.002019 / 0.002041 / 0.001997; 1% over it is left where a call has two or
+// three tiles.  Costs 1.6% of the masked call (46.2 -> 47.0 us), nothing that shows of the others.
+constexpr int tile_own(int rg) { return rg == 4 ? 5 : 3; }
+constexpr float kTileDrop = 3.f;
 constexpr float kTileLn2 = 0.6931471805599453f;
 
 // Row groups of a workgroup: 4 (128 rows, one wavefront per 32), or 2 (64 rows, two
@@ -168,12 +178,14 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             for (int i = n == 0 ? 1 : 0; i + 1 < 16; i += 2) mx = fmaxf(fmaxf(mx, s[n][i]), s[n][i + 1]);
         return mx;
     };
-    // Moves the reference points that the tile's scores exceed by more than 2^kTileLazy.
-    auto rescale = [&](const f32x16 (&s)[NB]) {
+    // Moves the reference points that the tile's scores exceed by more than 2^kTileLazy (own: that
+    // they do not stay below by 2^kTileDrop).
+    auto rescale = [&](const f32x16 (&s)[NB], bool own) {
         const float lmax = block_max(s);
-        if (__builtin_amdgcn_ballot_w64(lmax * xs > thr)) {
+        const float at = own ? thr - (kTileLazy + kTileDrop) : thr;
+        if (__builtin_amdgcn_ballot_w64(lmax * xs > at)) {
             const float mt = fmaxf(lmax, other_half(lmax)) * xs;
-            const bool move = mt > thr;
+            const bool move = mt > at;
             const float alpha = move ? __builtin_amdgcn_exp2f(m - mt) : 1.f;  // 0 while m was -inf
             if (move) {
                 m = mt;
@@ -230,8 +242,8 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
         }
     };
     // Softmax and PV of a tile alone, from its scores.
-    auto finish = [&](f32x16 (&s)[NB], uint32_t t0, uint32_t t1) {
-        rescale(s);
+    auto finish = [&](f32x16 (&s)[NB], uint32_t t0, uint32_t t1, bool own) {
+        rescale(s, own);
         v8 pb[NB][2], vr[LA];
 #pragma unroll
         for (int j = 0; j < LA; ++j) vr[j] = v_frag(t0, t1, j);
@@ -258,7 +270,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             if (t + 2 < nt) request_k(t + 2, t & 1);
             request_v(t + 1, (t + 1) & 1);
             edge(s, t);
-            rescale(s);
+            rescale(s, t < tile_own(RG));
 #pragma unroll
             for (int n = 0; n < NB; ++n) sn[n] = splat16(0.f);
             __builtin_amdgcn_sched_barrier(0);
@@ -281,7 +293,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             edge(s, t);
             uint32_t t0 = v_addr(t & 1) + ad.tr0, t1 = v_addr(t & 1) + ad.tr1;
             __asm__ volatile("" : "+v"(t0), "+v"(t1));
-            finish(s, t0, t1);
+            finish(s, t0, t1, t < tile_own(RG));
         };
         if (nt > 0) {
             request_k(0, 0);
@@ -354,6 +366,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
             }
             skip = __builtin_amdgcn_readfirstlane(__syncthreads_or(keeps)) != 0;
         }
+        int met = 0;       // tiles the wavefront has worked on
         MRaw raw[NB][16];  // the staged tile's mask values
         auto load_mask = [&](MRaw (&x)[NB][16], int t) {
             const int key0 = t * KT + kw + 4 * h2;
@@ -418,7 +431,7 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
                     for (int n = 0; n < NB; ++n)
 #pragma unroll
                         for (int i = 0; i < 16; ++i) s[n][i] = masked_score(s[n][i], c2, ml[n][i]);
-                    finish(s, t0, t1);
+                    finish(s, t0, t1, met++ < tile_own(RG));
                 }
                 t = tn;
                 buf ^= 1;

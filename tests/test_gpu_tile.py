@@ -321,3 +321,40 @@ def test_additive_mask_rounds_once(native, dev, d):
     once = math.hypot(2.0**-6 / math.sqrt(12) * math.log(2), 2.0**-11 / math.sqrt(3) * math.sqrt(2))
     print(f"d {d}: {got:.2e}, one rounding {once:.2e}", flush=True)
     assert got <= 1.15 * once  # (one rounding: 15% for what is left of a small sample)
+
+
+@pytest.mark.parametrize("b,h,s,d,kind,kernel", [
+    (8, 16, 1000, 128, "causal", "tile128"),
+    (7, 12, 1000, 96, "causal", "tile128"),
+    (8, 8, 1000, 128, "plain", "tile128"),
+    (8, 8, 1000, 64, "add", "tile128"),
+    (4, 8, 1000, 128, "add", "tile64"),
+])  # fmt: skip
+def test_as_close_to_float64_as_the_general_kernel(native, dev, b, h, s, d, kind, kernel):
+    """The same rows through the tile kernel and, one batch entry at a time, through
+    attn_fwd_kernel: the tile kernel's result is no further from float64 (half a percent for
+    the roundings' chance)."""
+    print(f"as close {b}x{h}x{s}x{d} {kind}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(s + d)
+    q, k, v = (torch.randn(b, h, s, d, generator=g, device=dev).bfloat16() for _ in range(3))
+    m = bias = None
+    seen = torch.ones(s, s, dtype=torch.bool, device=dev)
+    if kind == "add":
+        keep = (torch.rand(1, 1, s, s, generator=g, device=dev) >= 0.1) & seen.tril()
+        keep[..., 0] = True
+        m = torch.zeros(1, 1, s, s, device=dev).masked_fill(~keep, -math.inf).bfloat16()
+        bias = m[0, 0]
+    elif kind == "causal":
+        bias = torch.zeros(s, s, device=dev).masked_fill(~seen.tril(), -math.inf)
+    attend = torch.ops.aten._scaled_dot_product_fused_attention_overrideable
+    causal = kind == "causal"
+    assert _kernel(q, k, v, m, causal) == kernel and _kernel(q[:1], k[:1], v[:1], m, causal) == "general"
+    out = attend(q, k, v, m, 0.0, causal)[0]
+    off = general = 0.0
+    for i in range(b):
+        want, _, _ = _attend(q[i], k[i], v[i], bias, 1 / math.sqrt(d))
+        one = attend(q[i : i + 1], k[i : i + 1], v[i : i + 1], m, 0.0, causal)[0][0]
+        off += (out[i].double() - want).square().sum().item()
+        general += (one.double() - want).square().sum().item()
+    print(f"  tile {off**0.5:.4f} general {general**0.5:.4f} ratio {(off / general) ** 0.5:.4f}", flush=True)
+    assert off <= 1.005**2 * general
