@@ -139,6 +139,13 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
             lse_n = lg[gi_ * p.ls[1] + min(r0 + lane, g.lq - 1) * p.ls[2]];
         }
     };
+    // Before the fragments' loads, whose values are selected from as they come: after them the
+    // first tiles would start a memory round trip later (the whole backward of 8x2/30x30x80 14.4 ->
+    // 13.7 us, 11x6/3x23x128 additive 17.4 -> 16.7).  Not at head dim 64 without a mask, where three
+    // registers spill and 14x16x87/14x64 took 13.6 instead of 13.1.
+    constexpr bool EARLY = VL || MK != MK_NONE;
+    if constexpr (EARLY)
+        if (split < items) request(gi, bi, 0);
     const typename TL::Addr ad = TL::addr(lane);
     v8 kf[DC], vf[VL ? 1 : DC];
     {
@@ -175,22 +182,35 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
         if constexpr (MASKED) {
             const int64_t msz = static_cast<int64_t>(sizeof(MRaw));
             const int64_t b0 = g.mbase + h * p.ms[1] + r0b * g.mrow;
-            const bool fast = g.mrow >= 0 && g.mkey >= 0 && kw0 + 31 < g.lk && r0b + 31 < g.lq &&
-                              (32 * g.mrow + g.lk * g.mkey) * msz < (int64_t{1} << 30) &&
-                              b0 + 31 * g.mrow + (kw0 + 31) * g.mkey < g.mend;
-            if (fast) {
+            const int rlast = min(31, g.lq - 1 - r0b), klast = min(kw0 + 31, g.lk - 1);
+            const bool flat = g.mrow >= 0 && g.mkey >= 0 && (32 * g.mrow + g.lk * g.mkey) * msz < (int64_t{1} << 30) &&
+                              b0 + rlast * g.mrow + klast * g.mkey < g.mend;
+            // (Uniform.)  32-bit offsets from the block's first row; rows past the last and keys
+            // past the last read those (rows in order: the clamp is a minimum of offsets).
+            if (flat) {
                 const auto rs = buffer_rsrc(static_cast<const MRaw*>(p.mask) + b0, 0x7fffffffu);
-                const uint32_t off = static_cast<uint32_t>((4 * h2 * g.mrow + key * g.mkey) * msz);
-                MRaw raw[16];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int so = static_cast<int>((8 * (i / 4) + i % 4) * g.mrow * msz);
+                auto load = [&](uint32_t off, int so) -> MRaw {
                     if constexpr (sizeof(MRaw) == 1)
-                        raw[i] = __builtin_amdgcn_raw_buffer_load_b8(rs, off, so, 0);
+                        return __builtin_amdgcn_raw_buffer_load_b8(rs, off, so, 0);
                     else if constexpr (sizeof(MRaw) == 2)
-                        raw[i] = __builtin_amdgcn_raw_buffer_load_b16(rs, off, so, 0);
+                        return __builtin_amdgcn_raw_buffer_load_b16(rs, off, so, 0);
                     else
-                        raw[i] = __builtin_bit_cast(MRaw, __builtin_amdgcn_raw_buffer_load_b32(rs, off, so, 0));
+                        return __builtin_bit_cast(MRaw, __builtin_amdgcn_raw_buffer_load_b32(rs, off, so, 0));
+                };
+                uint32_t step = static_cast<uint32_t>(g.mrow * msz);
+                __asm__ volatile("" : "+s"(step));  // (else its multiples live across the loop)
+                const uint32_t row = 4 * h2 * step;
+                const uint32_t col = static_cast<uint32_t>(min(key, g.lk - 1)) * static_cast<uint32_t>(g.mkey * msz);
+                MRaw raw[16];
+                if (rlast == 31) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        raw[i] = load(row + col, (8 * (i / 4) + i % 4) * step);
+                } else {
+                    const uint32_t most = rlast * step;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        raw[i] = load(min(row + (8 * (i / 4) + i % 4) * step, most) + col, 0);
                 }
 #pragma unroll
                 for (int i = 0; i < 16; ++i) ml[i] = mask_value_of<MK>(raw[i]);
@@ -316,7 +336,8 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    if (split < items) request(gi, bi, 0);
+    if constexpr (!EARLY)
+        if (split < items) request(gi, bi, 0);
     int buf = 0;
     for (int it = split; it < items; it += p.splits) {
         const int h = kvh * p.group + gi, r0 = (rfirst + bi) * TR;
@@ -437,24 +458,6 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
     const int rr = min(row, vrows - 1);  // rows past the end repeat the last (never written)
     const int pos = rr / G, h = kvh * G + (rr - pos * G);
 
-    v8 qf[DC], of[DC];
-    {
-        const T* qp = static_cast<const T*>(p.q) + g.qb + h * p.qs[1] + static_cast<int64_t>(g.q0 + pos) * p.qs[2];
-        const T* dp = static_cast<const T*>(p.dout) + g.dob + h * p.dos[1] + static_cast<int64_t>(g.q0 + pos) * p.dos[2];
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            qf[c] = frag16<v8>(qp, 0, 0, 1, 16 * c + 8 * h2, p.d);
-            of[c] = frag16<v8>(dp, 0, 0, 1, 16 * c + 8 * h2, p.dval);
-        }
-    }
-    const float nd = p.nd[static_cast<int64_t>(h) * p.rows_total + g.row_base + pos];
-    float l2;
-    bool raw;
-    row_stats(p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + pos) * p.ls[2]], true, l2, raw);
-    f32x16 dq[DB];
-#pragma unroll
-    for (int b = 0; b < DB; ++b) dq[b] = splat16(0.f);
-
     // Causal: keys below lim are visible to this row; those below lim_w to every row of
     // the wavefront, none at or past kend_w to any.
     const int lim = p.causal ? min(g.lk, pos + 1 + g.coff) : g.lk;
@@ -475,6 +478,28 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
         TL::request(kbase, kst, k0, g.lk, p.d * ES, ok, wave, lds0 + buf * 2 * TILE_B);
         TL::request(vbase, vst, k0, g.lk, p.dval * ES, ov, wave, lds0 + (buf * 2 + 1) * TILE_B);
     };
+    const int kstep = p.ksplit * TR;
+    int k0 = ksp * TR;
+    if (k0 < kend) request(k0, 0);  // (before the row's own loads, as in bwd_dkdv)
+
+    v8 qf[DC], of[DC];
+    {
+        const T* qp = static_cast<const T*>(p.q) + g.qb + h * p.qs[1] + static_cast<int64_t>(g.q0 + pos) * p.qs[2];
+        const T* dp = static_cast<const T*>(p.dout) + g.dob + h * p.dos[1] + static_cast<int64_t>(g.q0 + pos) * p.dos[2];
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            qf[c] = frag16<v8>(qp, 0, 0, 1, 16 * c + 8 * h2, p.d);
+            of[c] = frag16<v8>(dp, 0, 0, 1, 16 * c + 8 * h2, p.dval);
+        }
+    }
+    const float nd = p.nd[static_cast<int64_t>(h) * p.rows_total + g.row_base + pos];
+    float l2;
+    bool raw;
+    row_stats(p.lse[g.lb + h * p.ls[1] + static_cast<int64_t>(g.q0 + pos) * p.ls[2]], true, l2, raw);
+    f32x16 dq[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b) dq[b] = splat16(0.f);
+
     const typename TL::Addr ad = TL::addr(lane);
     typedef typename MaskRaw<MK>::type MRaw;
     constexpr bool MASKED = MK != MK_NONE;
@@ -497,9 +522,15 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
 #pragma unroll
                 for (int i = 0; i < 16; ++i) ml[i] = mask_value_of<MK>(x[i / 4].e[i % 4]);
             } else {
+                // Keys past the last read the last; a packed mask's end as in mask_at, but as a
+                // clamped load and a select (a branch around each load would make it wait for the
+                // one before).
 #pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    ml[i] = mask_at<MK>(p, g, h, pos, min(kb0 + 8 * (i / 4) + 4 * h2 + i % 4, g.lk - 1));
+                for (int i = 0; i < 16; ++i) {
+                    const int64_t at = moff + min(kb0 + 8 * (i / 4) + 4 * h2 + i % 4, g.lk - 1) * g.mkey;
+                    const float x = mask_logit_of<MK>(static_cast<const MRaw*>(p.mask)[min(at, g.mend - 1)]);
+                    ml[i] = at < g.mend ? x : kMaskedLogit;
+                }
             }
             if (__builtin_amdgcn_ballot_w64(raw)) {
 #pragma unroll
@@ -558,9 +589,6 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    const int kstep = p.ksplit * TR;
-    int k0 = ksp * TR;
-    if (k0 < kend) request(k0, 0);
     int buf = 0;
     for (; k0 < kend; k0 += kstep) {
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (as in bwd_dkdv)

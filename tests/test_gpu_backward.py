@@ -546,3 +546,50 @@ def test_backward_in_a_workspace_of_the_plans_size(native, dev, b, hq, hk, s, d)
     assert (work[n.value :] == 0xAB).all()
     for got, t in zip(grads, ts):
         assert torch.equal(got, t.grad)
+
+
+def _close_to_float64(got, want, dtype, what):
+    """P, dS, out and the gradient itself round to the type, O in the row dot too: five half ulps
+    of what the gradient's size is made of, in the mean over a tensor."""
+    half_ulp = 2.0**-9 if dtype == torch.bfloat16 else 2.0**-12
+    off = ((got.cpu().double() - want).norm() / want.norm()).item()
+    print(f"  {what} {off:.2e}", flush=True)
+    assert torch.isfinite(got).all() and off <= 5 * half_ulp, (what, off)
+
+
+@pytest.mark.parametrize("layout", ["rows", "keys first", "every second key", "per batch", "per head"])
+@pytest.mark.parametrize("kind", ["bool", "additive", "float32"])
+@pytest.mark.parametrize("b,h,sq,sk,d", [(2, 3, 22, 22, 72), (2, 2, 33, 65, 64), (3, 2, 70, 90, 128), (2, 2, 40, 31, 32)])
+def test_masked_blocks_at_the_edges(native, dev, b, h, sq, sk, d, kind, layout):
+    """Masks in every stride order over row and key counts off the 32x32 blocks."""
+    print(f"mask edges {b}x{h}x{sq}/{sk}x{d} {kind} {layout}", flush=True)
+    g = C.gen(sq + d + len(layout))
+    dtype = torch.bfloat16
+    q, go = (C.randn(g, b, h, sq, d) for _ in range(2))
+    k, v = (C.randn(g, b, h, sk, d) for _ in range(2))
+    lead = {"per batch": (b, 1), "per head": (1, h)}.get(layout, (1, 1))
+    mask = torch.randn(*lead, sq, sk, generator=g)
+    if kind == "additive":
+        mask = mask.to(dtype)
+    hidden = torch.rand(*lead, sq, sk, generator=g) < 0.3
+    hidden[..., 0] = False
+    mask = ~hidden if kind == "bool" else mask.masked_fill(hidden, -torch.inf)
+    if layout == "keys first":
+        placed = mask.transpose(-1, -2).contiguous().to(dev).transpose(-1, -2)
+    elif layout == "every second key":
+        placed = torch.zeros(*lead, sq, 2 * sk, dtype=mask.dtype, device=dev)[..., ::2]
+        placed.copy_(mask)
+    elif layout == "per batch":
+        placed = mask[:, :, :1].to(dev).expand(-1, -1, sq, -1)  # one row of keys for every row
+        mask = mask[:, :, :1].expand(-1, -1, sq, -1)
+    else:
+        placed = mask.to(dev)
+    ts = [t.to(dev).requires_grad_() for t in (q, k, v)]
+    native.reset_counters()
+    F.scaled_dot_product_attention(*ts, attn_mask=placed).backward(go.to(dev))
+    assert native.counters()["attention_backward"] == 1
+    rs = [t.double().requires_grad_() for t in (q, k, v)]
+    bias = torch.zeros(mask.shape, dtype=torch.float64).masked_fill(~mask, -torch.inf) if kind == "bool" else mask.double()
+    (torch.softmax(rs[0] @ rs[1].transpose(-1, -2) / d**0.5 + bias, -1) @ rs[2]).backward(go.double())
+    for name, a, r in zip(("dq", "dk", "dv"), ts, rs):
+        _close_to_float64(a.grad, r.grad, dtype, name)
