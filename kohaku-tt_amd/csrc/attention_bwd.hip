@@ -836,7 +836,11 @@ struct BwdPlan {
 // they leave one workgroup per CU, only for calls that give no CU two: 2x12x251x128 causal
 // 19 against 26, 1x8x100x128 15 against 18; but 32x14/2x80x128 46 against 34.  64-row dQ
 // workgroups only where 128 rows leave CUs idle (4x16x1024x64, 512 workgroups: 95 against
-// 83; 1x14/2x2048x64, 224 workgroups: 54 against 57).
+// 83; 1x14/2x2048x64, 224 workgroups: 54 against 57).  Those past 64 split only until both
+// passes' workgroups take every CU once (splits for two per CU / as here, attn_bwd_grads):
+// 1x8x1024x128 57 / 32, 56; 2x8/2x463x128 37.5 / 29.0, 33.6 (additive mask 49.7 / 36.7, 48.6);
+// 1x16/8x600x80 44.8 / 34.7, 39.9; 3x4/1 x 1000 rows x 200 keys x 80 29.6 / 28.1, 28.3 (masked
+// 38.4 / 39.1, 38.3).
 constexpr int64_t kTileItems = 72;
 constexpr int64_t kTileMaxWgs = 2048;
 constexpr int64_t kTileFewWgs = 256;
@@ -868,8 +872,12 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     if (bwd_ksplit_override() > 0)
         pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
     pl.grid.tiles_q = static_cast<int>(ceil_div(a->seq_q * G, pl.grid.half_q ? 64 : 128));
-    pl.grid.nk = static_cast<int>(nk * pl.splits);
     pl.grid.nq = static_cast<int>(units * pl.grid.tiles_q * pl.ksplit);
+    // (64-key workgroups past head dim 64: one per CU, both passes' in one round.)
+    if (pl.grid.half_k && dp > 64)
+        pl.splits = static_cast<int>(std::min<int64_t>(
+            pl.splits, std::max<int64_t>(1, (kTileFewWgs - pl.grid.nq + nk / 2) / nk)));
+    pl.grid.nk = static_cast<int>(nk * pl.splits);
     return pl;
 }
 
