@@ -231,6 +231,10 @@ int kmi_attn_bwd_plan_bytes(const kmi_attn_bwd_args* args, size_t* bytes);
  * to five times as much (1 x 24 heads x 4396 x 128: 1027 MB against 216 MB). */
 int kmi_attn_bwd_workspace_bytes(const kmi_attn_bwd_args* args, size_t* bytes);
 
+/* The kernel that forms the gradients of `args`, a static string: "tile" (attn_bwd_tile_kernel)
+ * or "general" (attn_bwd_grads).  For tests and profiles. */
+int kmi_attn_bwd_kernel(const kmi_attn_bwd_args* args, const char** name);
+
 /* Enqueues the attention backward of `args` on `stream` (hipStream_t). */
 int kmi_attn_bwd(const kmi_attn_bwd_args* args, void* workspace, size_t workspace_bytes,
                  void* stream);

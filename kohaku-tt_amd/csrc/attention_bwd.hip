@@ -23,8 +23,8 @@
 //                    together with the key-split dQ partials
 //
 // Head dims padded to 128 or less run the gradients on attn_bwd_tile_kernel
-// (attention_bwd_tile.hpp, 32x32x16 MFMAs); wider ones on attn_bwd_grads here (16x16x32
-// MFMAs: 32 keys' dK and dV at 256 do not fit the tile kernel's registers).
+// (attention_bwd_tile.hpp, 32x32x16 MFMAs); wider ones (32 keys' dK and dV at 256 do not fit
+// its registers) and the calls of small_call on attn_bwd_grads here (16x16x32 MFMAs).
 //
 // Probabilities follow the forward exactly: keys past the causal limit or masked
 // (logit <= -5e5) get P = 0; a row whose lse carries the -5e5 offset of a fully-masked
@@ -660,10 +660,14 @@ __device__ __forceinline__ void attn_bwd_dq(const BwdParams& p, const int bid) {
 // neither reads the other's output), their workgroups interleaved in proportion (block b
 // is dQ workgroup floor(b n_dq / n) when that count steps at b, else a dK / dV workgroup),
 // so that the two kinds share every CU from the start.
-// At these head dims the accumulators alone take a wavefront per SIMD's registers: one
-// workgroup per CU.
+// Workgroups per CU (the register budget it compiles to, without spills); past head dim 128
+// the accumulators alone take a wavefront per SIMD's registers.
+constexpr int bwd_min_blocks(int dp, bool plain) {
+    return dp <= 64 ? (plain ? 4 : 3) : (dp <= 128 ? (plain ? 3 : 2) : 1);
+}
+
 template <typename T, int DP, int MK, bool DV>
-__global__ __launch_bounds__(BWD_THREADS, 1) void attn_bwd_grads(
+__global__ __launch_bounds__(BWD_THREADS, bwd_min_blocks(DP, MK == MK_NONE && !DV)) void attn_bwd_grads(
     const BwdParams p, const int kv_blocks, const int dq_blocks) {
     const int64_t b = blockIdx.x, n = static_cast<int64_t>(kv_blocks) + dq_blocks;
     const int q0 = static_cast<int>(b * dq_blocks / n), q1 = static_cast<int>((b + 1) * dq_blocks / n);
@@ -769,8 +773,8 @@ const char* check_bwd(const kmi_attn_bwd_args* a) {
 int64_t rows_total_of(const kmi_attn_bwd_args* a) { return a->cu_seqlens_q ? a->total_q : a->batch * a->seq_q; }
 int64_t keys_total_of(const kmi_attn_bwd_args* a) { return a->cu_seqlens_q ? a->total_k : a->batch * a->seq_k; }
 
-// Split rules of attn_bwd_grads (head dims padded past 128; the others' workspace figure
-// too, see bwd_ws_bytes): a dK / dV workgroup takes at most kBwdItemsPerWg64 (query head,
+// Split rules of attn_bwd_grads (head dims padded past 128 and small calls; the others'
+// workspace figure too, see bwd_ws_bytes): a dK / dV workgroup takes at most kBwdItemsPerWg64 (query head,
 // 32-row block) items up to head dim 64 and kBwdItemsPerWg128 at 128 (in proportion fewer
 // past it), a dQ workgroup at most kBwdTilesPerWg 32-key tiles; below kBwdMinWgs workgroups
 // of a kind, splits go down to kBwdMinItems items (or tiles) each.
@@ -814,7 +818,7 @@ void grads_splits(const kmi_attn_bwd_args* a, int& splits, int& ksplit) {
 }
 
 struct BwdPlan {
-    bool tile;  // attn_bwd_tile_kernel (padded head dims up to 128), else attn_bwd_grads
+    bool tile;  // attn_bwd_tile_kernel, else attn_bwd_grads
     int splits, ksplit;
     BwdGrid grid;
 };
@@ -846,11 +850,29 @@ constexpr int64_t kTileMaxWgs = 2048;
 constexpr int64_t kTileFewWgs = 256;
 constexpr int64_t kTileMinItems = 7;
 
+// Whether a call of head dims padded to 128 or less runs on attn_bwd_grads: with at most 32 rows
+// per query head and one 64-key tile a workgroup of either kernel is one chain of loads, products
+// and stores, and attn_bwd_grads' is shorter (its four wavefronts share a 32x32 block that takes
+// one wavefront of the tile kernel).  Measured (us of the whole backward, attn_bwd_grads / tile):
+//   no mask: 1x8x20x32 7.0 / 8.0, 1x8x20x64 7.8 / 9.3, 8x14/2x22x64 14.0 / 16.7, 64x16 x 17 rows x
+//     50 keys x 64 21.5 / 26.0 (64x12/2x32x64 17.5 / 17.0), 1x8x20x128 10.0 / 11.1, 4x12 x 32 rows
+//     x 64 keys x 128 10.5 / 11.9; past 64 (batch, query head) pairs the tile kernel leads there
+//     (64x12/2x32x80 23.4 / 17.1, 32x16/8x24x128 15.6 / 13.6)
+//   masked: 8x14/2x22x64 22 / 24, 1x8x20x64 9.5 / 11.2; head dim 32 4x12 x 32 rows x 64 keys 10.6 /
+//     9.4, 80 2x14/2x32 25.3 / 23.5, 128 28.6 / 25.1
+//   more rows: 4x16/4x50x64 14.9 / 13.0, 16x16x64x64 11.4 / 11.7; more keys: 24 rows x 130 keys x
+//     64, 32x24 37.5 / 37.3, 16x14/2x24x130x128 22 / 20
+// (By the query heads, not the K/V heads: see dQ in bwd_plan.)
+bool small_call(const kmi_attn_bwd_args* a, int64_t dp) {
+    if (a->seq_q > 32 || a->seq_k > 64) return false;
+    return dp == 64 || (a->mask_mode == KMI_MASK_NONE && (dp == 32 || a->batch * a->heads_q <= 64));
+}
+
 BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     BwdPlan pl{};
     const int64_t dp = padded_head_dim(std::max(a->head_dim, bwd_value_dim(a)));
     const int64_t units = a->batch * a->heads_kv, G = a->heads_q / a->heads_kv;
-    pl.tile = dp <= 128;
+    pl.tile = dp <= 128 && !small_call(a, dp);
     if (!pl.tile) {
         grads_splits(a, pl.splits, pl.ksplit);
         return pl;
@@ -914,7 +936,7 @@ size_t bwd_ws_bytes(const kmi_attn_bwd_args* a) {
     return std::max(bwd_plan_bytes(a), layout_bytes(bwd_layout(a, splits, ksplit)));
 }
 
-// The gradient kernel of head dims padded past 128.
+// attn_bwd_grads' launch.
 template <typename T, int DP, int MK>
 hipError_t launch_grads(const BwdParams& p, hipStream_t s) {
     const int64_t ntk = ceil_div(p.seq_k, KW), nqb = ceil_div(p.seq_q, QW);
@@ -941,6 +963,15 @@ hipError_t launch_grads_mask(const BwdParams& p, int mk, hipStream_t s) {
     }
 }
 
+// The calls that small_call sends here (masks at head dim 64 only).
+template <typename T, int DP>
+hipError_t launch_grads_small(const BwdParams& p, int mk, hipStream_t s) {
+    if constexpr (DP == 64)
+        return launch_grads_mask<T, DP>(p, mk, s);
+    else
+        return mk == MK_NONE ? launch_grads<T, DP, MK_NONE>(p, s) : hipErrorInvalidValue;
+}
+
 // The call's launches: row dots, gradients, split sums.
 template <typename T, int DP>
 hipError_t launch_bwd(const BwdParams& p, const BwdPlan& pl, int mk, hipStream_t s) {
@@ -952,7 +983,7 @@ hipError_t launch_bwd(const BwdParams& p, const BwdPlan& pl, int mk, hipStream_t
         hipLaunchKernelGGL((attn_bwd_rowdot<T, DP, false>), grd, dim3(BWD_THREADS), 0, s, p);
     hipError_t err;
     if constexpr (DP <= 128)
-        err = launch_tile<T, DP>(p, pl.grid, mk, s);
+        err = pl.tile ? launch_tile<T, DP>(p, pl.grid, mk, s) : launch_grads_small<T, DP>(p, mk, s);
     else
         err = launch_grads_mask<T, DP>(p, mk, s);
     if (err != hipSuccess) return err;
@@ -996,6 +1027,15 @@ extern "C" int kmi_attn_bwd_plan_bytes(const kmi_attn_bwd_args* a, size_t* bytes
     if (!bytes) return fail(KMI_EINVAL, "kmi_attn_bwd_plan_bytes: null bytes");
     if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd_plan_bytes: ") + why);
     *bytes = bwd_plan_bytes(a);
+    return KMI_OK;
+}
+
+extern "C" int kmi_attn_bwd_kernel(const kmi_attn_bwd_args* a, const char** name) {
+    using namespace kmi;
+    using namespace kmi::bwd;
+    if (!name) return fail(KMI_EINVAL, "kmi_attn_bwd_kernel: null name");
+    if (const char* why = check_bwd(a)) return fail(KMI_EINVAL, std::string("kmi_attn_bwd_kernel: ") + why);
+    *name = bwd_plan(a).tile ? "tile" : "general";
     return KMI_OK;
 }
 

@@ -24,6 +24,7 @@ EXPORTS = (
     "kmi_attn_fwd_noalloc",
     "kmi_attn_bwd_plan_bytes",
     "kmi_attn_bwd_workspace_bytes",
+    "kmi_attn_bwd_kernel",
     "kmi_attn_bwd",
     "kmi_layer_norm_fwd",
     "kmi_rms_norm_fwd",
@@ -147,6 +148,7 @@ def lib():
         h.kmi_attn_fwd_noalloc.argtypes = [ctypes.POINTER(AttnArgs), vp]
         h.kmi_attn_bwd_plan_bytes.argtypes = [ctypes.POINTER(AttnBwdArgs), ctypes.POINTER(ctypes.c_size_t)]
         h.kmi_attn_bwd_workspace_bytes.argtypes = [ctypes.POINTER(AttnBwdArgs), ctypes.POINTER(ctypes.c_size_t)]
+        h.kmi_attn_bwd_kernel.argtypes = [ctypes.POINTER(AttnBwdArgs), ctypes.POINTER(ctypes.c_char_p)]
         h.kmi_attn_bwd.argtypes = [ctypes.POINTER(AttnBwdArgs), vp, ctypes.c_size_t, vp]
         h.kmi_layer_norm_fwd.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i32, i32, i32, ctypes.c_double, vp]
         h.kmi_rms_norm_fwd.argtypes = [vp, vp, vp, vp, vp, i64, i64, i32, i32, i32, ctypes.c_double, vp]

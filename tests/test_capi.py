@@ -245,6 +245,34 @@ def test_backward_takes_what_its_plan_needs(sizes, floats):
     assert "kmi_attn_bwd_plan_bytes" in lib.kmi_last_error().decode()
 
 
+@pytest.mark.parametrize(
+    "sizes,masked,kernel",
+    [
+        # (batch, heads_q, heads_kv, seq_q, seq_k, head_dim): the lines of small_call
+        ((4, 14, 2, 32, 64, 64), False, "general"),
+        ((64, 16, 16, 32, 64, 40), True, "general"),
+        ((4, 14, 2, 33, 64, 64), False, "tile"),
+        ((4, 14, 2, 32, 65, 64), False, "tile"),
+        ((1, 2, 2, 1, 1, 32), False, "general"),
+        ((1, 2, 2, 1, 1, 32), True, "tile"),
+        ((4, 16, 4, 32, 64, 128), False, "general"),
+        ((4, 16, 4, 32, 64, 72), True, "tile"),
+        ((5, 13, 1, 32, 64, 128), False, "tile"),
+        ((1, 2, 2, 1000, 1000, 136), False, "general"),
+    ],
+)  # fmt: skip
+def test_backward_kernel_by_size(sizes, masked, kernel):
+    lib, a, name = capi.lib(), capi.AttnBwdArgs(), ctypes.c_char_p()
+    a.q = a.k = a.v = a.out = a.grad_out = a.lse = a.grad_q = a.grad_k = a.grad_v = 0x1000
+    a.dtype = capi.KMI_BF16
+    a.batch, a.heads_q, a.heads_kv, a.seq_q, a.seq_k, a.head_dim = sizes
+    if masked:
+        a.mask, a.mask_mode, a.mask_dtype = 0x1000, capi.KMI_MASK_STRIDED, capi.KMI_BOOL
+    assert lib.kmi_attn_bwd_kernel(ctypes.byref(a), ctypes.byref(name)) == capi.KMI_OK
+    assert name.value.decode() == kernel
+    assert lib.kmi_attn_bwd_kernel(ctypes.byref(a), None) == capi.KMI_EINVAL
+
+
 def test_rms_norm_backward_rejects_malformed_calls_before_launch():
     lib = capi.lib()
     n = ctypes.c_size_t()
