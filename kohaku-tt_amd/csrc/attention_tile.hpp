@@ -376,6 +376,29 @@ __device__ __forceinline__ void attn_tile(const AttnParams& p, unsigned char* sm
                 for (int n = 0; n < NB; ++n)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) __builtin_memcpy(&x[n][4 * q], src + 32 * n + 8 * q, 4 * sizeof(MRaw));
+            } else if (mvec && lk >= 4) {
+                // The last, partial tile: four keys per load that end with the last key at most,
+                // shifted into place (whatever lies past the last key is not seen).  Key by key
+                // its 16 or 32 loads and their addresses cost more than a whole tile.
+                const MRaw* src = mp + mrow;
+#pragma unroll
+                for (int n = 0; n < NB; ++n)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int k = key0 + 32 * n + 8 * q, from = min(k, lk - 4), by = min(k - from, 3);
+                        if constexpr (sizeof(MRaw) == 4) {
+                            MRaw e[4];
+                            __builtin_memcpy(e, src + from, sizeof(e));
+                            if (by & 1) e[0] = e[1], e[1] = e[2], e[2] = e[3];
+                            if (by & 2) e[0] = e[2], e[1] = e[3];
+                            __builtin_memcpy(&x[n][4 * q], e, sizeof(e));
+                        } else {
+                            typename std::conditional<sizeof(MRaw) == 2, uint64_t, uint32_t>::type e;
+                            __builtin_memcpy(&e, src + from, sizeof(e));
+                            e >>= 8 * static_cast<int>(sizeof(MRaw)) * by;
+                            __builtin_memcpy(&x[n][4 * q], &e, sizeof(e));
+                        }
+                    }
             } else {
 #pragma unroll
                 for (int n = 0; n < NB; ++n)

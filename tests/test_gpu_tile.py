@@ -137,8 +137,13 @@ ROUTED = [
     (32, 16, 16, 31, 300, 256, False, "f32", BF, "tile64"),
 ]  # fmt: skip
 
+# Masked calls whose last key tile is partial: fewer than four keys, and every remainder of four.
+PARTIAL = [(6, 16, 16, 128, sk, d, False, kind, BF, "tile64")
+           for sk in (3, 4, 5, 31, 66, 127, 129, 190) for d in (64, 128) for kind in ("bool", "add", "f32", "pad")]  # fmt: skip
+PARTIAL += [(28, 16, 16, 70, sk, 64, False, kind, HF, "tile128") for sk in (5, 66, 191) for kind in ("bool", "add", "f32", "pad")]
 
-@pytest.mark.parametrize("case", CASES + ROUTED, ids=lambda c: "x".join(map(str, c)))
+
+@pytest.mark.parametrize("case", CASES + ROUTED + PARTIAL, ids=lambda c: "x".join(map(str, c)))
 def test_dense_calls_meet_float64(native, dev, case):
     b, hq, hk, sq, sk, d, causal, mask, dtype = case[:9]
     print(f"tile {case}", flush=True)
