@@ -844,7 +844,11 @@ struct BwdPlan {
 // passes' workgroups take every CU once (splits for two per CU / as here, attn_bwd_grads):
 // 1x8x1024x128 57 / 32, 56; 2x8/2x463x128 37.5 / 29.0, 33.6 (additive mask 49.7 / 36.7, 48.6);
 // 1x16/8x600x80 44.8 / 34.7, 39.9; 3x4/1 x 1000 rows x 200 keys x 80 29.6 / 28.1, 28.3 (masked
-// 38.4 / 39.1, 38.3).
+// 38.4 / 39.1, 38.3).  A few workgroups over 256 cost less than a split fewer (261 of them there),
+// many a round (1x10x609x128, 300: 40.2 against 25.6).  Fewer than 32 64-key workgroups with six
+// 64-row items or more take two items each, since the chain of items is all there is (one split /
+// as here, attn_bwd_grads): 5x4/1 x 78 rows x 16 keys x 64 17.9 / 13.9, 15.1; 1x16/8x154x64
+// additive 23.5 / 17.7, 21.2; 1x14/2x128x128 23.1 / 20.3; not from 32 on (1x4x500x64 16.4 / 17.9).
 constexpr int64_t kTileItems = 72;
 constexpr int64_t kTileMaxWgs = 2048;
 constexpr int64_t kTileFewWgs = 256;
@@ -855,17 +859,17 @@ constexpr int64_t kTileMinItems = 7;
 // and stores, and attn_bwd_grads' is shorter (its four wavefronts share a 32x32 block that takes
 // one wavefront of the tile kernel).  Measured (us of the whole backward, attn_bwd_grads / tile):
 //   no mask: 1x8x20x32 7.0 / 8.0, 1x8x20x64 7.8 / 9.3, 8x14/2x22x64 14.0 / 16.7, 64x16 x 17 rows x
-//     50 keys x 64 21.5 / 26.0 (64x12/2x32x64 17.5 / 17.0), 1x8x20x128 10.0 / 11.1, 4x12 x 32 rows
-//     x 64 keys x 128 10.5 / 11.9; past 64 (batch, query head) pairs the tile kernel leads there
-//     (64x12/2x32x80 23.4 / 17.1, 32x16/8x24x128 15.6 / 13.6)
+//     50 keys x 64 21.5 / 26.0 (64x12/2x32x64 17.5 / 17.0), 1x8x20x128 10.0 / 11.1, 4x24x22x128
+//     10.4 / 11.5, 5x32/8x20x128 14.5 / 15.3; past 160 (batch, query head) pairs the tile kernel
+//     leads there with GQA (64x12/2x32x80 23.4 / 17.1, 32x16/8x24x128 15.6 / 13.6)
 //   masked: 8x14/2x22x64 22 / 24, 1x8x20x64 9.5 / 11.2; head dim 32 4x12 x 32 rows x 64 keys 10.6 /
-//     9.4, 80 2x14/2x32 25.3 / 23.5, 128 28.6 / 25.1
+//     9.4, 80 2x14/2x32 25.3 / 23.5, 128 28.6 / 25.1 (but 4x24x22x128 12.3 / 13.9)
 //   more rows: 4x16/4x50x64 14.9 / 13.0, 16x16x64x64 11.4 / 11.7; more keys: 24 rows x 130 keys x
 //     64, 32x24 37.5 / 37.3, 16x14/2x24x130x128 22 / 20
 // (By the query heads, not the K/V heads: see dQ in bwd_plan.)
 bool small_call(const kmi_attn_bwd_args* a, int64_t dp) {
     if (a->seq_q > 32 || a->seq_k > 64) return false;
-    return dp == 64 || (a->mask_mode == KMI_MASK_NONE && (dp == 32 || a->batch * a->heads_q <= 64));
+    return dp == 64 || (a->mask_mode == KMI_MASK_NONE && (dp == 32 || a->batch * a->heads_q <= 160));
 }
 
 BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
@@ -890,7 +894,9 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     const int64_t work = G * ceil_div(a->seq_q, 32);
     const int64_t by_work = std::min(ceil_div(work, kTileItems), ceil_div(kTileMaxWgs, nk));
     const int64_t by_fill = nk < kTileFewWgs ? std::min(ceil_div(2 * kTileFewWgs, nk), work / kTileMinItems) : 1;
-    pl.splits = static_cast<int>(std::max<int64_t>(1, std::min(std::max(by_work, by_fill), kBwdMaxSplits)));
+    const int64_t by_few =
+        pl.grid.half_k && nk < 32 && G * ceil_div(a->seq_q, 64) >= 6 ? std::min(G * ceil_div(a->seq_q, 64) / 2, kTileFewWgs / 2 / nk) : 1;
+    pl.splits = static_cast<int>(std::max<int64_t>(1, std::min(std::max({by_work, by_fill, by_few}), kBwdMaxSplits)));
     if (bwd_ksplit_override() > 0)
         pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
     pl.grid.tiles_q = static_cast<int>(ceil_div(a->seq_q * G, pl.grid.half_q ? 64 : 128));
@@ -898,7 +904,7 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     // (64-key workgroups past head dim 64: one per CU, both passes' in one round.)
     if (pl.grid.half_k && dp > 64)
         pl.splits = static_cast<int>(std::min<int64_t>(
-            pl.splits, std::max<int64_t>(1, (kTileFewWgs - pl.grid.nq + nk / 2) / nk)));
+            pl.splits, std::max<int64_t>(1, (kTileFewWgs + 8 - pl.grid.nq) / nk)));
     pl.grid.nk = static_cast<int>(nk * pl.splits);
     return pl;
 }

@@ -227,6 +227,10 @@ def test_backward_rejects_malformed_calls_before_launch():
         ((1, 24, 24, 4396, 4396, 128), 24 * 4396 + 2 * (24 * 2 * 4396 * 128)),
         # 64-key workgroups at one per CU: 128 and 128 dQ ones fill the chip, so no split
         ((1, 8, 8, 1024, 1024, 128), 8 * 1024),
+        # 100 beside 100 of them: no second round for a split
+        ((1, 10, 10, 609, 609, 72), 10 * 609),
+        # five with eight 64-row items: four splits of two
+        ((5, 4, 1, 78, 16, 64), 4 * 5 * 78 + 2 * (4 * 5 * 16 * 64)),
         # 32 beside 116 dQ ones: four splits
         ((2, 8, 2, 463, 463, 80), 8 * 2 * 463 + 2 * (2 * 4 * 2 * 463 * 96)),
         # past head dim 128 the bound and the plan are one: 48 of two items
@@ -257,7 +261,8 @@ def test_backward_takes_what_its_plan_needs(sizes, floats):
         ((1, 2, 2, 1, 1, 32), True, "tile"),
         ((4, 16, 4, 32, 64, 128), False, "general"),
         ((4, 16, 4, 32, 64, 72), True, "tile"),
-        ((5, 13, 1, 32, 64, 128), False, "tile"),
+        ((5, 32, 8, 32, 64, 128), False, "general"),
+        ((12, 14, 2, 32, 64, 128), False, "tile"),
         ((1, 2, 2, 1000, 1000, 136), False, "general"),
     ],
 )  # fmt: skip
