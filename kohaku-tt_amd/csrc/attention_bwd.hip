@@ -836,23 +836,28 @@ struct BwdPlan {
 //   1x14/2x2048x64 causal (64, 448): 8* 54, 10 52, 12 55
 //   4x12x512x64 causal (384, 16): 1* 22, 2 33
 // 64-key dK / dV workgroups (two wavefronts per 32 keys) at padded head dims up to 64:
-// 4x16x1024x64 83 against 93 with 128 keys, 3x32/8x1718x40 295 against 309.  Past 64, where
-// they leave one workgroup per CU, only for calls that give no CU two: 2x12x251x128 causal
-// 19 against 26, 1x8x100x128 15 against 18; but 32x14/2x80x128 46 against 34.  64-row dQ
-// workgroups only where 128 rows leave CUs idle (4x16x1024x64, 512 workgroups: 95 against
-// 83; 1x14/2x2048x64, 224 workgroups: 54 against 57).  Those past 64 split only until both
-// passes' workgroups take every CU once (splits for two per CU / as here, attn_bwd_grads):
-// 1x8x1024x128 57 / 32, 56; 2x8/2x463x128 37.5 / 29.0, 33.6 (additive mask 49.7 / 36.7, 48.6);
-// 1x16/8x600x80 44.8 / 34.7, 39.9; 3x4/1 x 1000 rows x 200 keys x 80 29.6 / 28.1, 28.3 (masked
-// 38.4 / 39.1, 38.3).  A few workgroups over 256 cost less than a split fewer (261 of them there),
-// many a round (1x10x609x128, 300: 40.2 against 25.6).  Fewer than 32 64-key workgroups with six
-// 64-row items or more take two items each, since the chain of items is all there is (one split /
-// as here, attn_bwd_grads): 5x4/1 x 78 rows x 16 keys x 64 17.9 / 13.9, 15.1; 1x16/8x154x64
-// additive 23.5 / 17.7, 21.2; 1x14/2x128x128 23.1 / 20.3; not from 32 on (1x4x500x64 16.4 / 17.9).
+// 4x16x1024x64 83 against 93 with 128 keys, 3x32/8x1718x40 295 against 309.  Past 64 they leave
+// one workgroup per CU: only where their splits and the dQ workgroups make one round (a few over
+// 256 cost less than a split fewer) of at most kTileHalfItems 64-row items each.  (128 keys / 64
+// at two rounds / as here, attn_bwd_grads): 1x8x1024x128 - / 57 / 32, 56; 2x8/2x463x128 33 / 38 /
+// 29, 34; 16x4/2 x 190 rows x 250 keys x 80 29 / 24 / 17, 26; 18x8/2x106x80 28 / 25 / 19, 25; but
+// 1x16/8x600x80 (20 items) 32 / 45 / 35, 40; 1x16/2x1500x80 (376 items) 225 with one split.
+// Fewer than 64 64-key workgroups with six items or more split to two (from 32 on four) each, as
+// the chain of items is all there is (one split / as here, attn_bwd_grads): 5x4/1 x 78 rows x 16
+// keys x 64 17.9 / 13.9, 15.1; 1x16/8x154x64 additive 23.5 / 17.7, 21.2; 1x14/2x128x128 23.1 / 20.3;
+// but 1x4x500x64 16.4 / 17.9 with two each.
+// 64-row dQ workgroups (two wavefronts share a row's keys) only where 128 rows leave CUs idle
+// (4x16x1024x64, 512 workgroups: 95 against 83; 1x14/2x2048x64, 224 workgroups: 54 against 57);
+// past head dim 64, with few keys to share, only up to kTileHalfRows of them (8x12x256x80, 384:
+// 29.6 against 24.7; 19x6/3 x 168 rows x 97 keys x 80, 342: 27.0 against 21.9; 3x4/1 x 1000 rows
+// x 200 keys x 128, 192: 31.1 against 36.8).
 constexpr int64_t kTileItems = 72;
 constexpr int64_t kTileMaxWgs = 2048;
 constexpr int64_t kTileFewWgs = 256;
 constexpr int64_t kTileMinItems = 7;
+constexpr int64_t kTileHalfRows = 192;
+constexpr int64_t kTileHalfKeys = 320;
+constexpr int64_t kTileHalfItems = 16;
 
 // Whether a call of head dims padded to 128 or less runs on attn_bwd_grads: with at most 32 rows
 // per query head and one 64-key tile a workgroup of either kernel is one chain of loads, products
@@ -884,27 +889,29 @@ BwdPlan bwd_plan(const kmi_attn_bwd_args* a) {
     // dQ: by the query heads (a call with K / V repeated per query head splits alike, so its
     // dQ is the same bit for bit).
     const int64_t nq = a->batch * a->heads_q * ceil_div(a->seq_q, 128), tiles = ceil_div(a->seq_k, 64);
-    pl.grid.half_q = nq < kTileFewWgs;
-    const int64_t nqw = pl.grid.half_q ? a->batch * a->heads_q * ceil_div(a->seq_q, 64) : nq;
+    const int64_t nq64 = a->batch * a->heads_q * ceil_div(a->seq_q, 64);
+    pl.grid.half_q = nq < kTileFewWgs && (dp <= 64 || nq64 <= kTileHalfRows || a->seq_k > kTileHalfKeys);
+    const int64_t nqw = pl.grid.half_q ? nq64 : nq;
     pl.ksplit = static_cast<int>(std::max<int64_t>(
         1, std::min<int64_t>({ceil_div(kTileFewWgs, 2 * nqw), tiles / 8, kBwdMaxKsplit})));
     const int64_t nk64 = units * ceil_div(a->seq_k, 64);
-    pl.grid.half_k = dp <= 64 || nk64 + nqw <= kTileFewWgs;
+    pl.grid.tiles_q = static_cast<int>(ceil_div(a->seq_q * G, pl.grid.half_q ? 64 : 128));
+    // (Room: splits of 64-key workgroups at one per CU beside the dQ workgroups.)
+    const int64_t rows64 = G * ceil_div(a->seq_q, 64);  // a 64-key workgroup's items, unsplit
+    const int64_t room = (kTileFewWgs + 8 - units * pl.grid.tiles_q * pl.ksplit) / nk64;
+    pl.grid.half_k = dp <= 64 || (room > 0 && rows64 <= kTileHalfItems * room);
     const int64_t nk = pl.grid.half_k ? nk64 : units * ceil_div(a->seq_k, 128);
     const int64_t work = G * ceil_div(a->seq_q, 32);
     const int64_t by_work = std::min(ceil_div(work, kTileItems), ceil_div(kTileMaxWgs, nk));
     const int64_t by_fill = nk < kTileFewWgs ? std::min(ceil_div(2 * kTileFewWgs, nk), work / kTileMinItems) : 1;
-    const int64_t by_few =
-        pl.grid.half_k && nk < 32 && G * ceil_div(a->seq_q, 64) >= 6 ? std::min(G * ceil_div(a->seq_q, 64) / 2, kTileFewWgs / 2 / nk) : 1;
+    const int64_t by_few = pl.grid.half_k && nk <= kTileFewWgs / 4 && rows64 >= 6
+                               ? std::min(rows64 / (nk < kTileFewWgs / 8 ? 2 : 4), kTileFewWgs / 2 / nk)
+                               : 1;
     pl.splits = static_cast<int>(std::max<int64_t>(1, std::min(std::max({by_work, by_fill, by_few}), kBwdMaxSplits)));
     if (bwd_ksplit_override() > 0)
         pl.ksplit = static_cast<int>(std::min<int64_t>({bwd_ksplit_override(), kBwdMaxKsplit, tiles}));
-    pl.grid.tiles_q = static_cast<int>(ceil_div(a->seq_q * G, pl.grid.half_q ? 64 : 128));
     pl.grid.nq = static_cast<int>(units * pl.grid.tiles_q * pl.ksplit);
-    // (64-key workgroups past head dim 64: one per CU, both passes' in one round.)
-    if (pl.grid.half_k && dp > 64)
-        pl.splits = static_cast<int>(std::min<int64_t>(
-            pl.splits, std::max<int64_t>(1, (kTileFewWgs + 8 - pl.grid.nq) / nk)));
+    if (pl.grid.half_k && dp > 64) pl.splits = static_cast<int>(std::min<int64_t>(pl.splits, room));
     pl.grid.nk = static_cast<int>(nk * pl.splits);
     return pl;
 }

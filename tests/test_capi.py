@@ -225,13 +225,15 @@ def test_backward_rejects_malformed_calls_before_launch():
         ((1, 14, 2, 2048, 2048, 64), 14 * 2048 + 2 * (2 * 8 * 2048 * 64)),
         # 840 of 138 items: two splits of at most 72
         ((1, 24, 24, 4396, 4396, 128), 24 * 4396 + 2 * (24 * 2 * 4396 * 128)),
-        # 64-key workgroups at one per CU: 128 and 128 dQ ones fill the chip, so no split
+        # 128 64-key workgroups and 128 dQ ones at one per CU: no room for a split
         ((1, 8, 8, 1024, 1024, 128), 8 * 1024),
-        # 100 beside 100 of them: no second round for a split
-        ((1, 10, 10, 609, 609, 72), 10 * 609),
-        # five with eight 64-row items: four splits of two
+        # 100 beside 100 of them: as little
+        ((1, 10, 10, 609, 609, 72), 10 * 609 + 2),
+        # five with eight 64-row items at head dim 64: four splits of two
         ((5, 4, 1, 78, 16, 64), 4 * 5 * 78 + 2 * (4 * 5 * 16 * 64)),
-        # 32 beside 116 dQ ones: four splits
+        # 128 beside 96 dQ ones of 128 rows
+        ((16, 4, 2, 190, 250, 80), 4 * 16 * 190),
+        # 32 beside 116 dQ ones of 64 rows: four splits
         ((2, 8, 2, 463, 463, 80), 8 * 2 * 463 + 2 * (2 * 4 * 2 * 463 * 96)),
         # past head dim 128 the bound and the plan are one: 48 of two items
         ((1, 12, 12, 256, 256, 256), None),
