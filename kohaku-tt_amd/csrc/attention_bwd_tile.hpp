@@ -141,9 +141,9 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
     };
     // Before the fragments' loads, whose values are selected from as they come: after them the
     // first tiles would start a memory round trip later (the whole backward of 8x2/30x30x80 14.4 ->
-    // 13.7 us, 11x6/3x23x128 additive 17.4 -> 16.7).  Not at head dim 64 without a mask, where three
-    // registers spill and 14x16x87/14x64 took 13.6 instead of 13.1.
-    constexpr bool EARLY = VL || MK != MK_NONE;
+    // 13.7 us, 11x6/3x23x128 additive 17.4 -> 16.7).  Not up to head dim 64, where it costs
+    // registers (three spilled without a mask; causal 2x10x4096x64 206 instead of 200).
+    constexpr bool EARLY = VL;
     if constexpr (EARLY)
         if (split < items) request(gi, bi, 0);
     const typename TL::Addr ad = TL::addr(lane);
@@ -198,7 +198,7 @@ __device__ __forceinline__ void bwd_dkdv(const BwdParams& p, unsigned char* smem
                         return __builtin_bit_cast(MRaw, __builtin_amdgcn_raw_buffer_load_b32(rs, off, so, 0));
                 };
                 uint32_t step = static_cast<uint32_t>(g.mrow * msz);
-                __asm__ volatile("" : "+s"(step));  // (else its multiples live across the loop)
+                if constexpr (DP > 32) __asm__ volatile("" : "+s"(step));  // (else its multiples live across the loop)
                 const uint32_t row = 4 * h2 * step;
                 const uint32_t col = static_cast<uint32_t>(min(key, g.lk - 1)) * static_cast<uint32_t>(g.mkey * msz);
                 MRaw raw[16];
@@ -480,7 +480,9 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
     };
     const int kstep = p.ksplit * TR;
     int k0 = ksp * TR;
-    if (k0 < kend) request(k0, 0);  // (before the row's own loads, as in bwd_dkdv)
+    constexpr bool EARLY = DP > 64;  // (as in bwd_dkdv)
+    if constexpr (EARLY)
+        if (k0 < kend) request(k0, 0);
 
     v8 qf[DC], of[DC];
     {
@@ -589,6 +591,8 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    if constexpr (!EARLY)
+        if (k0 < kend) request(k0, 0);
     int buf = 0;
     for (; k0 < kend; k0 += kstep) {
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (as in bwd_dkdv)
@@ -643,7 +647,7 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
 
 // Wavefronts per SIMD the kernel is held to: what its LDS leaves room for, three up to head dim
 // 64 (168 registers), two past it with 128-key dK / dV workgroups (214 and 254), one with 64-key
-// ones.  Unmasked kernels spill no vector registers; masked ones up to 13 (head dim 64).  The
+// ones.  Unmasked kernels spill no vector registers; masked ones up to 15 (head dim 64).  The
 // build fails past _build.TILE_VGPR_SPILLS.
 constexpr int bwd_waves(int dp, bool half) { return dp <= 64 ? 3 : (half ? 1 : 2); }
 
