@@ -26,7 +26,7 @@
 //   2x8/2x3062x128 causal 320 -> 161  (300 -> 597)
 //   1x14/2x2048x64 causal  72 -> 51   (263 -> 373)
 //   8 packed x 16/8 x 128 causal, 64 to 1024 tokens 153 -> 92 (211 -> 354)
-//   2x12x2433x128, additive mask 1425 -> 586 (128 -> 311)
+//   2x12x2433x128, additive mask 1425 -> 480 (128 -> 380)
 // What mattered on the way (1x24x4396x128): no spill in the loop (1351 with fragments
 // spilled -> 984 with V in LDS and one code path per block); swizzles for 64 banks (LDS busy
 // 39% -> 19% of the time); the order of the products (925 -> 861).
@@ -647,7 +647,7 @@ __device__ __forceinline__ void bwd_dq(const BwdParams& p, unsigned char* smem, 
 
 // Wavefronts per SIMD the kernel is held to: what its LDS leaves room for, three up to head dim
 // 64 (168 registers), two past it with 128-key dK / dV workgroups (214 and 254), one with 64-key
-// ones.  Unmasked kernels spill no vector registers; masked ones up to 15 (head dim 64).  The
+// ones.  Unmasked kernels spill no vector registers; masked ones up to 14 (head dim 64).  The
 // build fails past _build.TILE_VGPR_SPILLS.
 constexpr int bwd_waves(int dp, bool half) { return dp <= 64 ? 3 : (half ? 1 : 2); }
 

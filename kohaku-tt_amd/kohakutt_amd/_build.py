@@ -82,7 +82,7 @@ SOURCE_FLAGS["attention_d64.hip"] = SOURCE_FLAGS["attention_d64.hip"] + [RESOURC
 TILE_SOURCES = [src for src in HIP_SOURCES if re.fullmatch(r"attention_(tile|bwd)_d\d+\.hip", src)]
 for _src in TILE_SOURCES:
     SOURCE_FLAGS[_src] = SOURCE_FLAGS.get(_src, []) + [RESOURCE_REMARKS]
-# The most vector registers a tile kernel may spill (15 today, masked backward at head dim 64).
+# The most vector registers a tile kernel may spill (14 today, masked backward at head dim 64).
 # Their waits count no loads, so a spill is slow, not wrong: 1x24x4396x128 backward with its
 # fragments spilled took 1351 us instead of 984.
 TILE_VGPR_SPILLS = 16
