@@ -870,10 +870,17 @@ constexpr int64_t kTileHalfItems = 16;
 //   masked: 8x14/2x22x64 22 / 24, 1x8x20x64 9.5 / 11.2; head dim 32 4x12 x 32 rows x 64 keys 10.6 /
 //     9.4, 80 2x14/2x32 25.3 / 23.5, 128 28.6 / 25.1 (but 4x24x22x128 12.3 / 13.9)
 //   more rows: 4x16/4x50x64 14.9 / 13.0, 16x16x64x64 11.4 / 11.7; more keys: 24 rows x 130 keys x
-//     64, 32x24 37.5 / 37.3, 16x14/2x24x130x128 22 / 20
+//     64, 32x24 37.5 / 37.3, 16x14/2x24x130x128 22 / 20; but thousands of them are the same chain
+//     again in each workgroup (no mask, not causal): 8x16 x 32 rows x 4000 keys x 64 0.62 of the
+//     tile kernel's time, x 128 0.93, x 32 0.73; 1000 keys (2048 tiles) 0.88, 1.07, 1.04
 // (By the query heads, not the K/V heads: see dQ in bwd_plan.)
+constexpr int64_t kSmallKeyTiles = 4096;
 bool small_call(const kmi_attn_bwd_args* a, int64_t dp) {
-    if (a->seq_q > 32 || a->seq_k > 64) return false;
+    if (a->seq_q > 32) return false;
+    if (a->mask_mode == KMI_MASK_NONE && !a->causal &&
+        a->batch * a->heads_q * ceil_div(a->seq_k, 64) >= kSmallKeyTiles)
+        return true;
+    if (a->seq_k > 64) return false;
     return dp == 64 || (a->mask_mode == KMI_MASK_NONE && (dp == 32 || a->batch * a->heads_q <= 160));
 }
 

@@ -258,6 +258,10 @@ def test_backward_takes_what_its_plan_needs(sizes, floats):
         ((4, 14, 2, 32, 64, 64), False, "general"),
         ((64, 16, 16, 32, 64, 40), True, "general"),
         ((4, 14, 2, 33, 64, 64), False, "tile"),
+        ((8, 16, 16, 32, 2048, 128), False, "general"),
+        ((8, 16, 16, 32, 2048, 128), True, "tile"),
+        ((8, 16, 16, 32, 1984, 128), False, "tile"),
+        ((8, 16, 16, 33, 2048, 128), False, "tile"),
         ((4, 14, 2, 32, 65, 64), False, "tile"),
         ((1, 2, 2, 1, 1, 32), False, "general"),
         ((1, 2, 2, 1, 1, 32), True, "tile"),

@@ -596,7 +596,8 @@ def test_masked_blocks_at_the_edges(native, dev, b, h, sq, sk, d, kind, layout):
 
 
 @pytest.mark.parametrize("mask", ["none", "causal", "bool"])
-@pytest.mark.parametrize("b,hq,hk,sq,sk", [(1, 2, 2, 1, 1), (2, 6, 3, 17, 50), (1, 14, 2, 32, 64), (2, 4, 1, 33, 64), (2, 4, 4, 32, 65)])
+@pytest.mark.parametrize("b,hq,hk,sq,sk", [(1, 2, 2, 1, 1), (2, 6, 3, 17, 50), (1, 14, 2, 32, 64), (2, 4, 1, 33, 64), (2, 4, 4, 32, 65),
+                                              (4, 32, 8, 9, 2050)])
 @pytest.mark.parametrize("d,dtype", [(24, torch.bfloat16), (64, torch.float16), (72, torch.bfloat16), (128, torch.float16)])
 def test_few_rows_and_keys(native, dev, b, hq, hk, sq, sk, d, dtype, mask):
     """Both sides of the line between attn_bwd_grads and the tile kernel."""
